@@ -288,11 +288,12 @@ __device__ __forceinline__ double pow23_start(double x) {
 }
 
 // ----------------------------------------------------------------------------
-// FP64 Kepler solve (Markley 1995).  Input: M reduced to [-pi, pi].
-// Output: sin E, cos E (and E for M >= 0 through kepler_fp64_E).
+// FP64 Kepler solve without a table (Markley 1995; PREC 0 above KT_EMAX or for
+// short series, see planet_sc).  Input: M reduced to [-pi, pi].  Output:
+// sin E, cos E.
 // ----------------------------------------------------------------------------
-__device__ __forceinline__ void kepler_fp64_E(double M, const PlanetC& pc, const SinCosTab& tb, double& E,
-                                              double& sE, double& cE) {
+__device__ __forceinline__ void kepler_fp64(double M, const PlanetC& pc, const SinCosTab& tb, double& sE,
+                                            double& cE) {
     const double e = pc.e;
     const double Ma = __builtin_fabs(M);
     const double ome = 1.0 - e;
@@ -333,22 +334,16 @@ __device__ __forceinline__ void kepler_fp64_E(double M, const PlanetC& pc, const
     const double cd = __builtin_fma(dd, __builtin_fma(dd, 1.0 / 24.0, -0.5), 1.0);
     sE = __builtin_fma(s, cd, c * sd);
     cE = __builtin_fma(c, cd, -s * sd);
-    E = E1 + d5;
     if (M < 0.0) sE = -sE;
 }
 
-__device__ __forceinline__ void kepler_fp64(double M, const PlanetC& pc, const SinCosTab& tb, double& sE,
-                                            double& cE) {
-    double E;
-    kepler_fp64_E(M, pc, tb, E, sE, cE);
-}
-
 // ----------------------------------------------------------------------------
-// Per-vector Kepler tables (mixed path).  For one parameter vector the
+// Per-vector Kepler tables.  For one parameter vector the
 // eccentricity of a planet is fixed, so E(M) on [0, pi] is tabulated once at
 // KT_N nodes M_j = j h (h = pi / (KT_N - 1)) as (E_j, h dE/dM_j) in FP32;
 // each epoch then takes the cubic Hermite interpolant between its two nodes
-// and one FP64 step.  The table is kept in one of two forms: the nodes
+// and one FP64 step, on the FP64 path to FP64 accuracy (kepler_fp64_tab), on
+// the mixed path as described next.  The table is kept in one of two forms: the nodes
 // (float2, 512 B per planet), or the interpolant's coefficients on each of
 // the KT_N - 1 intervals and, as interval KT_N - 1, its linear extension
 // past pi, where rounding can put |M| (float4, 1 KiB per planet, five fewer
@@ -492,7 +487,7 @@ __device__ __forceinline__ void ktab_fill(const PlanetC& pc, int lane, float4& o
 // step converges from either side of the root.
 template <bool HALLEY>
 __device__ __forceinline__ void kepler_fp64_step(double Ma, float Ef, double e, const SinCosTab& tb, double& sE,
-                                                 double& cE) {
+                                                 double& cE, double& rD) {
     const double E0 = (double)Ef;
     double s, c;
     // Near periastron at high e the step amplifies an error in sin E0 by
@@ -519,29 +514,109 @@ __device__ __forceinline__ void kepler_fp64_step(double Ma, float Ef, double e, 
         const double cd = __builtin_fma(dd, -0.5, 1.0);
         sE = __builtin_fma(c, sd, s * cd);
         cE = __builtin_fma(-s, sd, c * cd);
+        rD = rcp64_1(__builtin_fma(e, -cE, 1.0));
     } else {
         sE = __builtin_fma(c, dl, s);
         cE = __builtin_fma(-s, dl, c);
+        // 1 / (1 - e cos E) from the step's reciprocal: |h| <= 1.3e-6 (the
+        // move of e cos E, and r1's 4.6e-8), so 1 + h + h^2 leaves 2e-18; a
+        // fresh reciprocal with one refinement costs 1.8 times as much issue
+        // time (7.1 ns against an FMA's 2.1) and leaves 2e-15.
+        const double h = __builtin_fma(-__builtin_fma(e, -cE, 1.0), r1, 1.0);
+        rD = __builtin_fma(r1, __builtin_fma(h, h, h), r1);
     }
 }
 
-// (sin E, cos E) of the planet at time t.  PREC 0: FP64 Markley; PREC 1:
-// mixed, on the path kmode (kt_mode of the slot's mask, a wave-uniform
-// scalar so that each choice is a scalar branch), with `kt` the planet's
-// per-vector table (either form).  tp as in planet_M.
+// FP64 path: the step from the FP32 table start Ef to FP64 accuracy, with
+// (sin E, cos E) and 1 / (1 - e cos E).  With f1, f2, f3 the derivatives of
+// f = E - e sin E - M at the start, a = f2 / f1, b = f3 / f1 and dn = -f / f1,
+// the root lies at
+//   dn - (a/2) dn^2 + (a^2/2 - b/6) dn^3 + O(dn^4)
+// from it (the inverse series of f).  WIDE (table start at 0.5 < e <= 0.75,
+// <= 3.5e-5 rad off): all three terms, leaving under 5e-18 rad, and the
+// rotation to the third order.  Else (<= 6.1e-7 rad off up to e = 0.5, 7.3e-7
+// after the FP32 Halley step up to 0.95): two terms leave 2e-18 rad, and the
+// rotation's cubic term (7e-20) is dropped.  The start's own precision does
+// not reach the result: what is left is the rounding of FP64 f and of the
+// rotation, as after the Markley start.  1 / (1 - e cos E) comes from the
+// step's reciprocal r1 by the series of 1 / (1 - h), h = 1 - (1 - e cos E) r1
+// (|h| <= 2.3e-6, 4e-5 with WIDE: the next term is below 1.2e-17).
+// The path is bound by FP64 issue; Markley's start and correction take about
+// 92 FP64 operations and 7 FP64 reciprocals per planet-epoch, this about 45
+// and one.  Measured, Markley alone against this: batched lnL of 2560 vectors,
+// 3 planets x 1530 epochs, 66.7 -> 45.5 us; stretch sweeps of 16 x 1024 walkers,
+// 7 planets x 10^4 epochs, 5.0 -> 3.6 ms; adjoint of 16,384 vectors, 5 planets x
+// 2000 epochs, 1.38 -> 1.16 ms; the term's error against long double is the
+// same (rms 1.3e-16 to 1.6e-16 K up to e = 0.95).
+template <bool WIDE>
+__device__ __forceinline__ void kepler_fp64_tab(double Ma, float Ef, double e, const SinCosTab& tb, double& sE,
+                                                double& cE, double& rD) {
+    const double E0 = (double)Ef;
+    const int k = round_half_up(Ef * (float)SC_INV_H);
+    const double kd = (double)k;
+    const double d = __builtin_fma(-kd, SC_H_LO, __builtin_fma(-kd, SC_H, E0));
+    const double2 sc = tb.v[k];
+    const double d2 = d * d;
+    const double sd0 = __builtin_fma(d * d2, __builtin_fma(d2, 1.0 / 120.0, -1.0 / 6.0), d);
+    const double cd0 = __builtin_fma(d2, __builtin_fma(d2, __builtin_fma(d2, -1.0 / 720.0, 1.0 / 24.0), -0.5), 1.0);
+    const double s = __builtin_fma(sc.x, cd0, sc.y * sd0);
+    const double c = __builtin_fma(sc.y, cd0, -sc.x * sd0);
+    const double f0 = E0 - __builtin_fma(e, s, Ma);
+    const double f1 = __builtin_fma(e, -c, 1.0);
+    const double r1 = rcp64_1(f1);
+    const double dn = -f0 * r1;
+    const double ha = -0.5 * (e * s) * r1;            // -a / 2
+    double dl;
+    if (WIDE) {
+        const double b6 = __builtin_fma(f1, r1 * (1.0 / 6.0), -r1 * (1.0 / 6.0));   // -b / 6: f3 = 1 - f1
+        dl = dn * __builtin_fma(dn, __builtin_fma(dn, __builtin_fma(2.0 * ha, ha, b6), ha), 1.0);
+    } else {
+        dl = dn * __builtin_fma(dn, ha, 1.0);
+    }
+    const double dd = dl * dl;
+    const double cd = -0.5 * dd;                      // cos dl - 1
+    const double sd = WIDE ? __builtin_fma(dl * dd, -1.0 / 6.0, dl) : dl;
+    sE = __builtin_fma(c, sd, __builtin_fma(s, cd, s));
+    cE = __builtin_fma(-s, sd, __builtin_fma(c, cd, c));
+    const double h = __builtin_fma(-__builtin_fma(e, -cE, 1.0), r1, 1.0);
+    double q = __builtin_fma(h, h, h);
+    if (WIDE) q = __builtin_fma(h, q, h);
+    rD = __builtin_fma(r1, q, r1);
+}
+
+// Reciprocal of the path: two Newton steps (FP64) or one (mixed).
+template <int PREC>
+__device__ __forceinline__ double rcp_path(double x) {
+    return PREC == 0 ? rcp64(x) : rcp64_1(x);
+}
+
+// (sin E, cos E) of the planet at time t and 1 / (1 - e cos E), on the path
+// kmode (kt_mode of the slot's mask, a wave-uniform scalar so that each choice
+// is a scalar branch), with `kt` the planet's per-vector table (either form).
+// PREC 0: to FP64 accuracy, from the table start (kepler_fp64_tab) or, without
+// one, from Markley's; PREC 1: mixed.  tp as in planet_M.
 template <int PREC, class KTE>
 __device__ __forceinline__ void planet_sc(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, double t,
-                                          double& sE, double& cE, bool tp, int kmode) {
+                                          double& sE, double& cE, double& rD, bool tp, int kmode) {
     // Both paths reduce the same FP64 mean anomaly: the mixed path's M is
     // rounded exactly as the FP64 path's, so its error near periastron at
     // high e (amplified by dE/dM = 1 / (1 - e cos E)) stays the FP64 path's.
     const double M = reduce_2pi(planet_M(pc, t, tp));
-    if (PREC == 0) {
-        kepler_fp64(M, pc, tb, sE, cE);
-        return;
-    }
     const double Ma = __builtin_fabs(M);
     const float Mf = (float)Ma;
+    if (PREC == 0) {
+        if (kmode & KT_F_TABLE) {
+            float Ef = ktab_start(kt, Mf);
+            if (kmode & KT_F_H32) Ef = kepler_fp32_halley(Ef, Mf, pc);
+            if ((kmode & (KT_F_H32 | KT_F_H64)) == KT_F_H64) kepler_fp64_tab<true>(Ma, Ef, pc.e, tb, sE, cE, rD);
+            else kepler_fp64_tab<false>(Ma, Ef, pc.e, tb, sE, cE, rD);
+            sE = __builtin_copysign(sE, M);
+        } else {
+            kepler_fp64(M, pc, tb, sE, cE);
+            rD = rcp64(__builtin_fma(pc.e, -cE, 1.0));
+        }
+        return;
+    }
     float Ef;
     if (kmode & KT_F_TABLE) {
         Ef = ktab_start(kt, Mf);
@@ -551,27 +626,20 @@ __device__ __forceinline__ void planet_sc(const PlanetC& pc, const SinCosTab& tb
         // near periastron at e -> 1 it may leave [0, pi], so it is clamped
         Ef = __builtin_amdgcn_fmed3f(kepler_fp32_start(Mf, pc), 0.0f, (float)PI_D);
     }
-    if (kmode & KT_F_H64) kepler_fp64_step<true>(Ma, Ef, pc.e, tb, sE, cE);
-    else kepler_fp64_step<false>(Ma, Ef, pc.e, tb, sE, cE);
+    if (kmode & KT_F_H64) kepler_fp64_step<true>(Ma, Ef, pc.e, tb, sE, cE, rD);
+    else kepler_fp64_step<false>(Ma, Ef, pc.e, tb, sE, cE, rD);
     // E(-M) = -E(M), and sin E >= 0 on [0, pi]: the sign of M, one bit insert
     // (a rounding-level negative sE at E ~ 0 or pi comes back positive).
     sE = __builtin_copysign(sE, M);
-}
-
-// Reciprocal of the path: two Newton steps (FP64) or one (mixed).
-template <int PREC>
-__device__ __forceinline__ double rcp_path(double x) {
-    return PREC == 0 ? rcp64(x) : rcp64_1(x);
 }
 
 // Planet term at time t (see planet_sc).
 template <int PREC, class KTE>
 __device__ __forceinline__ double planet_mu(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, double t,
                                            bool tp, int kmode) {
-    double sE, cE;
-    planet_sc<PREC>(pc, tb, kt, t, sE, cE, tp, kmode);
-    const double den = __builtin_fma(pc.e, -cE, 1.0);
-    return __builtin_fma(pc.c1, cE, pc.c2 * sE) * rcp_path<PREC>(den);
+    double sE, cE, rD;
+    planet_sc<PREC>(pc, tb, kt, t, sE, cE, rD, tp, kmode);
+    return __builtin_fma(pc.c1, cE, pc.c2 * sE) * rD;
 }
 
 // ----------------------------------------------------------------------------

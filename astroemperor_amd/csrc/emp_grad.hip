@@ -73,10 +73,9 @@ struct GradWaveLDS {
 template <int PREC, class KTE>
 __device__ __forceinline__ void planet_wgrad(const PlanetC& pc, const SinCosTab& tab, const KTE* kt, double t,
                                              double w, double (&a)[5], bool tp, int kmode) {
-    double sE, cE;
-    planet_sc<PREC>(pc, tab, kt, t, sE, cE, tp, kmode);
+    double sE, cE, rD;
+    planet_sc<PREC>(pc, tab, kt, t, sE, cE, rD, tp, kmode);
     const double e = pc.e;
-    const double rD = rcp_path<PREC>(__builtin_fma(e, -cE, 1.0));
     const double u = cE - e, v = pc.bq * sE;
     const double sfw = __builtin_fma(v, pc.cw, u * pc.sw) * rD;     // sin(f + w)
     const double cfw = __builtin_fma(u, pc.cw, -(v * pc.sw)) * rD;  // cos(f + w)
@@ -867,9 +866,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EXT == 
     for (int j = g; j <= SC_N; j += NT) s_tile.tab.v[j] = md.sctab[j];
     if (wave == 0) slot_setup(md, sl, lane);
     __syncthreads();
-    if (PREC == 1)      // the mixed path's per-vector Kepler tables, one planet per wave
-        for (int p = wave; p < md.K; p += NW)
-            if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
+    for (int p = wave; p < md.K; p += NW)       // the per-vector Kepler tables, one planet per wave
+        if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
     __syncthreads();
     const int kmask = wave_uniform(sl.ktab_mask);
     constexpr bool tp = TP;
@@ -913,8 +911,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EXT == 
         for (int p = 0; p < KMAX; ++p) {
             if (p < md.K) {
                 const PlanetC& pc = sl.planet[p];
-                planet_sc<PREC>(pc, s_tile.tab, sl.ktab[p], t, sE[p], cE[p], tp, kt_mode(kmask, p));
-                mu += __builtin_fma(pc.c1, cE[p], pc.c2 * sE[p]) * rcp_path<PREC>(__builtin_fma(pc.e, -cE[p], 1.0));
+                double rD;
+                planet_sc<PREC>(pc, s_tile.tab, sl.ktab[p], t, sE[p], cE[p], rD, tp, kt_mode(kmask, p));
+                mu += __builtin_fma(pc.c1, cE[p], pc.c2 * sE[p]) * rD;
             }
         }
         if (valid) {

@@ -159,15 +159,15 @@ __device__ __forceinline__ void epoch_store(const ModelDev& md, TileLDS& tl, int
     }
 }
 
-// Per-slot constants, then (mixed path) the per-vector Kepler tables, one
-// planet per wave of the slot.  The sin/cos table must already be in LDS.
+// Per-slot constants, then the per-vector Kepler tables, one planet per wave
+// of the slot.  The sin/cos table must already be in LDS.
 // All threads of the workgroup call this (it holds two barriers).
 template <int PREC, int WPT, class SL>
 __device__ __forceinline__ void slot_prepare(const ModelDev& md, SL& sl, const TileLDS& tl, bool live,
                                              int wsub, int lane) {
     if (live && wsub == 0) slot_setup(md, sl, lane);
     __syncthreads();
-    if (PREC == 1 && live) {
+    if (live) {
         for (int p = wsub; p < md.K; p += WPT)
             if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
     }

@@ -187,7 +187,7 @@ __device__ void pt_eval_accept(const ModelDev& md, const PTView& pv, const TaskO
     __syncthreads();
     if (live && wsub == 0) slot_setup(md, sl, lane);
     __syncthreads();
-    if (PREC == 1 && live) {       // per-vector Kepler tables, one planet per wave
+    if (live) {       // per-vector Kepler tables, one planet per wave
         for (int p = wsub; p < md.K; p += WPT)
             if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
     }
