@@ -202,13 +202,13 @@ __device__ inline PlanetC planet_setup(const double* th, int param, int use_c) {
     pc.e = e;
     pc.c1 = A * (1.0 - e) * (1.0 + e) * cw;
     pc.c2 = -A * q * sw;
-    pc.mk_a1 = MK_A1 / (1.0 + e);
+    pc.mk_a1 = MK_A1 * rcp64(1.0 + e);      // a starter's constant
     pc.mk_d0 = 3.0 * (1.0 - e);
     pc.K = A;
     pc.cw = cw;
     pc.sw = sw;
     pc.bq = q;
-    pc.ibq = 1.0 / q;
+    pc.ibq = rcp64(q);
     if (pc.bad) {   // the reference evaluates to NaN here; make that explicit
         pc.c1 = __builtin_nan("");
         pc.c2 = __builtin_nan("");
@@ -590,56 +590,76 @@ __device__ __forceinline__ double rcp_path(double x) {
     return PREC == 0 ? rcp64(x) : rcp64_1(x);
 }
 
-// (sin E, cos E) of the planet at time t and 1 / (1 - e cos E), on the path
-// kmode (kt_mode of the slot's mask, a wave-uniform scalar so that each choice
-// is a scalar branch), with `kt` the planet's per-vector table (either form).
-// PREC 0: to FP64 accuracy, from the table start (kepler_fp64_tab) or, without
-// one, from Markley's; PREC 1: mixed.  tp as in planet_M.
-template <int PREC, class KTE>
-__device__ __forceinline__ void planet_sc(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, double t,
-                                          double& sE, double& cE, double& rD, bool tp, int kmode) {
+// (sin E, cos E) of the planet at each of the lane's NE times and
+// 1 / (1 - e cos E), on the path kmode (kt_mode of the slot's mask, a
+// wave-uniform scalar so that each choice is a scalar branch), with `kt` the
+// planet's per-vector table (either form).  The epochs' chains are independent
+// and sit in one basic block each.  PREC 0: to FP64 accuracy, from the table
+// start (kepler_fp64_tab) or, without one, from Markley's; PREC 1: mixed.  tp
+// as in planet_M.
+template <int PREC, int NE, class KTE>
+__device__ __forceinline__ void planet_sc(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, const double (&t)[NE],
+                                          double (&sE)[NE], double (&cE)[NE], double (&rD)[NE], bool tp, int kmode) {
     // Both paths reduce the same FP64 mean anomaly: the mixed path's M is
     // rounded exactly as the FP64 path's, so its error near periastron at
     // high e (amplified by dE/dM = 1 / (1 - e cos E)) stays the FP64 path's.
-    const double M = reduce_2pi(planet_M(pc, t, tp));
-    const double Ma = __builtin_fabs(M);
-    const float Mf = (float)Ma;
-    if (PREC == 0) {
-        if (kmode & KT_F_TABLE) {
-            float Ef = ktab_start(kt, Mf);
-            if (kmode & KT_F_H32) Ef = kepler_fp32_halley(Ef, Mf, pc);
-            if ((kmode & (KT_F_H32 | KT_F_H64)) == KT_F_H64) kepler_fp64_tab<true>(Ma, Ef, pc.e, tb, sE, cE, rD);
-            else kepler_fp64_tab<false>(Ma, Ef, pc.e, tb, sE, cE, rD);
-            sE = __builtin_copysign(sE, M);
-        } else {
-            kepler_fp64(M, pc, tb, sE, cE);
-            rD = rcp64(__builtin_fma(pc.e, -cE, 1.0));
+    double M[NE], Ma[NE];
+    float Mf[NE], Ef[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        M[i] = reduce_2pi(planet_M(pc, t[i], tp));
+        Ma[i] = __builtin_fabs(M[i]);
+        Mf[i] = (float)Ma[i];
+    }
+    if (kmode & KT_F_TABLE) {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) Ef[i] = ktab_start(kt, Mf[i]);
+        if (kmode & KT_F_H32) {
+#pragma unroll
+            for (int i = 0; i < NE; ++i) Ef[i] = kepler_fp32_halley(Ef[i], Mf[i], pc);
+        }
+    } else if (PREC == 0) {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            kepler_fp64(M[i], pc, tb, sE[i], cE[i]);
+            rD[i] = rcp64(__builtin_fma(pc.e, -cE[i], 1.0));
         }
         return;
-    }
-    float Ef;
-    if (kmode & KT_F_TABLE) {
-        Ef = ktab_start(kt, Mf);
-        if (kmode & KT_F_H32) Ef = kepler_fp32_halley(Ef, Mf, pc);
     } else {
         // the Markley start always takes the FP32 Halley step (kt_flags);
         // near periastron at e -> 1 it may leave [0, pi], so it is clamped
-        Ef = __builtin_amdgcn_fmed3f(kepler_fp32_start(Mf, pc), 0.0f, (float)PI_D);
+#pragma unroll
+        for (int i = 0; i < NE; ++i)
+            Ef[i] = __builtin_amdgcn_fmed3f(kepler_fp32_start(Mf[i], pc), 0.0f, (float)PI_D);
     }
-    if (kmode & KT_F_H64) kepler_fp64_step<true>(Ma, Ef, pc.e, tb, sE, cE, rD);
-    else kepler_fp64_step<false>(Ma, Ef, pc.e, tb, sE, cE, rD);
+    if (PREC == 0) {
+        if ((kmode & (KT_F_H32 | KT_F_H64)) == KT_F_H64) {
+#pragma unroll
+            for (int i = 0; i < NE; ++i) kepler_fp64_tab<true>(Ma[i], Ef[i], pc.e, tb, sE[i], cE[i], rD[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NE; ++i) kepler_fp64_tab<false>(Ma[i], Ef[i], pc.e, tb, sE[i], cE[i], rD[i]);
+        }
+    } else if (kmode & KT_F_H64) {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) kepler_fp64_step<true>(Ma[i], Ef[i], pc.e, tb, sE[i], cE[i], rD[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NE; ++i) kepler_fp64_step<false>(Ma[i], Ef[i], pc.e, tb, sE[i], cE[i], rD[i]);
+    }
     // E(-M) = -E(M), and sin E >= 0 on [0, pi]: the sign of M, one bit insert
     // (a rounding-level negative sE at E ~ 0 or pi comes back positive).
-    sE = __builtin_copysign(sE, M);
+#pragma unroll
+    for (int i = 0; i < NE; ++i) sE[i] = __builtin_copysign(sE[i], M[i]);
 }
 
 // Planet term at time t (see planet_sc).
 template <int PREC, class KTE>
 __device__ __forceinline__ double planet_mu(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, double t,
                                            bool tp, int kmode) {
-    double sE, cE, rD;
-    planet_sc<PREC>(pc, tb, kt, t, sE, cE, rD, tp, kmode);
-    return __builtin_fma(pc.c1, cE, pc.c2 * sE) * rD;
+    double sE[1], cE[1], rD[1];
+    planet_sc<PREC, 1>(pc, tb, kt, {t}, sE, cE, rD, tp, kmode);
+    return __builtin_fma(pc.c1, cE[0], pc.c2 * sE[0]) * rD[0];
 }
 
 // ----------------------------------------------------------------------------

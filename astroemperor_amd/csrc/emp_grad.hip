@@ -60,10 +60,10 @@ struct GradWave {
     static constexpr int N = SAI + (EXT >= 1 ? SAIMAX : 0);
 };
 constexpr int WN_ACC = KMAX * 5, WN_N = KMAX * 5 + AMAX;
-template <int EXT>
+template <int EXT, int NW = NWAVES>
 struct GradWaveLDS {
-    double acc[NWAVES][GradWave<EXT>::N];
-    double nat[NWAVES][WN_N];
+    double acc[NW][GradWave<EXT>::N];
+    double nat[NW][WN_N];
 };
 
 // w times the derivatives of one planet's term at time t with respect to its
@@ -73,8 +73,9 @@ struct GradWaveLDS {
 template <int PREC, class KTE>
 __device__ __forceinline__ void planet_wgrad(const PlanetC& pc, const SinCosTab& tab, const KTE* kt, double t,
                                              double w, double (&a)[5], bool tp, int kmode) {
-    double sE, cE, rD;
-    planet_sc<PREC>(pc, tab, kt, t, sE, cE, rD, tp, kmode);
+    double sE1[1], cE1[1], rD1[1];
+    planet_sc<PREC, 1>(pc, tab, kt, {t}, sE1, cE1, rD1, tp, kmode);
+    const double sE = sE1[0], cE = cE1[0], rD = rD1[0];
     const double e = pc.e;
     const double u = cE - e, v = pc.bq * sE;
     const double sfw = __builtin_fma(v, pc.cw, u * pc.sw) * rD;     // sin(f + w)
@@ -487,12 +488,29 @@ __device__ __forceinline__ double plain_w(const ModelDev& md, const SL& sl, cons
     return w;
 }
 
+// The single-pass kernel's sums over the epochs, with C = cos f, S = sin f / b,
+// s = sin(f + w), q = 1 + e C = b^2 / D and tau the time the phase counts from:
+//   n0 = sum w s q^2 tau, n1 = sum w s q^2, n2 = sum w s S (q + 1),
+//   n3 = sum w C, n4 = sum w S,
+// to the sums of w times the natural-parameter derivatives (those of
+// planet_wgrad): the constants of the planet and the parts that do not depend
+// on the epoch (wsum = sum w) come in once per vector instead of per epoch.
+__device__ __forceinline__ void nat_basis(const PlanetC& pc, double wsum, double (&n)[5]) {
+    const double kb = -pc.K * pc.ibq * pc.ibq * pc.ibq, bs = pc.bq * n[4], ew = pc.e * wsum;
+    n[0] *= kb;
+    n[1] *= kb;
+    n[2] = pc.K * (pc.cw * wsum - pc.ibq * n[2]);
+    n[4] = pc.cw * ew + (pc.cw * n[3] - pc.sw * bs);
+    n[3] = -pc.K * (pc.sw * ew + (pc.sw * n[3] + pc.cw * bs));
+}
+
 // Adds the per-wave partial sums of a slot in wave order, maps the natural
 // gradients to the parameterisation and writes lnL and the free gradient of
 // vector b.  All threads of the workgroup call this (it holds barriers).
-template <int EXT, int WPT, class SL>
+// BASIS: the planets' sums are those of the single-pass kernel (nat_basis).
+template <int EXT, int WPT, bool BASIS = false, int NW = NWAVES, class SL>
 __device__ __forceinline__ void grad_finish(const ModelDev& md, const SL& sl, GradLDS& gl,
-                                            const GradWaveLDS<EXT>& s_gw, bool live, int wave, int wsub, int lane,
+                                            const GradWaveLDS<EXT, NW>& s_gw, bool live, int wave, int wsub, int lane,
                                             double lnl_v, int64_t b, double* __restrict__ out_lnl,
                                             double* __restrict__ out_grad, unsigned long long* nonfinite, int* stale) {
     using GW = GradWave<EXT>;
@@ -536,14 +554,20 @@ __device__ __forceinline__ void grad_finish(const ModelDev& md, const SL& sl, Gr
             const PlanetC& pc = sl.planet[p];
             const double* th = sl.theta + md.off_kep + 5 * p;
             double* gp = gl.g + md.off_kep + 5 * p;
-            const double per = 2.0 * PI_D / pc.freq;
-            const double gP = gl.nat[p][0] * (-pc.freq / per);
-            const double gph = gl.nat[p][1];
-            const double ge = gl.nat[p][2], gw = gl.nat[p][3], gA = gl.nat[p][4];
+            double nat[5];
+            for (int q = 0; q < 5; ++q) nat[q] = gl.nat[p][q];
+            if (BASIS) {
+                double wsum = 0.0;                   // sum of w over all epochs
+                for (int k = 0; k < md.I; ++k) wsum += gl.g[md.off_off + k];
+                nat_basis(pc, wsum, nat);
+            }
+            const double gP = nat[0] * (-pc.freq * pc.freq * INV_TWO_PI);     // dfreq/dP = -freq^2 / (2 pi)
+            const double gph = nat[1];
+            const double ge = nat[2], gw = nat[3], gA = nat[4];
             const int prm = md.param;
             const bool lnP = (prm == 2 || prm == 6 || prm == 7);
             const bool sc = (prm == 1 || prm == 2 || prm == 4 || prm == 7);
-            gp[0] = lnP ? gP * per : gP;
+            gp[0] = lnP ? -nat[0] * pc.freq : gP;
             if (prm == 2) {
                 const double As = th[1], Ac = th[2], A = pc.K;
                 gp[1] = gA * 2.0 * As + gph * (Ac / A);
@@ -734,9 +758,12 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
 
 // ---------------------------------------------------------------------------
 // Single-pass adjoint for models whose moving average has order 1 or is
-// absent: eight waves per vector, one vector per workgroup, one epoch per
-// lane per tile.  Each planet's Kepler solve is done once per epoch; its
-// (sin E, cos E) stay in registers from the model to the derivatives.
+// absent: NW waves per vector, one vector per workgroup, two consecutive epochs
+// per lane per tile, loaded straight from global memory (the data of all
+// vectors are the same few hundred KB, in L2).  Each planet's Kepler solve is
+// done once per epoch; cos f, sin f and 1 / D stay in registers from the model
+// to the derivatives, and every lane keeps its own five sums per planet over
+// the whole series, reduced over the wave once per vector.
 //
 // The MA(1) adjoint is carried forward.  Within a tile the reverse
 // recurrence lambda_i = u_i + a_{i+1} lambda_{i+1} composes (a suffix scan
@@ -749,7 +776,18 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
 //   sum_n (S_B^n + Lambda_n S_A^n) = sum_n (S_B^n + B^n R_n),
 //   R_0 = 0, R_{n+1} = A^n R_n + S_A^n.
 // Every such sum keeps a total and an R state and is complete after one pass
-// over the epochs; no eps row is stored.
+// over the epochs; no eps row is stored.  S_B needs no tile map, which is why
+// it can stay in a lane's registers; S_A is reduced per tile, but only by the
+// waves in which some A_i matters (the tile's last, unless the MA is nearly a
+// random walk).  The waves take the tile's segments in turn (rotated by one
+// every tile), so that this work falls on every SIMD alike.
+//
+// Bound by VALU issue (104 to 112 instructions per planet-epoch against the
+// 205 of one epoch per lane with five sums per planet reduced in every tile;
+// the VALU issues in about 70% of the cycles).  Measured before and after:
+// 8192 vectors of 7 planets x 10^4 epochs, MA(1), mixed, 3.76 -> 2.46 ms; 16,384
+// of 5 planets x 2000 epochs, FP64 (with its table start), 1.16 -> 0.58 ms, a
+// third of that from grouping the epochs by instrument (emp_model_host).
 // ---------------------------------------------------------------------------
 
 // Per-lane sums of the per-instrument terms (offset, jitter, MA(1)
@@ -779,6 +817,48 @@ struct InsAcc1 {
         atomicAdd(&rst[GW::MAT + km * GW::QM], matR);
         mac = macR = mat = matR = 0.0;
     }
+    // The end of the pass: the lanes that share an instrument are summed over
+    // the wave (in a fixed order) and added by one lane, one instrument after
+    // the other, instead of 64 atomics on the same few addresses.  Whole wave
+    // active.
+    template <int EXT>
+    __device__ __forceinline__ void flush_all(bool ma, double* tot, double* rst, int lane) {
+        using GW = GradWave<EXT>;
+        unsigned long long left = __ballot(k >= 0);
+        while (left) {
+            const int kk = __builtin_amdgcn_readlane(k, (int)__builtin_ctzll(left));
+            const bool in = k == kk;
+            const double so = wave_sum(in ? off : 0.0), sj = wave_sum(in ? jit : 0.0);
+            const double sr = ma ? wave_sum(in ? offR : 0.0) : 0.0;
+            if (lane == 0) {
+                tot[GW::OFF + kk] += so;
+                rst[GW::OFF + kk] += sr;
+                tot[GW::JIT + kk] += sj;
+            }
+            left &= ~__ballot(in);
+        }
+        if (!ma) return;
+        left = __ballot(km >= 0);
+        while (left) {
+            const int kk = __builtin_amdgcn_readlane(km, (int)__builtin_ctzll(left));
+            const bool in = km == kk;
+            const double sc = wave_sum(in ? mac : 0.0), st = wave_sum(in ? mat : 0.0);
+            if (lane == 0) {
+                tot[GW::MAC + kk * GW::QM] += sc;
+                tot[GW::MAT + kk * GW::QM] += st;
+            }
+            left &= ~__ballot(in);
+        }
+    }
+    // The move to the next tile, whose map is (tA, tB).
+    __device__ __forceinline__ void move(double tA, double tB) {
+        off = __builtin_fma(tB, offR, off);
+        mac = __builtin_fma(tB, macR, mac);
+        mat = __builtin_fma(tB, matR, mat);
+        offR *= tA;
+        macR *= tA;
+        matR *= tA;
+    }
     template <int EXT>
     __device__ __forceinline__ void to(int kk, int kkm, double* tot, double* rst) {
         if (kk != k) {
@@ -792,66 +872,49 @@ struct InsAcc1 {
     }
 };
 
-// The epochs of one tile of the single-pass kernel (NT of them) and the
-// sin/cos table; thread j stages epoch tb + j, its loads issued a tile ahead.
-template <int NT>
-struct Tile1LDS {
-    double t[NT], y[NT], s2[NT], dt[NT];
-    int ins[NT];
-    SinCosTab tab;
-};
+// Value of the next lane (lane 63: `last`), of the previous one (lane 0:
+// `first`): DPP wave_shl:1 and wave_shr:1.  Whole wave active.
+__device__ __forceinline__ double wave_next(double v, double last) { return dpp_f64<0x130, 0xf>(last, v); }
+__device__ __forceinline__ double wave_prev(double v, double first) { return dpp_f64<0x138, 0xf>(first, v); }
 
-template <int NT>
-__device__ __forceinline__ void tile1_prefetch(const ModelDev& md, int tb, EpochRegs& r) {
-    const int n = tb + (int)threadIdx.x;
-    if (n < md.N) {
-        r.t = md.t[n];
-        r.y = md.y[n];
-        r.s2 = md.s2[n];
-        r.ins = md.ins[n];
-        r.dt = md.ma_active ? md.dt[n] : 0.0;
-    }
-}
+// The planets' constants are read from LDS where they are used: without this
+// the compiler keeps those of all planets in registers over the tiles.
+__device__ __forceinline__ void reload_lds() { asm volatile("" ::: "memory"); }
 
-template <int NT>
-__device__ __forceinline__ void tile1_store(const ModelDev& md, Tile1LDS<NT>& tl, int tb, const EpochRegs& r) {
-    const int j = threadIdx.x;
-    if (tb + j < md.N) {
-        tl.t[j] = r.t;
-        tl.y[j] = r.y;
-        tl.s2[j] = r.s2;
-        tl.ins[j] = r.ins;
-        tl.dt[j] = r.dt;
-    }
-}
-
-template <int EXT>
+template <int EXT, int NW>
 struct Grad1LDS {
-    double rst[NWAVES][GradWave<EXT>::N];    // R states of the per-instrument sums (per wave)
-    double natR[NWAVES][WN_N];               // R states of the planet and acceleration sums (per wave)
-    double suf[2][NWAVES][2];                // suffix maps of the waves (double-buffered)
+    double rst[NW][GradWave<EXT>::N];    // R states of the per-instrument sums (per wave)
+    double natR[NW][WN_N];               // R states of the planet and acceleration sums (per wave)
+    double2 fwd[2][NW], suf[2][NW];      // per segment: its forward and suffix maps (double-buffered)
+    double first[2][NW];                 // its first epoch's multiplier
 };
 
 // Single-pass adjoint (above).  EXT: 0 plain models, 1 with the terms added
-// after the MA.  NW waves per workgroup (one vector), tiles of 64 NW epochs.
-// TP: the model's planets are parameterised by the time of periastron
-// (model_tp), a template parameter so that no planet-epoch branches on it.
-// `stale` as in k_lnl_grad.
-template <int PREC, int EXT, int NW, bool TP>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EXT == 0 ? 4 : 3))) void k_lnl_grad1(ModelDev md, const double* __restrict__ theta, int64_t B,
-                                                       int64_t ld, double* __restrict__ out_lnl,
-                                                       double* __restrict__ out_grad, unsigned long long* nonfinite,
-                                                       int* stale) {
-    constexpr int WPT = NW, NT = 64 * NW, TILE1 = NT;
-    constexpr bool POST = EXT >= 1;
+// after the MA.  MA: the model may have a moving average.  NW waves per
+// workgroup (one vector), tiles of 128 NW epochs.  KM: the instance holds up to
+// KM planets' values and sums in registers (8 and 4 VGPRs per planet).  TP: the model's planets are parameterised by the
+// time of periastron (model_tp), a template parameter so that no planet-epoch
+// branches on it.  `stale` as in k_lnl_grad.
+// Waves per SIMD that an instance is compiled for: as many as its registers
+// allow with little or no spilling (KM 4 / 6 / 8: 115 / 128 / 154 VGPRs without
+// the moving average; with it 128, 165 and 168, the last with 34 spilled, which
+// still beats 198 VGPRs at two waves per SIMD, 2.49 against 2.82 ms).
+constexpr int GRAD1_FEW = 4;
+constexpr int grad1_occ(bool ma, int km) { return km <= 4 || (km <= 6 && !ma) ? 4 : 3; }
+template <int PREC, int EXT, bool MA, int NW, int KM, bool TP>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_occ(MA, KM)))) void k_lnl_grad1(
+    ModelDev md, const double* __restrict__ theta, int64_t B, int64_t ld, double* __restrict__ out_lnl,
+    double* __restrict__ out_grad, unsigned long long* nonfinite, int* stale) {
+    constexpr int NT = 64 * NW, NE = 2, TILE1 = NT * NE;
+    constexpr bool POST = EXT >= 1, tp = TP;
     using GW = GradWave<EXT>;
-    __shared__ SlotLDS<1> sl;
+    __shared__ SlotLDSt<float4, KM> sl;
     __shared__ GradLDS gl;
-    __shared__ GradWaveLDS<EXT> s_gw;
-    __shared__ Grad1LDS<EXT> s_g1;
-    __shared__ Tile1LDS<TILE1> s_tile;
+    __shared__ GradWaveLDS<EXT, NW> s_gw;
+    __shared__ Grad1LDS<EXT, NW> s_g1;
+    __shared__ SinCosTab s_tab;
     __shared__ ScanLDS s_scan;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = threadIdx.x;
+    const int wave = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63, g = threadIdx.x;
     const int64_t b = blockIdx.x;
     if (b >= B || (stale && stale[b] == 0)) return;     // the whole workgroup: one vector
     expand_theta(md, sl, theta + b * ld, g, NT);
@@ -863,267 +926,321 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(EXT == 
     double* wnatR = s_g1.natR[wave];
     for (int j = lane; j < GW::N; j += 64) wacc[j] = wrst[j] = 0.0;
     for (int j = lane; j < WN_N; j += 64) wnat[j] = wnatR[j] = 0.0;
-    for (int j = g; j <= SC_N; j += NT) s_tile.tab.v[j] = md.sctab[j];
+    for (int j = g; j <= SC_N; j += NT) s_tab.v[j] = md.sctab[j];
+    __syncthreads();
     if (wave == 0) slot_setup(md, sl, lane);
     __syncthreads();
     for (int p = wave; p < md.K; p += NW)       // the per-vector Kepler tables, one planet per wave
         if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
     __syncthreads();
     const int kmask = wave_uniform(sl.ktab_mask);
-    constexpr bool tp = TP;
     const int ri5 = red5_index(lane), ri4 = red4_index(lane);    // the sums a lane holds after a reduction
 
-    const bool ma = md.ma_active;
+    const bool ma = MA && md.ma_active;
+    double mu0 = 0.0;                   // the planets' constant parts, sum of K e cos w
+    for (int p = 0; p < md.K; ++p) mu0 = __builtin_fma(sl.planet[p].K * sl.planet[p].e, sl.planet[p].cw, mu0);
+    // The sums of each planet (nat_basis): the first four exchanged between
+    // lanes 32 and 16 apart, so that each quarter of the wave holds one of
+    // them (acc4), the fifth per lane (acc1).
+    double acc4[KM], acc1[KM];
+#pragma unroll
+    for (int p = 0; p < KM; ++p) acc4[p] = acc1[p] = 0.0;
     double chi = 0.0, prod = 1.0;
     int pexp = 0;
     double carry = 0.0;                 // eps of the last epoch so far
-    int parity = 0, sparity = 0;
+    int parity = 0, rot = wave;         // rot: the tile's segment this wave takes
     InsAcc1 ia;
-    EpochRegs nx{};
-    tile1_prefetch<TILE1>(md, 0, nx);
-    for (int tb = 0; tb < md.N; tb += TILE1) {
-        const int tn = min(TILE1, md.N - tb);
-        __syncthreads();                // the previous tile's readers are done
-        tile1_store<TILE1>(md, s_tile, tb, nx);
-        __syncthreads();
-        if (tb + TILE1 < md.N) tile1_prefetch<TILE1>(md, tb + TILE1, nx);
-        const int j = g;
-        const bool valid = j < tn;
-        // Stage 1: every planet's (sin E, cos E), the model and the residual.
-        // Every lane solves the planets, a lane past the series' end at
-        // t = 0: its values are finite and its weights (wB, wA) exactly zero,
-        // so neither these arrays nor the derivatives below are cleared.
-        double sE[KMAX], cE[KMAX];
-        double t = 0.0, r = 0.0, err2 = 1.0, mu = 0.0;
-        int k = 0;
-        if (valid) {
-            t = s_tile.t[j];
-            k = s_tile.ins[j];
-            mu = sl.gam[k];
-            if (md.acc) {
-                const double x = t - md.t0;
-                double v = 0.0;
-                for (int a = 0; a < md.acc; ++a) v = __builtin_fma(v, x, sl.acc[a]);
-                mu += v * x;
-            }
-        }
+    double tnx[NE];                     // the next tile's times, loaded a tile ahead
 #pragma unroll
-        for (int p = 0; p < KMAX; ++p) {
+    for (int i = 0; i < NE; ++i) {
+        const int n = NE * g + i;
+        tnx[i] = n < md.N ? md.t[n] : 0.0;
+    }
+    for (int tb = 0; tb < md.N; tb += TILE1) {
+        const int n0 = tb + NE * (rot * 64 + lane);
+        const int seg = rot;
+        rot = rot + 1 == NW ? 0 : rot + 1;
+        // Every lane solves the planets, a lane past the series' end at t = 0:
+        // its values are finite and its weights (wB, wA) exactly zero.
+        double t[NE], y[NE], err2[NE], dtc[NE], mu[NE];
+        int k[NE];
+        bool valid[NE];
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            const int n = n0 + i, nn = tb + TILE1 + NE * (rot * 64 + lane) + i;
+            valid[i] = n < md.N;
+            t[i] = tnx[i];
+            tnx[i] = nn < md.N ? md.t[nn] : 0.0;
+            mu[i] = mu0;
+        }
+        auto load_rest = [&]() {
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                const int n = n0 + i;
+                k[i] = 0;
+                y[i] = 0.0;
+                err2[i] = 1.0;
+                dtc[i] = 0.0;
+                if (valid[i]) {
+                    k[i] = md.ins[n];
+                    y[i] = md.y[n];
+                    err2[i] = md.s2[n];
+                    if (ma) dtc[i] = md.dt[n];
+                }
+            }
+        };
+        reload_lds();
+        // Stage 1: every planet's C = cos f and S = sin f / b, and the model.
+        double C[KM][NE], S[KM][NE];
+#pragma unroll
+        for (int p = 0; p < KM; ++p) {
             if (p < md.K) {
                 const PlanetC& pc = sl.planet[p];
-                double rD;
-                planet_sc<PREC>(pc, s_tile.tab, sl.ktab[p], t, sE[p], cE[p], rD, tp, kt_mode(kmask, p));
-                mu += __builtin_fma(pc.c1, cE[p], pc.c2 * sE[p]) * rD;
-            }
-        }
-        if (valid) {
-            err2 = s_tile.s2[j] + sl.jit2[k];
-            r = s_tile.y[j] - mu;
-            ia.to<EXT>(k, md.ma_global ? 0 : k, wacc, wrst);
-        }
-        // The MA filter, forward (the same scan and composition as block_lnl).
-        double eps = r, em1 = 0.0;      // eps of this epoch and of the previous one
-        if (ma) {
-            double a = 1.0, bb = 0.0;
-            if (valid) {
-                const double dtj = s_tile.dt[j];
-                if (md.ma_wfixed) a = -(sl.ma_c[k] * dtj);
-                else a = dtj < 0.0 ? 0.0 : -(sl.ma_c[k] * exp(-dtj / sl.ma_tau[k]));
-                bb = r;
-            }
-            wave_affine_scan(a, bb, lane);
-            if (lane == 63) { s_scan.tot[parity][wave][0] = a; s_scan.tot[parity][wave][1] = bb; }
-            __syncthreads();
-            // (pa, pb): the maps of waves 0 .. w composed
-            double e0 = carry;
-            if (wave == 0) eps = __builtin_fma(a, carry, bb);
-            double pa = s_scan.tot[parity][0][0], pb = s_scan.tot[parity][0][1];
-            for (int w = 1; w < WPT; ++w) {
-                if (w == wave) {
-                    e0 = __builtin_fma(pa, carry, pb);
-                    eps = __builtin_fma(a, e0, bb);
+                double sE[NE], cE[NE], rD[NE];
+                planet_sc<PREC, NE>(pc, s_tab, sl.ktab[p], t, sE, cE, rD, tp, kt_mode(kmask, p));
+                const double e = pc.e, kc = pc.K * pc.cw, ks = pc.c2;
+#pragma unroll
+                for (int i = 0; i < NE; ++i) {
+                    C[p][i] = (cE[i] - e) * rD[i];
+                    S[p][i] = sE[i] * rD[i];
+                    mu[i] = __builtin_fma(kc, C[p][i], __builtin_fma(ks, S[p][i], mu[i]));
                 }
-                const double ta = s_scan.tot[parity][w][0], tbv = s_scan.tot[parity][w][1];
-                pb = __builtin_fma(ta, pb, tbv);
-                pa = ta * pa;
+            }
+        }
+        if (md.acc) {
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                const double x = t[i] - md.t0;
+                double v = 0.0;
+                for (int a = 0; a < md.acc; ++a) v = __builtin_fma(v, x, sl.acc[a]);
+                mu[i] += v * x;
+            }
+        }
+        load_rest();
+        double eps[NE], em[NE], am[NE];     // eps of the epoch and of the one before; its multiplier
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            eps[i] = em[i] = 0.0;
+            am[i] = 1.0;
+            if (valid[i]) {
+                err2[i] += sl.jit2[k[i]];
+                eps[i] = y[i] - (mu[i] + sl.gam[k[i]]);
+            }
+        }
+        // The MA filter, forward: the lane's two maps composed, a scan over
+        // the wave, the segments' maps composed through LDS.
+        double mnext_seg = 0.0;             // multiplier of the next segment's first epoch
+        if (ma) {
+#pragma unroll
+            for (int i = 0; i < NE; ++i)
+                if (valid[i]) am[i] = ma_mult(md, sl, k[i], dtc[i]);
+            const double b0 = eps[0];
+            double a = am[1] * am[0], bb = __builtin_fma(am[1], b0, eps[1]);
+            wave_affine_scan(a, bb, lane);
+            if (lane == 63) s_g1.fwd[parity][seg] = make_double2(a, bb);
+            if (lane == 0) s_g1.first[parity][seg] = am[0];
+            __syncthreads();
+            double e0 = carry;              // eps before this segment
+            double pa = 1.0, pb = 0.0;      // the maps of segments 0 .. w composed
+            double2 tot[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) tot[w] = s_g1.fwd[parity][w];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                if (w == seg) e0 = __builtin_fma(pa, carry, pb);
+                pb = w ? __builtin_fma(tot[w].x, pb, tot[w].y) : tot[w].y;
+                pa = w ? tot[w].x * pa : tot[w].x;
             }
             carry = __builtin_fma(pa, carry, pb);
-            parity ^= 1;
-            em1 = __shfl_up(eps, 1, 64);
-            if (lane == 0) em1 = e0;
+            if (seg + 1 < NW) mnext_seg = s_g1.first[parity][seg + 1];
+            const double e1 = __builtin_fma(a, e0, bb);       // the lane's last epoch
+            em[0] = wave_prev(e1, e0);
+            em[1] = __builtin_fma(am[0], em[0], b0);
+            eps[0] = em[1];
+            eps[1] = e1;
         }
         // The likelihood's terms.
-        double ef = 0.0, ie = 0.0;
-        if (valid) {
-            const double cs = (POST && has_post(md)) ? epoch_post(md, sl, s_tile.tab, t, tb + j, k) : 0.0;
-            ef = eps - cs;
-            ie = rcp_path<PREC>(err2);
-            chi = __builtin_fma(ef * ef, ie, chi);
-            prod *= err2;
-            pexp += __builtin_amdgcn_frexp_exp(prod);
-            prod = __builtin_amdgcn_frexp_mant(prod);
-            if (md.has_jit) ia.jit = __builtin_fma(sl.jit[k], ef * ef * ie * ie - ie, ia.jit);
-            if (POST && has_post(md)) post_accumulate<EXT>(md, sl, s_tile.tab, t, tb + j, k, ef * ie, wacc);
+        double ef[NE], ie[NE];
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            ef[i] = ie[i] = 0.0;
+            if (valid[i]) {
+                const double cs = (POST && has_post(md)) ? epoch_post(md, sl, s_tab, t[i], n0 + i, k[i]) : 0.0;
+                ef[i] = eps[i] - cs;
+                ie[i] = rcp_path<PREC>(err2[i]);
+                chi = __builtin_fma(ef[i] * ef[i], ie[i], chi);
+                prod *= err2[i];
+                pexp += __builtin_amdgcn_frexp_exp(prod);
+                prod = __builtin_amdgcn_frexp_mant(prod);
+                if (POST && has_post(md))
+                    post_accumulate<EXT>(md, sl, s_tab, t[i], n0 + i, k[i], ef[i] * ie[i], wacc);
+            }
         }
         // dlnL/dmu = wB + wA Lambda; lambda = lB + lA Lambda; (tA, tB) the tile's map.
-        double wB = 0.0, wA = 0.0, tA = 0.0, tB = 0.0;
+        double wB[NE], wA[NE], tA = 0.0, tB = 0.0;
         bool needA = false;
         if (!ma) {
-            wB = ef * ie;
-            ia.off += wB;
-        } else {
-            double u = 0.0, amul = 1.0;
-            if (valid) {
-                u = -ef * ie;
-                const int n1 = tb + j + 1;     // the next epoch's multiplier
-                amul = 0.0;
-                if (n1 < md.N) {
-                    const bool in_tile = j + 1 < tn;
-                    const int k1 = in_tile ? s_tile.ins[j + 1] : md.ins[n1];
-                    const double c1 = in_tile ? s_tile.dt[j + 1] : md.dt[n1];
-                    amul = ma_mult(md, sl, k1, c1);
-                }
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                wB[i] = ef[i] * ie[i];
+                wA[i] = 0.0;
             }
-            double sa = amul, sb = u;
+        } else {
+            // the multiplier of the epoch after the lane's last one
+            double m1 = wave_next(am[0], mnext_seg);
+            if (seg == NW - 1 && lane == 63 && n0 + NE < md.N) m1 = ma_mult(md, sl, md.ins[n0 + NE], md.dt[n0 + NE]);
+            if (n0 + NE >= md.N) m1 = 0.0;
+            const double m0 = n0 + 1 < md.N ? am[1] : 0.0;
+            const double u0 = -ef[0] * ie[0], u1 = -ef[1] * ie[1];
+            double sa = m0 * m1, sb = __builtin_fma(m0, u1, u0);
             wave_affine_suffix_scan(sa, sb, lane);
-            if (lane == 0) { s_g1.suf[sparity][wave][0] = sa; s_g1.suf[sparity][wave][1] = sb; }
+            if (lane == 0) s_g1.suf[parity][seg] = make_double2(sa, sb);
             __syncthreads();
-            // (pa, pb): the maps of waves WPT - 1 down to w composed
-            double lB = sb, lA = sa;
-            double pa = s_g1.suf[sparity][WPT - 1][0], pb = s_g1.suf[sparity][WPT - 1][1];
-            for (int w = WPT - 2; w >= 0; --w) {
-                if (w == wave) {
-                    lB = __builtin_fma(sa, pb, sb);
-                    lA = sa * pa;
+            // (pa, pb): the maps of segments NW - 1 down to w composed
+            double ia_ = 1.0, ib_ = 0.0;    // the map after this segment
+            double pa = 1.0, pb = 0.0;
+            double2 tot[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) tot[w] = s_g1.suf[parity][w];
+#pragma unroll
+            for (int w = NW - 1; w >= 0; --w) {
+                if (w == seg) {
+                    ia_ = pa;
+                    ib_ = pb;
                 }
-                const double ta = s_g1.suf[sparity][w][0], tbv = s_g1.suf[sparity][w][1];
-                pb = __builtin_fma(ta, pb, tbv);
-                pa = ta * pa;
+                pb = __builtin_fma(tot[w].x, pb, tot[w].y);
+                pa = tot[w].x * pa;
             }
             tA = pa;
             tB = pb;
-            sparity ^= 1;
-            if (valid) {
-                wB = -lB;
-                wA = -lA;
-            }
+            const double lB0 = __builtin_fma(sa, ib_, sb), lA0 = sa * ia_;
+            const double lB1 = __builtin_fma(m1, wave_next(lB0, ib_), u1), lA1 = m1 * wave_next(lA0, ia_);
+            wB[0] = valid[0] ? -lB0 : 0.0;
+            wA[0] = valid[0] ? -lA0 : 0.0;
+            wB[1] = valid[1] ? -lB1 : 0.0;
+            wA[1] = valid[1] ? -lA1 : 0.0;
             // A wave whose every |A_i| is below 2^-100 adds nothing measurable
             // through Lambda (the terms are under 1e-17 of any gradient the
             // data can give): it reduces the B parts alone.  With |a| <= 1/3,
             // every wave of a tile but the last is such a wave.
-            needA = __any(valid && __builtin_fabs(lA) > 0x1p-100);
-            // the sums this wave already holds in LDS move to the next tile
+            needA = __any(__builtin_fabs(wA[0]) > 0x1p-100 || __builtin_fabs(wA[1]) > 0x1p-100);
+            // the sums this wave already holds in LDS, and the lane's own,
+            // move to the next tile
             for (int e = lane; e < GW::COS; e += 64) {
                 const double R0 = wrst[e];
                 wacc[e] = __builtin_fma(tB, R0, wacc[e]);
                 wrst[e] = tA * R0;
             }
-            // this lane's sums: the epoch's terms, then the move to the next tile
-            double hc = 0.0, ht = 0.0;      // d a_j / d (c, tau) times eps_{j-1}
-            if (valid) {
-                const double col = s_tile.dt[j];
-                const bool start = md.ma_wfixed ? col == 0.0 : col < 0.0;
+            for (int e = lane; e < WN_N; e += 64) {
+                const double R0 = wnatR[e];
+                wnat[e] = __builtin_fma(tB, R0, wnat[e]);
+                wnatR[e] = tA * R0;
+            }
+            ia.move(tA, tB);
+        }
+        // The per-instrument sums of the lane's epochs.
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            if (!valid[i]) continue;
+            ia.to<EXT>(k[i], md.ma_global ? 0 : k[i], wacc, wrst);
+            ia.off += wB[i];
+            ia.offR += wA[i];
+            if (md.has_jit) ia.jit = __builtin_fma(sl.jit[k[i]], ef[i] * ef[i] * ie[i] * ie[i] - ie[i], ia.jit);
+            if (ma) {
+                // d a / d (c, tau) times the previous eps (none at a segment start)
+                const bool start = md.ma_wfixed ? dtc[i] == 0.0 : dtc[i] < 0.0;
                 if (!start) {
-                    const double wgt = md.ma_wfixed ? col : exp(-col / sl.ma_tau[k]);
-                    hc = em1 * -wgt;
+                    const double wgt = md.ma_wfixed ? dtc[i] : exp(-dtc[i] / sl.ma_tau[k[i]]);
+                    const double hc = em[i] * wgt;                      // lambda = -w
+                    ia.mac = __builtin_fma(wB[i], hc, ia.mac);
+                    ia.macR = __builtin_fma(wA[i], hc, ia.macR);
                     if (!md.ma_wfixed) {
-                        const double tau = sl.ma_tau[k];
-                        ht = em1 * -(sl.ma_c[k] * wgt * col / (tau * tau));
+                        const double tau = sl.ma_tau[k[i]];
+                        const double ht = hc * (sl.ma_c[k[i]] * dtc[i] / (tau * tau));
+                        ia.mat = __builtin_fma(wB[i], ht, ia.mat);
+                        ia.matR = __builtin_fma(wA[i], ht, ia.matR);
                     }
                 }
             }
-            ia.off += __builtin_fma(tB, ia.offR, wB);
-            ia.offR = __builtin_fma(tA, ia.offR, wA);
-            ia.mac += __builtin_fma(tB, ia.macR, lB * hc);
-            ia.macR = __builtin_fma(tA, ia.macR, lA * hc);
-            ia.mat += __builtin_fma(tB, ia.matR, lB * ht);
-            ia.matR = __builtin_fma(tA, ia.matR, lA * ht);
         }
-        // Stage 2: the planets one at a time, their derivatives from the
-        // stage-1 (sin E, cos E); one wave reduction per planet per tile.
+        // Stage 2: the planets' sums, from the stage-1 values.
+        reload_lds();
 #pragma unroll
-        for (int p = 0; p < KMAX; ++p) {
+        for (int p = 0; p < KM; ++p) {
             if (p < md.K) {
                 const PlanetC& pc = sl.planet[p];
-                double f[5];    // every lane (see stage 1)
-                {
-                    const double e = pc.e;
-                    const double rD = rcp_path<PREC>(__builtin_fma(e, -cE[p], 1.0));
-                    const double uu = cE[p] - e, vv = pc.bq * sE[p];
-                    const double sfw = __builtin_fma(vv, pc.cw, uu * pc.sw) * rD;    // sin(f + w)
-                    const double cfw = __builtin_fma(uu, pc.cw, -(vv * pc.sw)) * rD; // cos(f + w)
-                    const double Ks = pc.K * sfw;
-                    const double fM = -(Ks * pc.bq) * (rD * rD);
-                    f[0] = fM * (tp ? t - pc.tp : t);
-                    f[1] = fM;
-                    f[2] = __builtin_fma(-Ks, sE[p] * rD * __builtin_fma(pc.bq, rD, pc.ibq), pc.K * pc.cw);
-                    f[3] = -pc.K * __builtin_fma(e, pc.sw, sfw);
-                    f[4] = __builtin_fma(e, pc.cw, cfw);
+                const double e = pc.e, sw = pc.sw, bc = pc.bq * pc.cw;
+                double s[NE], q[NE];
+#pragma unroll
+                for (int i = 0; i < NE; ++i) {
+                    s[i] = __builtin_fma(C[p][i], sw, S[p][i] * bc);            // sin(f + w)
+                    q[i] = __builtin_fma(e, C[p][i], 1.0);                      // b^2 / D
                 }
-                // the B parts (one reduction for both cases), then with the MA
-                // the A parts, only where some lane's A is not negligible
-                const double b5[5] = {wB * f[0], wB * f[1], wB * f[2], wB * f[3], wB * f[4]};
-                const double sb = wave_reduce5(b5, lane);
-                double sa = 0.0;
-                if (ma && needA) {
-                    const double a5[5] = {wA * f[0], wA * f[1], wA * f[2], wA * f[3], wA * f[4]};
-                    sa = wave_reduce5(a5, lane);
-                }
-                if (ri5 >= 0) {
-                    const int e = 5 * p + ri5;
-                    if (ma) {
-                        const double R0 = wnatR[e];
-                        wnat[e] += __builtin_fma(tB, R0, sb);
-                        wnatR[e] = __builtin_fma(tA, R0, sa);
-                    } else {
-                        wnat[e] += sb;
+                auto sums = [&](const double (&w)[NE], double (&v)[5]) {
+#pragma unroll
+                    for (int i = 0; i < NE; ++i) {
+                        const double x = w[i] * s[i], xm = x * q[i] * q[i], xs = x * S[p][i];
+                        const double tau = tp ? t[i] - pc.tp : t[i];
+                        v[0] = i ? __builtin_fma(xm, tau, v[0]) : xm * tau;
+                        v[1] = i ? v[1] + xm : xm;
+                        v[2] = i ? __builtin_fma(xs, q[i], v[2] + xs) : __builtin_fma(xs, q[i], xs);
+                        v[3] = i ? __builtin_fma(w[i], C[p][i], v[3]) : w[i] * C[p][i];
+                        v[4] = i ? __builtin_fma(w[i], S[p][i], v[4]) : w[i] * S[p][i];
                     }
+                };
+                double v[5];
+                sums(wB, v);
+                acc4[p] += swap_add16(swap_add32(v[0], v[1]), swap_add32(v[2], v[3]));
+                acc1[p] += v[4];
+                if (needA) {        // the A parts, only where some lane's A is not negligible
+                    double a5[5];
+                    sums(wA, a5);
+                    wave_reduce_add5(a5, wnatR + 5 * p, lane, ri5);
                 }
             }
         }
         if (md.acc) {
-            double xq[AMAX] = {0.0, 0.0, 0.0, 0.0};
-            if (valid) {
-                const double x = t - md.t0;
+            double b4[AMAX] = {0.0, 0.0, 0.0, 0.0}, a4[AMAX] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                const double x = t[i] - md.t0;
                 double xp = x;
 #pragma unroll
                 for (int q = AMAX - 1; q >= 0; --q) {
                     if (q < md.acc) {
-                        xq[q] = xp;
+                        b4[q] = __builtin_fma(wB[i], xp, b4[q]);
+                        a4[q] = __builtin_fma(wA[i], xp, a4[q]);
                         xp *= x;
                     }
                 }
             }
-            const double b4[AMAX] = {wB * xq[0], wB * xq[1], wB * xq[2], wB * xq[3]};
-            if (!ma) {
-                wave_reduce_add4(b4, md.acc, wnat + WN_ACC, ri4);
-            } else {
-                const double sb = wave_reduce4(b4);
-                double sa = 0.0;
-                if (needA) {
-                    const double a4[AMAX] = {wA * xq[0], wA * xq[1], wA * xq[2], wA * xq[3]};
-                    sa = wave_reduce4(a4);
-                }
-                if (ri4 >= 0 && ri4 < md.acc) {
-                    const int e = WN_ACC + ri4;
-                    const double R0 = wnatR[e];
-                    wnat[e] += __builtin_fma(tB, R0, sb);
-                    wnatR[e] = __builtin_fma(tA, R0, sa);
-                }
-            }
+            wave_reduce_add4(b4, md.acc, wnat + WN_ACC, ri4);
+            if (needA) wave_reduce_add4(a4, md.acc, wnatR + WN_ACC, ri4);
         }
+        parity ^= 1;
     }
-    ia.flush_ins<EXT>(wacc, wrst);
-    ia.flush_ma<EXT>(wacc, wrst);
+#pragma unroll
+    for (int p = 0; p < KM; ++p)
+        if (p < md.K) {
+            double c = acc4[p];         // the rows of 16 lanes hold the sums 0, 2, 1, 3 (wave_reduce4)
+            c += dpp_mov_f64<0x128>(c);
+            c += dpp_mov_f64<0x141>(c);
+            c += dpp_mov_f64<0xB1>(c);
+            c += dpp_mov_f64<0x4E>(c);
+            if (ri4 >= 0) wnat[5 * p + ri4] += c;
+            const double v4 = wave_sum(acc1[p]);
+            if (lane == 0) wnat[5 * p + 4] += v4;
+        }
+    ia.flush_all<EXT>(ma, wacc, wrst, lane);
     double ldet = log(prod) + (double)pexp * LN2;
     chi = wave_sum(chi);
     ldet = wave_sum(ldet);
     if (lane == 0) { s_scan.red[wave][0] = chi; s_scan.red[wave][1] = ldet; }
     __syncthreads();
     double c2 = 0.0, l2 = 0.0;
-    for (int w = 0; w < WPT; ++w) { c2 += s_scan.red[w][0]; l2 += s_scan.red[w][1]; }
+    for (int w = 0; w < NW; ++w) { c2 += s_scan.red[w][0]; l2 += s_scan.red[w][1]; }
     const double lnl_v = -0.5 * (c2 + l2) + md.lnl_const;
-    grad_finish<EXT, WPT>(md, sl, gl, s_gw, true, wave, wave, lane, lnl_v, b, out_lnl, out_grad, nonfinite, stale);
+    grad_finish<EXT, NW, true>(md, sl, gl, s_gw, true, wave, wave, lane, lnl_v, b, out_lnl, out_grad, nonfinite, stale);
 }
 
 // Each model runs the instance with only the features it uses: the terms
@@ -1145,20 +1262,26 @@ static void launch_grad_t(const ModelDev& md, const double* th, int64_t B, int64
                            lnl, grad, nf, scratch, stale);
 }
 
-// The single-pass kernel runs models whose MA order is at most 1; by
-// default only those with at least GRAD1_MIN_N epochs: it keeps one epoch
-// per lane, so shorter series would leave lanes idle where the two-pass
-// kernel takes fewer waves per vector.  emp_model_set_grad_kernel overrides
-// the choice per model.
-constexpr int GRAD1_NW = 4;
-constexpr int GRAD1_MIN_N = 4 * 64 * GRAD1_NW;
+// The single-pass kernel runs every model whose MA order is at most 1, unless
+// emp_model_set_grad_kernel asks for the two-pass one.  Two waves per vector:
+// measured against 4 (whose waves wait for one another at the scans' barriers)
+// and 1 (whose tiles of 128 epochs repeat the A parts' reductions most often):
+// 8192 vectors of 7 planets x 10^4 epochs with MA(1), mixed, 2.49 ms against
+// 2.61 and 2.79; 16,384 of 5 planets x 2000 epochs, FP64, 0.72 against 0.83 and
+// 0.86.  Short series take it too: 8192 vectors of 2 planets, FP64, 64 / 73 /
+// 108 / 150 us at 150 / 256 / 512 / 1000 epochs against the two-pass kernel's
+// 84 / 86 / 168 / 238 (7 planets with MA(1), mixed: 135 / 139 / 223 / 361
+// against 172 / 166 / 320 / 536).
+constexpr int GRAD1_NW = 2;
+// Below this many epochs the two-pass kernel used to be the default: a batch
+// whose eps rows would not fit the allocation-free entry point's scratch stays
+// refused there.
+constexpr int NOALLOC_TWO_PASS_N = 1024;
 
 static bool use_grad1(const EmpModel* m) {
     const ModelDev& md = m->dev;
     if (md.ma_active && md.ma_q > 1) return false;
-    if (m->grad_kernel == EMP_GRAD_KERNEL_SINGLE_PASS) return true;
-    if (m->grad_kernel == EMP_GRAD_KERNEL_TWO_PASS) return false;
-    return md.N >= GRAD1_MIN_N;
+    return m->grad_kernel != EMP_GRAD_KERNEL_TWO_PASS;
 }
 
 extern "C" int emp_model_set_grad_kernel(EmpModel* m, int32_t which) {
@@ -1221,11 +1344,15 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
     if (use_grad1(m)) {
         const ModelDev& md = m->dev;
         if (precision != 0 && precision != 1) { emp_set_error("bad precision"); return EMP_EINVAL; }
-#define EMP_CASE1(P, E, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, GRAD1_NW, T>), dim3((unsigned)B), dim3(64 * GRAD1_NW), 0, s, md, th, B, ld, lnl, grad, nf, stale)
-#define EMP_CASE1T(P, E) { if (model_tp(md)) EMP_CASE1(P, E, true); else EMP_CASE1(P, E, false); }
+#define EMP_CASE1(P, E, A, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, GRAD1_NW, M, T>), dim3((unsigned)B), dim3(64 * GRAD1_NW), 0, s, md, th, B, ld, lnl, grad, nf, stale)
+#define EMP_CASE1M(P, E, A, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, GRAD1_FEW, T); else if (md.K <= 6) EMP_CASE1(P, E, A, 6, T); else EMP_CASE1(P, E, A, KMAX, T); }
+#define EMP_CASE1A(P, E, T) { if (md.ma_active) EMP_CASE1M(P, E, true, T) else EMP_CASE1M(P, E, false, T) }
+#define EMP_CASE1T(P, E) { if (model_tp(md)) EMP_CASE1A(P, E, true) else EMP_CASE1A(P, E, false) }
         if (precision == 0) { if (has_post(md)) EMP_CASE1T(0, 1) else EMP_CASE1T(0, 0) }
         else { if (has_post(md)) EMP_CASE1T(1, 1) else EMP_CASE1T(1, 0) }
 #undef EMP_CASE1T
+#undef EMP_CASE1A
+#undef EMP_CASE1M
 #undef EMP_CASE1
         EMP_HIP(hipGetLastError());
         return EMP_OK;
@@ -1317,7 +1444,9 @@ extern "C" int emp_lnl_grad_batch_noalloc(EmpModel* m, const double* theta, int6
         return EMP_EINVAL;
     }
     if (flags & ~EMP_GRAD_MIXED) { emp_set_error("unknown flags 0x%x", (unsigned)flags); return EMP_EINVAL; }
-    const size_t need = emp_grad_scratch_doubles(m, B);
+    size_t need = emp_grad_scratch_doubles(m, B);
+    if (m->grad_kernel == EMP_GRAD_KERNEL_AUTO && m->dev.ma_active && m->dev.N < NOALLOC_TWO_PASS_N)
+        need = (size_t)B * (size_t)m->dev.N;
     if (need > EMP_NOALLOC_SCRATCH_DOUBLES) {
         emp_set_error("batch of %lld vectors needs %zu doubles of scratch; the allocation-free entry point holds %zu",
                       (long long)B, need, (size_t)EMP_NOALLOC_SCRATCH_DOUBLES);

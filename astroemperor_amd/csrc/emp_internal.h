@@ -72,15 +72,16 @@ struct ModelDev {
 };
 
 // Per-slot LDS scratch of the likelihood kernels.  KTE: the entry of the
-// mixed path's Kepler tables (ktab_start), float4 intervals or float2 nodes.
-template <class KTE>
+// Kepler tables (ktab_start), float4 intervals or float2 nodes.  KP: planets
+// it holds.
+template <class KTE, int KP = KMAX>
 struct SlotLDSt {
     double theta[MAXD];
-    PlanetC planet[KMAX];
+    PlanetC planet[KP];
     double gam[IMAX], jit2[IMAX], ma_c[IMAX], ma_tau[IMAX], jit[IMAX];
     double acc[AMAX];
     double cosw[CMAX][3];      // per cosine term: (amplitude, angular frequency, phase)
-    KTE ktab[KMAX][KT_N];      // mixed path: per planet, the Kepler table
+    KTE ktab[KP][KT_N];        // per planet, the Kepler table
     int ktab_mask;             // bits 4 p .. 4 p + 2: planet p's Kepler path flags (kt_flags)
 };
 

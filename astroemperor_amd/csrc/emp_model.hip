@@ -286,11 +286,14 @@ int emp_model_host(const EmpModelDesc* d, ModelHost* h) {
     }
     const int N = d->n_epochs;
     // Device order: per-instrument MA needs each instrument's time series
-    // contiguous; otherwise keep the caller's (time) order.
+    // contiguous, and the global MA the caller's (time) order.  Without a
+    // moving average the order is free: grouped by instrument, a lane of the
+    // adjoint meets another instrument a few times per series instead of at
+    // every other epoch (each change costs it a round of LDS atomics).
     const bool by_ins = ma_active && !d->ma_global;
     h->order.resize(N);
     for (int i = 0; i < N; ++i) h->order[i] = i;
-    if (by_ins) std::stable_sort(h->order.begin(), h->order.end(), [&](int a, int b) { return d->ins[a] < d->ins[b]; });
+    if (by_ins || !ma_active) std::stable_sort(h->order.begin(), h->order.end(), [&](int a, int b) { return d->ins[a] < d->ins[b]; });
     h->t.resize(N); h->y.resize(N); h->s2.resize(N); h->dt.resize(N); h->ins.resize(N);
     for (int i = 0; i < N; ++i) {
         const int o = h->order[i];

@@ -54,8 +54,8 @@ extern "C" {
 #define EMP_GRAD_MIXED 2    /* emp_lnl_grad_batch: the mixed path's Kepler solve (EMP_MIXED accuracy) */
 
 /* Precision of the likelihood path. */
-#define EMP_FP64 0          /* FP64 arithmetic (the Kepler starter's roots and reciprocals at FP32 accuracy, which
-                                the FP64 fifth-order correction removes): the drop-in path */
+#define EMP_FP64 0          /* FP64 arithmetic (the Kepler solve starts from an FP32-accurate estimate, whose error
+                                its FP64 step removes): the drop-in path */
 #define EMP_MIXED 1         /* FP32 Kepler iterations + FP64 phase, final step, accumulation */
 
 /* Prior kinds (support/priors/<Kind>.prior). */
@@ -140,8 +140,8 @@ int emp_model_eval(EmpModel* model, const double* theta, double* model_out, doub
 /* No reference counterpart: lnL and dlnL/dtheta[free]
  * for a batch, by a hand-written adjoint kernel (FP64; with EMP_GRAD_MIXED the
  * Kepler solve of the mixed path, FP32 start and one FP64 step). grad is [B, ndim].
- * The two-pass adjoint kernel (emp_model_set_grad_kernel: MA orders above 1,
- * series shorter than 1024 epochs by default) keeps, with an active MA term,
+ * The two-pass adjoint kernel (MA orders above 1, or on request:
+ * emp_model_set_grad_kernel) keeps, with an active MA term,
  * a device scratch of B x n_epochs doubles in the model (grown on demand,
  * freed with the model); the single-pass kernel needs none. */
 int emp_lnl_grad_batch(EmpModel* model, const double* theta, int64_t B, int64_t ld,
@@ -154,7 +154,9 @@ int emp_lnl_grad_batch(EmpModel* model, const double* theta, int64_t B, int64_t 
  * EMP_NOALLOC_SCRATCH_DOUBLES doubles (64 MiB) that each device the library
  * runs on holds until the process ends; a batch needing more (with an active
  * MA term in the two-pass kernel, B x n_epochs doubles) is refused with
- * EMP_EINVAL.  The single-pass kernel uses no scratch.  Same results as
+ * EMP_EINVAL, and so is one with an active MA term and EMP_GRAD_KERNEL_AUTO
+ * on a series shorter than 1024 epochs, although the single-pass kernel that
+ * runs it uses no scratch.  Same results as
  * emp_lnl_grad_batch, bit for bit.  flags: 0 or EMP_GRAD_MIXED
  * (EMP_HOST_POINTERS is refused).  Call with the model's device current.
  * Every call on one device shares that device's array, and each launch
@@ -171,8 +173,8 @@ int emp_model_set_waves_per_theta(EmpModel* model, int32_t waves_per_theta);
  * model.  No counterpart in the reference (its gradients, where a caller
  * wants them, are finite differences of my_likelihood); the two kernels
  * give the same lnL and gradients to rounding.
- *   EMP_GRAD_KERNEL_AUTO: single-pass when the MA order is at most 1 and the
- *     series has at least 1024 epochs, else two-pass;
+ *   EMP_GRAD_KERNEL_AUTO: single-pass when the MA order is at most 1, else
+ *     two-pass;
  *   EMP_GRAD_KERNEL_TWO_PASS: likelihood with the MA residuals stored
  *     (B x N doubles of scratch), then the epochs in reverse;
  *   EMP_GRAD_KERNEL_SINGLE_PASS: one pass, no scratch; EMP_EUNSUP for MA
