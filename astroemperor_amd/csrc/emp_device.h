@@ -85,6 +85,28 @@ __device__ __forceinline__ double dpp_shr_one_f64(double src) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// Value of the next lane (lane 63: `last`), of the previous one (lane 0:
+// `first`): wave_shl:1 (0x130) and wave_shr:1 (0x138).  Whole wave active.
+__device__ __forceinline__ double wave_next(double v, double last) { return dpp_f64<0x130, 0xf>(last, v); }
+__device__ __forceinline__ double wave_prev(double v, double first) { return dpp_f64<0x138, 0xf>(first, v); }
+
+// Orders the LDS accesses of one wave: what its lanes wrote is what they read
+// afterwards (the wave's LDS operations complete in order; this keeps the
+// compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// The waves of one vector meet: nothing to wait for with one wave, else the
+// whole workgroup.
+template <int WPT>
+__device__ __forceinline__ void vec_sync() {
+    if (WPT == 1) wave_sync();
+    else __syncthreads();
+}
+
 // Value of lane k (uniform k) in every lane.
 __device__ __forceinline__ double readlane_f64(double v, int k) {
     const long long bits = __double_as_longlong(v);
@@ -376,10 +398,11 @@ __device__ __forceinline__ int kt_flags(bool table, double e) {
 }
 // Planet p's flags from SlotLDS::ktab_mask (four bits per planet).
 __device__ __forceinline__ int kt_mode(int kmask, int p) { return (int)(((unsigned)kmask >> (4 * p)) & 7u); }
-// Building a table costs about as much as 64 FP64 planet-epochs, and saves
-// the FP32 Markley starter's ~40 extra operations per epoch: it pays from
-// about 256 epochs on.
-constexpr int KT_MIN_EPOCHS = 256;
+// Building a table costs a wave one FP32 Kepler solve (64 nodes, one per lane),
+// less than the extra operations of a start without it over one chunk of 64
+// epochs: sweeps of 512 systems of 50 to 2000 epochs (median 200) take 727 / 674 /
+// 650 us with tables from 256 / 128 / 64 epochs on (mixed), 865 / 754 / 718 FP64.
+constexpr int KT_MIN_EPOCHS = 64;
 
 // The cubic Hermite interpolant on [M_j, M_j+1] in Horner form: with
 // d = E_j+1 - E_j and the scaled slopes s0 = h E'_j, s1 = h E'_j+1,
@@ -653,13 +676,14 @@ __device__ __forceinline__ void planet_sc(const PlanetC& pc, const SinCosTab& tb
     for (int i = 0; i < NE; ++i) sE[i] = __builtin_copysign(sE[i], M[i]);
 }
 
-// Planet term at time t (see planet_sc).
-template <int PREC, class KTE>
-__device__ __forceinline__ double planet_mu(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, double t,
-                                           bool tp, int kmode) {
-    double sE[1], cE[1], rD[1];
-    planet_sc<PREC, 1>(pc, tb, kt, {t}, sE, cE, rD, tp, kmode);
-    return __builtin_fma(pc.c1, cE[0], pc.c2 * sE[0]) * rD[0];
+// Planet term at the lane's NE times, added to mu (see planet_sc).
+template <int PREC, int NE, class KTE>
+__device__ __forceinline__ void planet_mu(const PlanetC& pc, const SinCosTab& tb, const KTE* kt, const double (&t)[NE],
+                                          double (&mu)[NE], bool tp, int kmode) {
+    double sE[NE], cE[NE], rD[NE];
+    planet_sc<PREC, NE>(pc, tb, kt, t, sE, cE, rD, tp, kmode);
+#pragma unroll
+    for (int i = 0; i < NE; ++i) mu[i] = __builtin_fma(__builtin_fma(pc.c1, cE[i], pc.c2 * sE[i]), rD[i], mu[i]);
 }
 
 // ----------------------------------------------------------------------------

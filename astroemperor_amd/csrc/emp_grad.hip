@@ -192,14 +192,6 @@ __device__ __forceinline__ void post_accumulate(const ModelDev& md, const SL& sl
     }
 }
 
-// MA(1) multiplier of epoch n (device order) from its instrument and its MA
-// column (the fixed-timescale weight, or dt with -1 at a segment start).
-template <class SL>
-__device__ __forceinline__ double ma_mult(const ModelDev& md, const SL& sl, int k, double col) {
-    if (md.ma_wfixed) return -(sl.ma_c[k] * col);
-    return col < 0.0 ? 0.0 : -(sl.ma_c[k] * exp(-col / sl.ma_tau[k]));
-}
-
 // Adjoint of MA(q), q >= 2, for one chunk (epochs in reverse): with
 // a_{n,c} the forward multipliers, lambda_n = u_n + sum_{c<q} a_{n+1+c,c}
 // lambda_{n+1+c}, an affine map on the state (lambda_n, ..., lambda_{n+Q-1})
@@ -399,13 +391,13 @@ __device__ __forceinline__ double ma_chunk_w(const ModelDev& md, const SL& sl, c
         lam_carry = __shfl(lam, 0, 64);
     } else {
         wave_affine_suffix_scan(sa, sb, lane);
-        if (lane == 0) { sc.tot[parity][wave][0] = sa; sc.tot[parity][wave][1] = sb; }
+        if (lane == 0) sc.tot[parity][wave] = make_double2(sa, sb);
         __syncthreads();
         const int w0 = wave - wsub;
         double pa = 1.0, pb = 0.0;
         for (int w = WPT - 1; w >= 0; --w) {
             if (w == wsub) lam = __builtin_fma(sa, __builtin_fma(pa, lam_carry, pb), sb);
-            const double ta = sc.tot[parity][w0 + w][0], tbv = sc.tot[parity][w0 + w][1];
+            const double ta = sc.tot[parity][w0 + w].x, tbv = sc.tot[parity][w0 + w].y;
             pb = __builtin_fma(ta, pb, tbv);
             pa = ta * pa;
         }
@@ -471,7 +463,9 @@ __device__ __forceinline__ double plain_w(const ModelDev& md, const SL& sl, cons
     constexpr bool POST = EXT >= 1;
     const double t = tl.t[j];
     const int k = tl.ins[j];
-    const double mu = epoch_mu<PREC>(md, sl, tl.tab, t, k, kmask);
+    double mu1[1];
+    epoch_mu<PREC, 1>(md, sl, tl.tab, {t}, {k}, kmask, mu1);
+    const double mu = mu1[0];
     const double err2 = tl.s2[j] + sl.jit2[k];
     const double cs = (POST && has_post(md)) ? epoch_post(md, sl, tl.tab, t, tb + j, k) : 0.0;
     const double r = tl.y[j] - mu - cs;
@@ -621,6 +615,13 @@ __device__ __forceinline__ void grad_finish(const ModelDev& md, const SL& sl, Gr
     }
 }
 
+// slot_prepare for workgroups of several vectors, whose waves all wait.
+template <int WPT, class SL>
+__device__ __forceinline__ void slot_prepare_wg(const ModelDev& md, SL& sl, bool live, int wsub, int lane) {
+    slot_prepare<WPT>(md, sl, live, wsub, lane);
+    __syncthreads();
+}
+
 // Adjoint kernel.  Per tile (forward without the MA, in reverse with it):
 // stage 1 finds w = dlnL/dmu of each lane's epochs (CPT chunks of 64 WPT
 // epochs, held in registers), stage 2 then takes the planets one at a time,
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
     __shared__ GradWaveLDS<EXT> s_gw;
     __shared__ TileLDS s_tile;
     __shared__ ScanLDS s_scan;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int slot = wave / WPT, wsub = wave % WPT;
     const int g = wsub * 64 + lane;
     const int64_t b = (int64_t)blockIdx.x * SLOTS + slot;
@@ -663,9 +664,9 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
     double* wnat = s_gw.nat[wave];
     for (int j = lane; j < GW::N; j += 64) wacc[j] = 0.0;
     for (int j = lane; j < WN_N; j += 64) wnat[j] = 0.0;
-    tab_load(md, s_tile);
+    tab_load(md, s_tile.tab);
     __syncthreads();
-    slot_prepare<PREC, WPT>(md, sl, s_tile, live, wsub, lane);
+    slot_prepare_wg<WPT>(md, sl, live, wsub, lane);
     const int kmask = wave_uniform(sl.ktab_mask);
     const bool tp = model_tp(md);
 
@@ -674,8 +675,7 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
     double lnl_v = 0.0;
     if (ma) {
         // Pass 1: the likelihood, storing eps.
-        lnl_v = block_lnl<PREC, WPT, false, true, true, POST>(md, sl, s_tile, s_scan, live, wsub, nullptr, nullptr,
-                                                             false, eps);
+        lnl_v = vec_lnl<PREC, WPT, false, true, EXT>(md, sl, s_tile.tab, s_scan, live, wsub, nullptr, nullptr, eps);
         __syncthreads();   // eps rows written by every wave of the slot
     }
     double chi = 0.0, prod = 1.0;
@@ -871,11 +871,6 @@ struct InsAcc1 {
         }
     }
 };
-
-// Value of the next lane (lane 63: `last`), of the previous one (lane 0:
-// `first`): DPP wave_shl:1 and wave_shr:1.  Whole wave active.
-__device__ __forceinline__ double wave_next(double v, double last) { return dpp_f64<0x130, 0xf>(last, v); }
-__device__ __forceinline__ double wave_prev(double v, double first) { return dpp_f64<0x138, 0xf>(first, v); }
 
 // The planets' constants are read from LDS where they are used: without this
 // the compiler keeps those of all planets in registers over the tiles.

@@ -64,7 +64,7 @@ struct ModelDev {
     const int* block_start;           // [nblocks + 1]
     const EmpPriorTerm* ecc_prior;    // [K]
     const int* pseq;                  // [npseq] prior terms in summation order (see PSEQ_*)
-    const PseqEntry* pseq_e;          // [npseq] the same, resolved (single-model engines; null in batches)
+    const PseqEntry* pseq_e;          // [npseq] the same, resolved
     int npseq;
     const double2* sctab;             // [SC_N + 1] (sin, cos) of k pi / SC_N
     double lnl_const;                 // -0.5 ln(2 pi) N
@@ -123,11 +123,10 @@ struct ModelHost {
     std::vector<EmpPriorTerm> prior, ecc;
 };
 int emp_model_host(const EmpModelDesc* d, ModelHost* h);
-// Every device array a likelihood kernel may read is set (pseq_e is only
-// used by the single-model engines and may be null).
+// Every device array a kernel may read is set.
 inline bool emp_model_dev_complete(const emp::ModelDev& m) {
     return m.t && m.y && m.s2 && m.dt && m.ins && m.inv_free && m.free_idx && m.fixed_val && m.prior &&
-           m.block_start && m.ecc_prior && m.pseq && m.sctab && m.sai && m.sai_base;
+           m.block_start && m.ecc_prior && m.pseq && m.pseq_e && m.sctab && m.sai && m.sai_base;
 }
 // (sin, cos) of k pi / SC_N, k = 0..SC_N, rounded from extended precision.
 void emp_sincos_table(std::vector<double2>& tab);
@@ -145,7 +144,7 @@ bool emp_fault_injected();
 // Likelihood launchers (emp_model.hip), used by the PT engine as well.
 // Waves per vector for B vectors: batched likelihoods, or (halfstep) the
 // PT half-step's proposals.
-int emp_pick_wpt(const EmpModel* m, int64_t B, int precision, bool halfstep = false);
+int emp_pick_wpt(const EmpModel* m, int64_t B, bool halfstep = false);
 int emp_launch_lnl(const EmpModel* m, const double* d_theta, int64_t B, int64_t ld,
                    double* d_lnl, int precision, int wpt, hipStream_t s);
 int emp_launch_prior(const EmpModel* m, const double* d_theta, int64_t B, int64_t ld,

@@ -1,11 +1,12 @@
-// Likelihood building blocks shared by the batched-lnL, model-eval and PT
-// kernels.
+// Likelihood building blocks shared by the batched-lnL, model-eval, adjoint
+// and PT kernels.
 //
-// Launch geometry: one workgroup = 8 wave64s.  The workgroup owns SLOTS =
-// 8 / WPT parameter vectors; each vector is processed by WPT waves whose
-// 64*WPT lanes stride over the epochs.  Epoch data (t, y, yerr^2, MA time
-// step, instrument tag) is staged into LDS in tiles of TILE epochs and shared
-// by all slots of the workgroup.
+// Launch geometry: a parameter vector belongs to WPT waves.  With WPT > 1 the
+// workgroup is those waves; with one wave per vector the waves of a workgroup
+// share the sin/cos table and nothing else.  The vector's waves walk the epochs
+// in chunks, each lane with two consecutive epochs (one in a last chunk of at
+// most 64 WPT), read straight from global memory: the data of every vector are
+// the same few KB to hundreds of KB, in L1 and L2.
 #pragma once
 #include "emp_internal.h"
 
@@ -58,17 +59,17 @@ __device__ inline double prior_seq(const ModelDev& md, const double* th) {
     return lp;
 }
 
-// Per-slot constants (planets, instruments, acceleration) into LDS.
-// Called by the slot's first wave; the caller synchronises afterwards.
+// Planet p's constants of the full parameter vector th.
+__device__ __forceinline__ PlanetC planet_slot(const ModelDev& md, const double* th, int p) {
+    PlanetC pc = planet_setup(th + md.off_kep + 5 * p, md.param, md.use_c);
+    pc.ktab = md.N >= KT_MIN_EPOCHS && pc.e <= KT_EMAX;
+    return pc;
+}
+
+// The slot's other constants (instruments, acceleration, cosine terms) and the
+// planets' Kepler path flags, kf those of planet `lane`.  Called by a whole wave.
 template <class SL>
-__device__ inline void slot_setup(const ModelDev& md, SL& sl, int lane) {
-    int kf = 0;
-    if (lane < md.K) {
-        PlanetC pc = planet_setup(sl.theta + md.off_kep + 5 * lane, md.param, md.use_c);
-        pc.ktab = md.N >= KT_MIN_EPOCHS && pc.e <= KT_EMAX;
-        kf = kt_flags(pc.ktab != 0, pc.e);
-        sl.planet[lane] = pc;
-    }
+__device__ __forceinline__ void slot_rest(const ModelDev& md, SL& sl, int lane, int kf) {
     // the whole wave calls these: flag bit b of planet p to mask bit 4 p + b
     unsigned m = 0;
     for (int b = 0; b < 3; ++b) {
@@ -107,6 +108,19 @@ __device__ inline void slot_setup(const ModelDev& md, SL& sl, int lane) {
     }
 }
 
+// Per-slot constants (planets, instruments, acceleration) into LDS.
+// Called by the slot's first wave; the caller synchronises afterwards.
+template <class SL>
+__device__ inline void slot_setup(const ModelDev& md, SL& sl, int lane) {
+    int kf = 0;
+    if (lane < md.K) {
+        const PlanetC pc = planet_slot(md, sl.theta, lane);
+        kf = kt_flags(pc.ktab != 0, pc.e);
+        sl.planet[lane] = pc;
+    }
+    slot_rest(md, sl, lane, kf);
+}
+
 struct TileLDS {
     double t[TILE], y[TILE], s2[TILE], dt[TILE];
     int ins[TILE];
@@ -114,8 +128,8 @@ struct TileLDS {
 };
 
 // The sin/cos table is read by every planet-epoch; load it once per workgroup.
-__device__ __forceinline__ void tab_load(const ModelDev& md, TileLDS& tl) {
-    for (int j = threadIdx.x; j <= SC_N; j += blockDim.x) tl.tab.v[j] = md.sctab[j];
+__device__ __forceinline__ void tab_load(const ModelDev& md, SinCosTab& tab) {
+    for (int j = threadIdx.x; j <= SC_N; j += blockDim.x) tab.v[j] = md.sctab[j];
 }
 
 __device__ __forceinline__ void tile_load(const ModelDev& md, TileLDS& tl, int tb, int tn) {
@@ -128,50 +142,18 @@ __device__ __forceinline__ void tile_load(const ModelDev& md, TileLDS& tl, int t
     }
 }
 
-// One epoch of a tile in registers.  Every launch that stages tiles has at
-// least TILE threads, so thread j holds epoch tb + j of the tile at tb: its
-// global loads are issued a tile ahead and stored to LDS when the tile's
-// turn comes.
-struct EpochRegs {
-    double t, y, s2, dt;
-    int ins;
-};
-
-__device__ __forceinline__ void epoch_prefetch(const ModelDev& md, int tb, EpochRegs& r) {
-    const int j = threadIdx.x, n = tb + j;
-    if (j < TILE && n < md.N) {
-        r.t = md.t[n];
-        r.y = md.y[n];
-        r.s2 = md.s2[n];
-        r.ins = md.ins[n];
-        r.dt = md.ma_active ? md.dt[n] : 0.0;
-    }
-}
-
-__device__ __forceinline__ void epoch_store(const ModelDev& md, TileLDS& tl, int tb, const EpochRegs& r) {
-    const int j = threadIdx.x;
-    if (j < TILE && tb + j < md.N) {
-        tl.t[j] = r.t;
-        tl.y[j] = r.y;
-        tl.s2[j] = r.s2;
-        tl.ins[j] = r.ins;
-        if (md.ma_active) tl.dt[j] = r.dt;
-    }
-}
-
 // Per-slot constants, then the per-vector Kepler tables, one planet per wave
-// of the slot.  The sin/cos table must already be in LDS.
-// All threads of the workgroup call this (it holds two barriers).
-template <int PREC, int WPT, class SL>
-__device__ __forceinline__ void slot_prepare(const ModelDev& md, SL& sl, const TileLDS& tl, bool live,
-                                             int wsub, int lane) {
+// of the slot.  Every wave of the vector calls this; the vector's theta must be
+// in the slot and visible to them.
+template <int WPT, class SL>
+__device__ __forceinline__ void slot_prepare(const ModelDev& md, SL& sl, bool live, int wsub, int lane) {
     if (live && wsub == 0) slot_setup(md, sl, lane);
-    __syncthreads();
+    vec_sync<WPT>();
     if (live) {
         for (int p = wsub; p < md.K; p += WPT)
             if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
     }
-    __syncthreads();
+    vec_sync<WPT>();
 }
 
 // A value that is the same in every lane of the wave (every kernel keeps
@@ -179,30 +161,38 @@ __device__ __forceinline__ void slot_prepare(const ModelDev& md, SL& sl, const T
 // branch on it is a scalar branch.
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Vectors per workgroup of the kernels whose vectors are independent: with one
+// wave per vector four of them share the workgroup's sin/cos table.
+constexpr int vecs_per_wg(int wpt) { return wpt == 1 ? 4 : 1; }
+
 // The model's planets are parameterised by the time of periastron
 // (block_repo.py:23-31, parameterisations 3 and 4).
 __host__ __device__ __forceinline__ bool model_tp(const ModelDev& md) { return md.param == 3 || md.param == 4; }
 
-// Model value (planets + offset + acceleration) of one epoch.  kmask: the
-// slot's SlotLDS::ktab_mask as a wave-uniform scalar.
-template <int PREC, class SL>
-__device__ __forceinline__ double epoch_mu(const ModelDev& md, const SL& sl, const SinCosTab& tb, double t, int k,
-                                           int kmask) {
-    double mu = sl.gam[k];
-    if (md.acc) {
-        const double x = t - md.t0;
-        double v = 0.0;
-        for (int a = 0; a < md.acc; ++a) v = __builtin_fma(v, x, sl.acc[a]);
-        mu += v * x;
+// Model value (planets + offset + acceleration) of the lane's NE epochs.
+// kmask: the slot's SlotLDS::ktab_mask as a wave-uniform scalar.
+template <int PREC, int NE, class SL>
+__device__ __forceinline__ void epoch_mu(const ModelDev& md, const SL& sl, const SinCosTab& tb, const double (&t)[NE],
+                                         const int (&k)[NE], int kmask, double (&mu)[NE]) {
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        mu[i] = sl.gam[k[i]];
+        if (md.acc) {
+            const double x = t[i] - md.t0;
+            double v = 0.0;
+            for (int a = 0; a < md.acc; ++a) v = __builtin_fma(v, x, sl.acc[a]);
+            mu[i] += v * x;
+        }
     }
     // The planet loop twice, one copy per parameterisation (a model-wide
     // choice), so that no planet-epoch branches on it.
     if (model_tp(md)) {
-        for (int p = 0; p < md.K; ++p) mu += planet_mu<PREC>(sl.planet[p], tb, sl.ktab[p], t, true, kt_mode(kmask, p));
+        for (int p = 0; p < md.K; ++p)
+            planet_mu<PREC, NE>(sl.planet[p], tb, sl.ktab[p], t, mu, true, kt_mode(kmask, p));
     } else {
-        for (int p = 0; p < md.K; ++p) mu += planet_mu<PREC>(sl.planet[p], tb, sl.ktab[p], t, false, kt_mode(kmask, p));
+        for (int p = 0; p < md.K; ++p)
+            planet_mu<PREC, NE>(sl.planet[p], tb, sl.ktab[p], t, mu, false, kt_mode(kmask, p));
     }
-    return mu;
 }
 
 // Phase freq * t + phase of cosine term c, rounded as numpy rounds
@@ -218,11 +208,12 @@ __device__ __forceinline__ double cos_phase(const SL& sl, int c, double t) {
 // 2628-2650), so the MA residuals do not contain them.
 __host__ __device__ inline bool has_post(const ModelDev& md) { return md.n_cos > 0 || md.sai_w > 0; }
 
-// Model features the common models do not use: the terms added after the MA
-// and MA orders above 1.  Kernels come in two instances, with and without
-// them, so that the common instance keeps its register budget.
-__host__ __device__ inline bool needs_ext(const ModelDev& md) {
-    return has_post(md) || (md.ma_active && md.ma_q > 1);
+// Model features the common models do not use: 0 none of them, 1 terms added
+// after the MA (activity and cosine terms), 2 also MA orders above 1.  Kernels
+// come in instances that compile the others out, so that the common ones keep
+// their register budget.
+__host__ __device__ inline int model_ext(const ModelDev& md) {
+    return md.ma_active && md.ma_q > 1 ? 2 : has_post(md) ? 1 : 0;
 }
 
 // Their sum at epoch n (device order; time t, instrument k): the activity
@@ -316,45 +307,70 @@ __device__ __forceinline__ void affq_step(double (&m)[Q][Q], double (&v)[Q]) {
     }
 }
 
-// One chunk of the order-q MA: the lane's epoch (valid: j of the tile at tb,
-// time tj, instrument k, residual r) and the state carried in from the
-// previous chunk (`carry`, updated).  Reads the tile only before the first
-// barrier.  Returns eps of the lane's epoch.  Whole wave active; with WPT > 1
-// all waves of the workgroup call this together (one barrier).
-template <int Q, int WPT, class SL>
-__device__ __forceinline__ double ma_chunk_q(const ModelDev& md, const SL& sl, const TileLDS& tl, bool valid,
-                                             int j, int tb, double tj, int k, double r, int lane, int wave,
-                                             int wsub, int& parity, double (&carry)[4]) {
-    __shared__ double qtot[2][MAX_WAVES][Q * Q + Q];
-    double m[Q][Q], v[Q];
+// The companion map of epoch n (time t, instrument k, residual r); the
+// identity for an epoch past the series' end.
+template <int Q, class SL>
+__device__ __forceinline__ void maq_map(const ModelDev& md, const SL& sl, bool valid, int n, double t, int k, double r,
+                                        double (&m)[Q][Q], double (&v)[Q]) {
 #pragma unroll
     for (int a = 0; a < Q; ++a) {
         v[a] = 0.0;
 #pragma unroll
         for (int b = 0; b < Q; ++b) m[a][b] = a == b ? 1.0 : 0.0;
     }
-    if (valid) {
-        const int q = md.ma_q;
-        const double* ph = sl.theta + md.off_ma + 2 * q * (md.ma_global ? 0 : k);
-        const int n = tb + j;
+    if (!valid) return;
+    const int q = md.ma_q;
+    const double* ph = sl.theta + md.off_ma + 2 * q * (md.ma_global ? 0 : k);
 #pragma unroll
-        for (int c = 0; c < Q; ++c) {
-            double a = 0.0;
-            const int n1 = n - 1 - c, j1 = j - 1 - c;
-            if (c < q && n1 >= 0) {
-                const int k1 = j1 >= 0 ? tl.ins[j1] : md.ins[n1];
-                if (md.ma_global || k1 == k) {
-                    const double t1 = j1 >= 0 ? tl.t[j1] : md.t[n1];
-                    a = -(ph[2 * c] * exp(-__builtin_fabs(tj - t1) / ph[2 * c + 1]));
-                }
-            }
-            m[0][c] = a;
+    for (int c = 0; c < Q; ++c) {
+        double a = 0.0;
+        const int n1 = n - 1 - c;
+        if (c < q && n1 >= 0 && (md.ma_global || md.ins[n1] == k))
+            a = -(ph[2 * c] * exp(-__builtin_fabs(t - md.t[n1]) / ph[2 * c + 1]));
+        m[0][c] = a;
+    }
+#pragma unroll
+    for (int a = 1; a < Q; ++a)
+#pragma unroll
+        for (int b = 0; b < Q; ++b) m[a][b] = b == a - 1 ? 1.0 : 0.0;
+    v[0] = r;
+}
+
+// One chunk of the order-q MA: the lane's NE epochs from n0 on (their times,
+// instruments, residuals) and the state carried in from the previous chunk
+// (`carry`, updated).  eps of the lane's epochs.  Whole wave active; with WPT > 1
+// all waves of the workgroup call this together (one barrier).
+template <int Q, int WPT, int NE, class SL>
+__device__ __forceinline__ void ma_chunk_q(const ModelDev& md, const SL& sl, const bool (&valid)[NE], int n0,
+                                           const double (&t)[NE], const int (&k)[NE], const double (&r)[NE], int lane,
+                                           int wave, int wsub, int& parity, double (&carry)[4], double (&eps)[NE]) {
+    __shared__ double qtot[2][MAX_WAVES][Q * Q + Q];
+    double m0[Q][Q], v0[Q], m[Q][Q], v[Q];
+    maq_map<Q>(md, sl, valid[0], n0, t[0], k[0], r[0], m0, v0);
+    if constexpr (NE == 1) {
+#pragma unroll
+        for (int a = 0; a < Q; ++a) {
+            v[a] = v0[a];
+#pragma unroll
+            for (int b = 0; b < Q; ++b) m[a][b] = m0[a][b];
         }
+    } else {
+        double m1[Q][Q], v1[Q];
+        maq_map<Q>(md, sl, valid[1], n0 + 1, t[1], k[1], r[1], m1, v1);
 #pragma unroll
-        for (int a = 1; a < Q; ++a)
+        for (int a = 0; a < Q; ++a) {
+            double acc = v1[a];
 #pragma unroll
-            for (int b = 0; b < Q; ++b) m[a][b] = b == a - 1 ? 1.0 : 0.0;
-        v[0] = r;
+            for (int b = 0; b < Q; ++b) acc = __builtin_fma(m1[a][b], v0[b], acc);
+            v[a] = acc;
+#pragma unroll
+            for (int c = 0; c < Q; ++c) {
+                double e = 0.0;
+#pragma unroll
+                for (int b = 0; b < Q; ++b) e = __builtin_fma(m1[a][b], m0[b][c], e);
+                m[a][c] = e;
+            }
+        }
     }
     affq_step<Q, 0x111, 0xf>(m, v);
     affq_step<Q, 0x112, 0xf>(m, v);
@@ -401,7 +417,7 @@ __device__ __forceinline__ double ma_chunk_q(const ModelDev& md, const SL& sl, c
         for (int a = 0; a < Q; ++a) carry[a] = s_all[a];
         parity ^= 1;
     }
-    double st[Q];
+    double st[Q];                       // the state after the lane's last epoch
 #pragma unroll
     for (int a = 0; a < Q; ++a) {
         double acc = v[a];
@@ -413,7 +429,13 @@ __device__ __forceinline__ double ma_chunk_q(const ModelDev& md, const SL& sl, c
 #pragma unroll
         for (int a = 0; a < Q; ++a) carry[a] = readlane_f64(st[a], 63);
     }
-    return st[0];
+    eps[NE - 1] = st[0];
+    if constexpr (NE == 2) {
+        double e = v0[0];
+#pragma unroll
+        for (int b = 0; b < Q; ++b) e = __builtin_fma(m0[0][b], wave_prev(st[b], sin_[b]), e);
+        eps[0] = e;
+    }
 }
 
 // One suffix step within rows of 16 lanes: lane i composes with lane i + n
@@ -457,131 +479,152 @@ __device__ __forceinline__ void wave_affine_suffix_scan(double& a, double& b, in
 }
 
 struct ScanLDS {
-    double tot[2][MAX_WAVES][2];
+    double2 tot[2][MAX_WAVES];     // per wave: its chunk's affine map (double-buffered)
     double red[MAX_WAVES][2];
 };
 
-// lnL of the slot's parameter vector.  All threads of the workgroup must
-// call this together (it contains workgroup barriers); `live` == false makes
-// a slot skip the arithmetic while still taking part in the barriers.  The
-// slot must be prepared (slot_prepare) and the sin/cos table loaded.
-// With WRITE the per-epoch model and err2 are stored (device order); with
-// WEPS the per-epoch MA-filtered residual eps (= r without MA; before the
-// terms added after the MA are taken off).
-// `resident`: the caller has already staged all epochs (md.N <= TILE) in tl.
-// `first`: the first tile's epochs, already loaded by the caller (else loaded
-// here).  With PF the next tile's loads are issued a tile ahead (launches
-// have at least TILE threads); without, each tile is loaded when its turn
-// comes (fewer registers).  POST = false compiles out the features of
-// needs_ext: the terms added after the moving average (activity and cosine
-// terms) and MA orders above 1.
-template <int PREC, int WPT, bool WRITE, bool WEPS = false, bool PF = true, bool POST = true, class SL>
-__device__ double block_lnl(const ModelDev& md, const SL& sl, TileLDS& tl, ScanLDS& sc,
-                            bool live, int wsub, double* out_model, double* out_err2, bool resident = false,
-                            double* out_eps = nullptr, const EpochRegs* first = nullptr) {
+// MA(1) multiplier of an epoch from its instrument and its MA column (the
+// fixed-timescale weight, or dt with -1 at a segment start).
+template <class SL>
+__device__ __forceinline__ double ma_mult(const ModelDev& md, const SL& sl, int k, double col) {
+    if (md.ma_wfixed) return -(sl.ma_c[k] * col);
+    return col < 0.0 ? 0.0 : -(sl.ma_c[k] * exp(-col / sl.ma_tau[k]));
+}
+
+// One chunk of the likelihood: NE consecutive epochs per lane from cb on.
+// Adds to the lane's chi^2 and log-determinant product; carries the MA state.
+template <int PREC, int WPT, bool WRITE, bool WEPS, int EXT, int NE, class SL>
+__device__ __forceinline__ void lnl_chunk(const ModelDev& md, const SL& sl, const SinCosTab& tab, ScanLDS& sc,
+                                          bool live, int cb, int lane, int wave, int wsub, int kmask, double& chi,
+                                          double& prod, int& pexp, double& carry, double (&qcarry)[4], int& parity,
+                                          double* out_model, double* out_err2, double* out_eps) {
+    const int n0 = cb + NE * (wsub * 64 + lane);
+    double t[NE], y[NE], err2[NE], dtc[NE], r[NE], mu[NE];
+    int k[NE];
+    bool valid[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        const int n = n0 + i;
+        valid[i] = live && n < md.N;
+        t[i] = y[i] = dtc[i] = r[i] = mu[i] = 0.0;
+        err2[i] = 1.0;
+        k[i] = 0;
+        if (valid[i]) {
+            t[i] = md.t[n];
+            k[i] = md.ins[n];
+            y[i] = md.y[n];
+            err2[i] = md.s2[n];
+            if (md.ma_active) dtc[i] = md.dt[n];
+        }
+    }
+    // a wave past the series' end only takes part in the scan's barrier
+    if (live && cb + NE * (wsub * 64) < md.N) {
+        epoch_mu<PREC, NE>(md, sl, tab, t, k, kmask, mu);
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            if (valid[i]) {
+                err2[i] += sl.jit2[k[i]];
+                r[i] = y[i] - mu[i];
+            }
+        }
+    }
+    double eps[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) eps[i] = r[i];
+    if (EXT == 2 && md.ma_active && md.ma_q > 1) {
+        if (md.ma_q == 2) ma_chunk_q<2, WPT, NE>(md, sl, valid, n0, t, k, r, lane, wave, wsub, parity, qcarry, eps);
+        else ma_chunk_q<4, WPT, NE>(md, sl, valid, n0, t, k, r, lane, wave, wsub, parity, qcarry, eps);
+    } else if (md.ma_active) {
+        double am[NE];
+#pragma unroll
+        for (int i = 0; i < NE; ++i) am[i] = valid[i] ? ma_mult(md, sl, k[i], dtc[i]) : 1.0;
+        double a = am[0], b = r[0];         // the lane's epochs composed
+        if constexpr (NE == 2) {
+            b = __builtin_fma(am[1], r[0], r[1]);
+            a = am[1] * am[0];
+        }
+        wave_affine_scan(a, b, lane);
+        double e0 = carry;                  // eps before this wave's epochs
+        if (WPT > 1) {
+            if (lane == 63) sc.tot[parity][wave] = make_double2(a, b);
+            __syncthreads();
+            const int w0 = wave - wsub;
+            double2 tot[WPT];
+#pragma unroll
+            for (int w = 0; w < WPT; ++w) tot[w] = sc.tot[parity][w0 + w];
+            double pa = tot[0].x, pb = tot[0].y;    // the maps of waves 0 .. w composed
+#pragma unroll
+            for (int w = 1; w < WPT; ++w) {
+                if (w == wsub) e0 = __builtin_fma(pa, carry, pb);
+                pb = __builtin_fma(tot[w].x, pb, tot[w].y);
+                pa = tot[w].x * pa;
+            }
+            carry = __builtin_fma(pa, carry, pb);
+            parity ^= 1;
+        }
+        eps[NE - 1] = __builtin_fma(a, e0, b);
+        if (WPT == 1) carry = readlane_f64(eps[NE - 1], 63);
+        if constexpr (NE == 2) eps[0] = __builtin_fma(am[0], wave_prev(eps[1], e0), r[0]);
+    }
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+        if (valid[i]) {
+            const double cs = (EXT >= 1 && has_post(md)) ? epoch_post(md, sl, tab, t[i], n0 + i, k[i]) : 0.0;
+            const double res = eps[i] - cs;
+            chi = __builtin_fma(res * res, rcp_path<PREC>(err2[i]), chi);
+            prod *= err2[i];
+            pexp += __builtin_amdgcn_frexp_exp(prod);
+            prod = __builtin_amdgcn_frexp_mant(prod);
+            if (WRITE) {
+                out_model[n0 + i] = mu[i] + (r[i] - eps[i]) + cs;
+                out_err2[n0 + i] = err2[i];
+            }
+            if (WEPS) out_eps[n0 + i] = eps[i];
+        }
+    }
+}
+
+// lnL of the parameter vector in slot sl, by its WPT waves (wave `wsub` of
+// them; `wave` in the workgroup).  With WPT > 1 all threads of the workgroup
+// call this together (it holds barriers); `live` == false then skips the
+// arithmetic.  The slot must be prepared (slot_prepare) and the sin/cos table
+// loaded.  With WRITE the per-epoch model and err2 are stored (device order);
+// with WEPS the per-epoch MA-filtered residual eps (= r without MA; before the
+// terms added after the MA are taken off).  EXT as model_ext.
+//
+// Bound by VALU issue for long series and large batches, by latency for small
+// ones.  Two consecutive epochs per lane: the planet's constants, the path's
+// branches and the MA scan (whose maps compose pairwise first) are paid once
+// for both, and their Kepler chains interleave.  One vector per workgroup (from
+// two waves on) and no tile staging: one barrier per chunk with the MA, none
+// without.  Measured against one epoch per lane with LDS tiles shared by the
+// vectors of a 512-thread workgroup: 8192 vectors of 7 planets x 10^4 epochs,
+// MA(1), mixed, 1.10 -> 1.01 ms; 2560 of 3 x 1530 FP64 45 -> 41 us; 1283 of 4 x
+// 783 with a sinusoid 43 -> 22 us (that instance also lost the MA orders above
+// 1, 84 -> 74 VGPRs); stretch sweeps at 16 x 1024 x 10^4, FP64, 3.6 -> 2.5 ms.
+template <int PREC, int WPT, bool WRITE, bool WEPS = false, int EXT = 2, class SL>
+__device__ double vec_lnl(const ModelDev& md, const SL& sl, const SinCosTab& tab, ScanLDS& sc, bool live, int wsub,
+                          double* out_model = nullptr, double* out_err2 = nullptr, double* out_eps = nullptr) {
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int G = 64 * WPT;
-    const int g = wsub * 64 + lane;
+    const int wave = wave_uniform(threadIdx.x >> 6);
+    constexpr int G = 64 * WPT;
     const int kmask = wave_uniform(sl.ktab_mask);
     double chi = 0.0, prod = 1.0;
     int pexp = 0;
     double carry = 0.0;
     double qcarry[4] = {0.0, 0.0, 0.0, 0.0};   // MA(q >= 2) state carried between chunks
     int parity = 0;
-    const bool staged = resident && md.N <= TILE;
-    // With the moving average over several waves, every chunk ends with the
-    // carry's barrier, after the chunk's last read of the tile.
-    const bool ma_sync = md.ma_active && WPT > 1;
-    EpochRegs nx{};
-    if (PF && !staged) {
-        if (first) nx = *first;
-        else epoch_prefetch(md, 0, nx);
-    }
-    for (int tb = 0; tb < md.N; tb += TILE) {
-        const int tn = min(TILE, md.N - tb);
-        if (!staged) {
-            if (tb == 0 || !ma_sync) __syncthreads();     // the tile's previous readers are done
-            if (PF) {
-                epoch_store(md, tl, tb, nx);
-                __syncthreads();
-                if (tb + TILE < md.N) epoch_prefetch(md, tb + TILE, nx);
-            } else {
-                tile_load(md, tl, tb, tn);
-                __syncthreads();
-            }
-        }
-        for (int cb = 0; cb < tn; cb += G) {
-            const int j = cb + g;
-            const bool valid = live && (j < tn);
-            // Everything this chunk needs from the tile is read before the MA
-            // scan: with the MA over several waves the scan's barrier is the
-            // last one before the next tile overwrites this one.
-            double r = 0.0, err2 = 1.0, mu = 0.0, tj = 0.0;
-            int k = 0;
-            if (valid) {
-                k = tl.ins[j];
-                tj = tl.t[j];
-                mu = epoch_mu<PREC>(md, sl, tl.tab, tj, k, kmask);
-                err2 = tl.s2[j] + sl.jit2[k];
-                r = tl.y[j] - mu;
-            }
-            double eps = r;
-            if (POST && md.ma_active && md.ma_q > 1) {
-                eps = md.ma_q == 2
-                          ? ma_chunk_q<2, WPT>(md, sl, tl, valid, j, tb, tj, k, r, lane, wave, wsub, parity, qcarry)
-                          : ma_chunk_q<4, WPT>(md, sl, tl, valid, j, tb, tj, k, r, lane, wave, wsub, parity, qcarry);
-            } else if (md.ma_active) {
-                double a = 1.0, b = 0.0;
-                if (valid) {
-                    const double dtj = tl.dt[j];
-                    if (md.ma_wfixed) a = -(sl.ma_c[k] * dtj);
-                    else a = dtj < 0.0 ? 0.0 : -(sl.ma_c[k] * exp(-dtj / sl.ma_tau[k]));
-                    b = r;
-                }
-                wave_affine_scan(a, b, lane);
-                if (WPT == 1) {
-                    eps = __builtin_fma(a, carry, b);
-                    carry = readlane_f64(eps, 63);
-                } else {
-                    if (lane == 63) { sc.tot[parity][wave][0] = a; sc.tot[parity][wave][1] = b; }
-                    __syncthreads();
-                    const int w0 = wave - wsub;
-                    // (pa, pb): the maps of waves 0 .. w of the vector composed
-                    if (wsub == 0) eps = __builtin_fma(a, carry, b);
-                    double pa = sc.tot[parity][w0][0], pb = sc.tot[parity][w0][1];
-                    for (int w = 1; w < WPT; ++w) {
-                        if (w == wsub) {
-                            eps = __builtin_fma(a, __builtin_fma(pa, carry, pb), b);
-                        }
-                        const double ta = sc.tot[parity][w0 + w][0], tbv = sc.tot[parity][w0 + w][1];
-                        pb = __builtin_fma(ta, pb, tbv);
-                        pa = ta * pa;
-                    }
-                    carry = __builtin_fma(pa, carry, pb);
-                    parity ^= 1;
-                }
-            }
-            if (valid) {
-                const double cs = (POST && has_post(md)) ? epoch_post(md, sl, tl.tab, tj, tb + j, k) : 0.0;
-                const double res = eps - cs;
-                chi = __builtin_fma(res * res, PREC == 1 ? rcp64_1(err2) : rcp64(err2), chi);
-                prod *= err2;
-                pexp += __builtin_amdgcn_frexp_exp(prod);
-                prod = __builtin_amdgcn_frexp_mant(prod);
-                if (WRITE) {
-                    out_model[tb + j] = mu + (r - eps) + cs;
-                    out_err2[tb + j] = err2;
-                }
-                if (WEPS) out_eps[tb + j] = eps;
-            }
-        }
-    }
+    int cb = 0;
+    for (; cb + G < md.N; cb += 2 * G)
+        lnl_chunk<PREC, WPT, WRITE, WEPS, EXT, 2>(md, sl, tab, sc, live, cb, lane, wave, wsub, kmask, chi, prod, pexp,
+                                                   carry, qcarry, parity, out_model, out_err2, out_eps);
+    if (cb < md.N)
+        lnl_chunk<PREC, WPT, WRITE, WEPS, EXT, 1>(md, sl, tab, sc, live, cb, lane, wave, wsub, kmask, chi, prod, pexp,
+                                                   carry, qcarry, parity, out_model, out_err2, out_eps);
     double ld = live ? log(prod) + (double)pexp * LN2 : 0.0;
     chi = wave_sum(chi);
     ld = wave_sum(ld);
     if (WPT > 1) {
-        __syncthreads();
         if (lane == 0) { sc.red[wave][0] = chi; sc.red[wave][1] = ld; }
         __syncthreads();
         chi = 0.0; ld = 0.0;

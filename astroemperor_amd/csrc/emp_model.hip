@@ -77,24 +77,25 @@ extern "C" int emp_device_info(int32_t* n_cu, int32_t* clock_khz, char* arch_nam
 // ---------------------------------------------------------------------------
 // Kernels.
 // ---------------------------------------------------------------------------
-template <int PREC, int WPT, bool POST>
-__global__ __launch_bounds__(BLOCK) void k_lnl(ModelDev md, const double* __restrict__ theta, int64_t B,
-                                               int64_t ld, double* __restrict__ out,
-                                               unsigned long long* nonfinite) {
-    constexpr int SLOTS = NWAVES / WPT;
+template <int PREC, int WPT, int EXT>
+__global__ __launch_bounds__(64 * WPT * vecs_per_wg(WPT)) void k_lnl(ModelDev md, const double* __restrict__ theta,
+                                                                    int64_t B, int64_t ld, double* __restrict__ out,
+                                                                    unsigned long long* nonfinite) {
+    constexpr int SLOTS = vecs_per_wg(WPT);
     __shared__ SlotLDS<SLOTS> s_slot[SLOTS];
-    __shared__ TileLDS s_tile;
+    __shared__ SinCosTab s_tab;
     __shared__ ScanLDS s_scan;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int slot = wave / WPT, wsub = wave % WPT;
     const int64_t b = (int64_t)blockIdx.x * SLOTS + slot;
     const bool live = b < B;
     SlotLDS<SLOTS>& sl = s_slot[slot];
     if (live) expand_theta(md, sl, theta + b * ld, wsub * 64 + lane, 64 * WPT);
-    tab_load(md, s_tile);
+    tab_load(md, s_tab);
     __syncthreads();
-    slot_prepare<PREC, WPT>(md, sl, s_tile, live, wsub, lane);
-    double v = block_lnl<PREC, WPT, false, false, true, POST>(md, sl, s_tile, s_scan, live, wsub, nullptr, nullptr);
+    if (WPT == 1 && !live) return;      // a whole wave; no workgroup barrier follows
+    slot_prepare<WPT>(md, sl, live, wsub, lane);
+    double v = vec_lnl<PREC, WPT, false, false, EXT>(md, sl, s_tab, s_scan, live, wsub);
     if (live && wsub == 0 && lane == 0) {
         if (!(v == v) || v == __builtin_inf()) {
             v = -__builtin_inf();
@@ -119,55 +120,59 @@ __global__ void k_prior(ModelDev md, const double* __restrict__ theta, int64_t B
 
 __global__ __launch_bounds__(BLOCK) void k_model_eval(ModelDev md, const double* __restrict__ theta,
                                                       double* out_model, double* out_err2) {
-    __shared__ SlotLDS<1> s_slot[1];
-    __shared__ TileLDS s_tile;
+    __shared__ SlotLDS<1> sl;
+    __shared__ SinCosTab s_tab;
     __shared__ ScanLDS s_scan;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    SlotLDS<1>& sl = s_slot[0];
+    const int lane = threadIdx.x & 63, wave = wave_uniform(threadIdx.x >> 6);
     expand_theta(md, sl, theta, threadIdx.x, BLOCK);
-    tab_load(md, s_tile);
+    tab_load(md, s_tab);
     __syncthreads();
-    slot_prepare<0, NWAVES>(md, sl, s_tile, true, wave, lane);
-    block_lnl<0, NWAVES, true>(md, sl, s_tile, s_scan, true, wave, out_model, out_err2);
+    slot_prepare<NWAVES>(md, sl, true, wave, lane);
+    vec_lnl<0, NWAVES, true>(md, sl, s_tab, s_scan, true, wave, out_model, out_err2);
 }
 
 // ---------------------------------------------------------------------------
 // Launchers.
 // ---------------------------------------------------------------------------
-// Models without the extended features (terms added after the MA, MA orders
-// above 1) run the variant that compiles them out (fewer registers).
+// Each model runs the instance with only the features it uses (model_ext).
 template <int PREC, int WPT>
 static void launch_lnl_t(const ModelDev& md, const double* th, int64_t B, int64_t ld, double* out,
                          unsigned long long* nf, hipStream_t s) {
-    constexpr int SLOTS = NWAVES / WPT;
+    constexpr int SLOTS = vecs_per_wg(WPT), NT = 64 * WPT * SLOTS;
     const int64_t grid = (B + SLOTS - 1) / SLOTS;
-    if (needs_ext(md))
-        hipLaunchKernelGGL((k_lnl<PREC, WPT, true>), dim3((unsigned)grid), dim3(BLOCK), 0, s, md, th, B, ld, out, nf);
-    else
-        hipLaunchKernelGGL((k_lnl<PREC, WPT, false>), dim3((unsigned)grid), dim3(BLOCK), 0, s, md, th, B, ld, out,
-                           nf);
+    switch (model_ext(md)) {
+        case 0: hipLaunchKernelGGL((k_lnl<PREC, WPT, 0>), dim3((unsigned)grid), dim3(NT), 0, s, md, th, B, ld, out, nf); break;
+        case 1: hipLaunchKernelGGL((k_lnl<PREC, WPT, 1>), dim3((unsigned)grid), dim3(NT), 0, s, md, th, B, ld, out, nf); break;
+        default: hipLaunchKernelGGL((k_lnl<PREC, WPT, 2>), dim3((unsigned)grid), dim3(NT), 0, s, md, th, B, ld, out, nf);
+    }
 }
 
-int emp_pick_wpt(const EmpModel* m, int64_t B, int precision, bool halfstep) {
+int emp_pick_wpt(const EmpModel* m, int64_t B, bool halfstep) {
     if (m->wpt_override) return m->wpt_override;
-    // Enough waves to give every SIMD (4 per CU) about 32 on the mixed path
-    // (from 4 waves per vector its Kepler tables are kept per interval) and
-    // 16 on the FP64 path, at least two waves per vector for series of 1024
-    // epochs or more, but never more lanes per vector than a third of the
-    // epochs for batched likelihoods, half for the PT half-step (whose few
-    // proposals make one walker's critical path the launch's length).
+    // Enough waves to give every SIMD (4 per CU) about 32, at least two waves
+    // per vector for series of 1024 epochs or more.  Batched likelihoods: never
+    // more lanes per vector than a third of the epochs.  The PT half-step, whose
+    // few proposals make one walker's critical path the launch's length: at
+    // least four epochs per lane, but one is enough while the launch has fewer
+    // than 4 waves per SIMD.
     // Measured batched lnL at 1 / 2 / 4 / 8 waves per vector, mixed and FP64:
-    // 7 planets x 10^4 epochs at 8192 vectors 1.48 / 1.31 / 1.28 / 1.37 ms
-    // and 3.07 / 3.01 / 3.06 / 3.15 ms; 5 planets x 2000 epochs at 65,536
-    // vectors 1.40 / 1.26 / 1.34 / 1.53 ms and 3.42 / 3.40 / 3.48 / 3.66 ms;
-    // 3 planets x 1530 epochs at 2560 vectors 72 / 56 / 52 / 59 us and
-    // 121 / 92 / 81 / 90 us.  The rule picks 4, 2, 2, 2, 4 and 4.
-    const int per_simd = precision == EMP_MIXED ? 32 : 16;
-    const int64_t target_waves = (int64_t)m->n_cu * 4 * per_simd;
-    const int wmin = m->dev.N >= 1024 ? 2 : 1;
-    const int max_lanes = halfstep ? m->dev.N / 2 : m->dev.N / 3;
+    // 7 planets x 10^4 epochs at 8192 vectors 1.10 / 1.10 / 1.01 / 1.04 ms and
+    // 1.31 / 1.34 / 1.24 / 1.26 ms; 3 planets x 1530 epochs at 2560 vectors 47 /
+    // 43 / 34 / 43 us and 53 / 49 / 41 / 48 us; 4 planets x 783 epochs with a
+    // sinusoid at 1283 vectors, mixed, 33 / 26 / 22 / 26 us (the rule: 4 in all);
+    // 5 planets x 2000 epochs at 65,536 vectors, mixed, 1.17 / 1.18 / 1.17 / 1.30
+    // ms (the rule: 2).  Stretch sweeps: 10 x 256 walkers at 1530 epochs, mixed,
+    // 111 / 87 / 77 / 78 us (the rule: 4), 6 x 60 at 3000 epochs, FP64, 179 / 111 /
+    // 75 / 64 us (8), 8 x 200 at 400 epochs 56 / 52 / 49 / 49 us (4), 16 x 1024 at
+    // 10^4 epochs 2.38 / 2.21 / 2.07 / 2.17 ms (4).
+    const int64_t simds = (int64_t)m->n_cu * 4;
+    const int N = m->dev.N, wmin = N >= 1024 ? 2 : 1;
     int wpt = 1;
-    while (wpt < 8 && (B * wpt < target_waves || wpt < wmin) && 64 * (wpt * 2) <= max_lanes) wpt *= 2;
+    while (wpt < 8 && (B * wpt < 32 * simds || wpt < wmin)) {
+        const int lanes = 64 * wpt * 2;
+        if (halfstep ? (lanes > N || (4 * lanes > N && B * wpt >= 4 * simds)) : 3 * lanes > N) break;
+        wpt *= 2;
+    }
     return wpt;
 }
 
@@ -175,7 +180,7 @@ int emp_launch_lnl(const EmpModel* m, const double* d_theta, int64_t B, int64_t 
                    int precision, int wpt, hipStream_t s) {
     if (B <= 0) return EMP_OK;
     const ModelDev& md = m->dev;
-    if (wpt <= 0) wpt = emp_pick_wpt(m, B, precision);
+    if (wpt <= 0) wpt = emp_pick_wpt(m, B);
 #define EMP_CASE(P, W)                                                                 \
     if (precision == P && wpt == W) {                                                  \
         launch_lnl_t<P, W>(md, d_theta, B, ld, d_lnl, m->d_nonfinite, s);              \
@@ -463,7 +468,7 @@ extern "C" int emp_model_create(const EmpModelDesc* d, EmpModel** out) {
         EMP_UP(tab, md.sctab);
     }
 #undef EMP_UP
-    if (!emp_model_dev_complete(md) || !md.pseq_e) {
+    if (!emp_model_dev_complete(md)) {
         emp_model_destroy(m);
         emp_set_error("a device array of the model is missing");
         return EMP_EINVAL;
@@ -596,7 +601,8 @@ extern "C" int emp_model_set_waves_per_theta(EmpModel* m, int32_t w) {
 
 extern "C" int emp_model_get_waves_per_theta(EmpModel* m, int32_t precision, int32_t* out) {
     if (!m || !out) { emp_set_error("null argument"); return EMP_EINVAL; }
-    *out = emp_pick_wpt(m, 1024, precision);
+    (void)precision;      // the rule is the same for both paths
+    *out = emp_pick_wpt(m, 1024);
     return EMP_OK;
 }
 

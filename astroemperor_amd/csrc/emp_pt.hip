@@ -181,20 +181,20 @@ __global__ __launch_bounds__(PRIOR_BLOCK) void k_pt_prior(ModelDev md, PTDev pd,
 
 // ---------------------------------------------------------------------------
 // Half-step, part 2: likelihood and acceptance of the proposals inside the
-// prior support, one slot of the workgroup per task; a workgroup whose tasks
-// all lie outside leaves at once.
+// prior support, one vector of the workgroup per task; a workgroup whose task
+// lies outside leaves at once.
 // ---------------------------------------------------------------------------
-template <int PREC, int WPT, bool POST>
-__global__ __launch_bounds__(BLOCK) void k_pt_half(ModelDev md, PTDev pd, int half, int step) {
-    constexpr int SLOTS = NWAVES / WPT;
+template <int PREC, int WPT, int EXT>
+__global__ __launch_bounds__(64 * WPT * vecs_per_wg(WPT)) void k_pt_half(ModelDev md, PTDev pd, int half, int step) {
+    constexpr int SLOTS = vecs_per_wg(WPT);
     __shared__ SlotLDS<SLOTS> s_slot[SLOTS];
-    __shared__ TileLDS s_tile;
+    __shared__ SinCosTab s_tab;
     __shared__ ScanLDS s_scan;
     __shared__ int s_acc[SLOTS];
     __shared__ TaskOps s_ops[SLOTS];
     (void)half;
     (void)step;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int slot = wave / WPT, wsub = wave % WPT;
     const int g = wsub * 64 + lane, G = 64 * WPT;
     const int b = blockIdx.x * SLOTS + slot;
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(BLOCK) void k_pt_half(ModelDev md, PTDev pd, int ha
     }
     const PTView pv = view_of(pd);
     SlotLDS<SLOTS>& sl = s_slot[slot];
-    tab_load(md, s_tile);      // published by pt_eval_accept's first barrier
+    tab_load(md, s_tab);
     if (live) {
         if (wsub == 0 && lane == 0) s_ops[slot] = pd.rec[b];
         const double* row = pd.prow + (size_t)b * pd.D;
@@ -215,10 +215,22 @@ __global__ __launch_bounds__(BLOCK) void k_pt_half(ModelDev md, PTDev pd, int ha
             sl.theta[j] = fi >= 0 ? row[fi] : md.fixed_val[j];
         }
     }
-    pt_eval_accept<PREC, WPT, true, POST>(md, pv, s_ops, live, sl, s_tile, s_scan, s_acc, slot, wsub, false,
-                              (unsigned long long*)(pd.sweep + 1));
-    // an accepted stretch move leaves the slot's gradient out of date
-    if (pd.lg_stale && live && wsub == 0 && lane == 0 && s_acc[slot]) pd.lg_stale[s_ops[slot].sk] = 1;
+    __syncthreads();
+    if (!live) return;                       // (one wave per vector: whole waves, no workgroup barrier follows)
+    const TaskOps& ops = s_ops[slot];        // read at the acceptance: not held in registers through the likelihood
+    slot_prepare<WPT>(md, sl, true, wsub, lane);
+    const double ll = vec_lnl<PREC, WPT, false, false, EXT>(md, sl, s_tab, s_scan, true, wsub);
+    if (wsub == 0 && lane == 0) {
+        atomicAdd((unsigned long long*)(pd.sweep + 1), 1ull);
+        s_acc[slot] = pt_decide(pv, ops, ll);
+        // an accepted stretch move leaves the slot's gradient out of date
+        if (pd.lg_stale && s_acc[slot]) pd.lg_stale[ops.sk] = 1;
+    }
+    vec_sync<WPT>();
+    if (s_acc[slot]) {
+        double* Xk = pd.X + (size_t)ops.sk * pd.D;
+        for (int d = g; d < md.D; d += G) Xk[d] = sl.theta[md.free_idx[d]];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -885,29 +897,29 @@ __global__ __launch_bounds__(PRIOR_BLOCK) void k_lg_accept(PTDev pd, int half, i
 // Host side.
 // ---------------------------------------------------------------------------
 // With events, the launch itself records them (start and end of the
-// kernel's execution, as a kernel trace measures it).  Models without the
-// extended features (activity or cosine terms, MA orders above 1) run the
-// variant that compiles them out (it keeps the one-slot variants within the
-// scalar-register budget of 8 waves per SIMD).
-template <int PREC, int WPT, bool POST>
+// kernel's execution, as a kernel trace measures it).  Each model runs the
+// instance with only the features it uses (model_ext).
+template <int PREC, int WPT, int EXT>
 static void launch_half_c(const ModelDev& md, const PTDev& pd, int half, int step, hipStream_t s, hipEvent_t e0,
                           hipEvent_t e1) {
-    constexpr int SLOTS = NWAVES / WPT;
+    constexpr int SLOTS = vecs_per_wg(WPT), NT = 64 * WPT * SLOTS;
     const int64_t tasks = (int64_t)pd.T * pd.W2;
     const int64_t grid = (tasks + SLOTS - 1) / SLOTS;
     if (e0)
-        hipExtLaunchKernelGGL((k_pt_half<PREC, WPT, POST>), dim3((unsigned)grid), dim3(BLOCK), 0, s, e0, e1, 0, md,
-                              pd, half, step);
+        hipExtLaunchKernelGGL((k_pt_half<PREC, WPT, EXT>), dim3((unsigned)grid), dim3(NT), 0, s, e0, e1, 0, md, pd,
+                              half, step);
     else
-        hipLaunchKernelGGL((k_pt_half<PREC, WPT, POST>), dim3((unsigned)grid), dim3(BLOCK), 0, s, md, pd, half,
-                           step);
+        hipLaunchKernelGGL((k_pt_half<PREC, WPT, EXT>), dim3((unsigned)grid), dim3(NT), 0, s, md, pd, half, step);
 }
 
 template <int PREC, int WPT>
 static void launch_half_t(const ModelDev& md, const PTDev& pd, int half, int step, hipStream_t s,
                           hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
-    if (needs_ext(md)) launch_half_c<PREC, WPT, true>(md, pd, half, step, s, e0, e1);
-    else launch_half_c<PREC, WPT, false>(md, pd, half, step, s, e0, e1);
+    switch (model_ext(md)) {
+        case 0: launch_half_c<PREC, WPT, 0>(md, pd, half, step, s, e0, e1); break;
+        case 1: launch_half_c<PREC, WPT, 1>(md, pd, half, step, s, e0, e1); break;
+        default: launch_half_c<PREC, WPT, 2>(md, pd, half, step, s, e0, e1);
+    }
 }
 
 // draw_swaps: this prior pass also draws the sweep's swap randoms (the last
@@ -1159,7 +1171,7 @@ extern "C" int emp_pt_create(EmpModel* m, const EmpPTDesc* desc, const double* b
     EMP_TRY(hipMemset(v.rec_owed, 0, sizeof(int)));
     EMP_TRY(hipDeviceSynchronize());     // the engine stream does not wait for the null stream
 #undef EMP_TRY
-    p->wpt = emp_pick_wpt(m, (int64_t)v.T * v.W2, d.precision, true);
+    p->wpt = emp_pick_wpt(m, (int64_t)v.T * v.W2, true);
     rc = eval_state(p);
     if (rc) { emp_pt_destroy(p); return rc; }
     *out = p;

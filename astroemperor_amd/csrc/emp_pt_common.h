@@ -113,32 +113,6 @@ __device__ inline double prior_proposal_wave(const ModelDev& md, const double* X
     return lp;
 }
 
-// Indices b < n with lp[b] > -inf, in increasing order, into list[]; every
-// thread of the workgroup (nthr threads, whole waves) gets the count.
-// s_wcnt: LDS scratch of one int per wave.
-__device__ inline int compact_live(const double* lp, int n, int* list, int* s_wcnt, int nthr) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = nthr >> 6;
-    int base = 0;
-    for (int c0 = 0; c0 < n; c0 += nthr) {
-        const int b = c0 + (int)threadIdx.x;
-        const bool f = b < n && lp[b] > -__builtin_inf();
-        const unsigned long long m = __ballot(f);
-        const int within = __popcll(m & ((1ull << lane) - 1ull));
-        if (lane == 0) s_wcnt[wave] = __popcll(m);
-        __syncthreads();
-        int off = base, tot = 0;
-        for (int w = 0; w < nw; ++w) {
-            const int c = s_wcnt[w];
-            if (w < wave) off += c;
-            tot += c;
-        }
-        if (f) list[off + within] = b;
-        __syncthreads();
-        base += tot;
-    }
-    return base;
-}
-
 // Acceptance operands of one stretch proposal that are fixed before its
 // likelihood is known: the Metropolis log ratio is
 //   ((D - 1) ln z + (beta lnL' - beta lnL)) + (ln pi' - ln pi),
@@ -166,77 +140,18 @@ __device__ __forceinline__ TaskOps pt_task_ops(const PTView& pv, const Proposal&
     return o;
 }
 
-// Likelihood and Metropolis acceptance of one slot's task whose proposal is
-// already in sl.theta (free and fixed parameters) and whose operands are in
-// s_ops[slot] (LDS, read only at the acceptance so that they do not occupy
-// registers through the likelihood): per-slot constants, the mixed path's
-// Kepler tables, lnL, acceptance, and the accepted position written back.
-// Every evaluated likelihood adds one to *n_lnl.  The sin/cos table must be
-// in `tile`; with `resident` all epochs are too.  All threads of the
-// workgroup call this together (it contains barriers).  POST = false
-// compiles the terms added after the MA out (models without them).
-template <int PREC, int WPT, bool PF = true, bool POST = true, class SL>
-__device__ void pt_eval_accept(const ModelDev& md, const PTView& pv, const TaskOps* s_ops, bool live, SL& sl,
-                               TileLDS& tile, ScanLDS& scan, int* s_acc, int slot, int wsub, bool resident,
-                               unsigned long long* n_lnl) {
-    const int lane = threadIdx.x & 63;
-    const int g = wsub * 64 + lane, G = 64 * WPT;
-    EpochRegs e0{};
-    const bool staged = resident && md.N <= TILE;
-    if (PF && !staged) epoch_prefetch(md, 0, e0);      // the first tile's loads overlap the set-up
-    __syncthreads();
-    if (live && wsub == 0) slot_setup(md, sl, lane);
-    __syncthreads();
-    if (live) {       // per-vector Kepler tables, one planet per wave
-        for (int p = wsub; p < md.K; p += WPT)
-            if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
-    }
-    __syncthreads();
-    double ll = block_lnl<PREC, WPT, false, false, PF, POST>(md, sl, tile, scan, live, wsub, nullptr, nullptr,
-                                                            resident, nullptr, (PF && !staged) ? &e0 : nullptr);
-    if (live && wsub == 0 && lane == 0) {
-        const TaskOps& ops = s_ops[slot];
-        int acc = 0;
-        atomicAdd(n_lnl, 1ull);
-        if (!(ll == ll) || ll == __builtin_inf()) ll = -__builtin_inf();
-        const double tn = ops.beta == 0.0 ? 0.0 : ops.beta * ll;
-        const double lnalpha = (ops.lz + (tn - ops.to)) + ops.dp;
-        if (ops.logu < lnalpha) {
-            pv.lnl[ops.sk] = ll;
-            pv.lnp[ops.sk] = ops.lp;
-            pv.accepted[ops.t * pv.W + ops.k] += 1;
-            acc = 1;
-        }
-        s_acc[slot] = acc;
-    }
-    __syncthreads();
-    if (live && s_acc[slot]) {
-        double* Xk = pv.X + (size_t)s_ops[slot].sk * pv.D;
-        for (int d = g; d < md.D; d += G) Xk[d] = sl.theta[md.free_idx[d]];
-    }
-}
-
-// One slot's task of a fused stretch half-step, for a task whose proposal
-// prior lp is already known (b < 0: no task for this slot in this pass):
-// proposal into LDS, then pt_eval_accept (without the tile prefetch: the
-// batched-systems kernel that calls this is register-bound).
-template <int PREC, int WPT, bool EXT = true, class SL>
-__device__ void pt_half_task(const ModelDev& md, const PTView& pv, long long sweep, int half, int step, int b,
-                             double lp, SL& sl, TileLDS& tile, ScanLDS& scan, int* s_acc, TaskOps* s_ops,
-                             int slot, int wsub, bool resident, unsigned long long* n_lnl) {
-    const int lane = threadIdx.x & 63;
-    const int g = wsub * 64 + lane, G = 64 * WPT;
-    const bool live = b >= 0 && lp > -__builtin_inf();
-    if (live) {
-        const Proposal pr = pt_propose(pv, sweep, half, step, b);
-        const double* Xk = pv.X + (size_t)pr.sk * pv.D;
-        const double* Xj = pv.X + (size_t)pr.sj * pv.D;
-        for (int d = g; d < md.D; d += G) sl.theta[md.free_idx[d]] = pt_prop_value(Xk, Xj, pr.z, d);
-        for (int q = g; q < md.Dfull; q += G)
-            if (md.inv_free[q] < 0) sl.theta[q] = md.fixed_val[q];
-        if (wsub == 0 && lane == 0) s_ops[slot] = pt_task_ops(pv, pr, lp, md.D);
-    }
-    pt_eval_accept<PREC, WPT, false, EXT>(md, pv, s_ops, live, sl, tile, scan, s_acc, slot, wsub, resident, n_lnl);
+// Metropolis acceptance of one task whose likelihood ll is known: decided by one
+// lane, which writes the slot's likelihood and prior and the count.  Returns
+// whether the proposal is accepted.
+__device__ __forceinline__ int pt_decide(const PTView& pv, const TaskOps& ops, double ll) {
+    if (!(ll == ll) || ll == __builtin_inf()) ll = -__builtin_inf();
+    const double tn = ops.beta == 0.0 ? 0.0 : ops.beta * ll;
+    const double lnalpha = (ops.lz + (tn - ops.to)) + ops.dp;
+    if (!(ops.logu < lnalpha)) return 0;
+    pv.lnl[ops.sk] = ll;
+    pv.lnp[ops.sk] = ops.lp;
+    pv.accepted[ops.t * pv.W + ops.k] += 1;
+    return 1;
 }
 
 __device__ __forceinline__ uint32_t swap_partner(const PTView& pv, long long sweep, int h, int i) {

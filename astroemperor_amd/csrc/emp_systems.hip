@@ -1,16 +1,18 @@
 // Batched independent systems: S separate RV models, each with its own
-// parallel-tempering ensemble, advanced together by ONE persistent kernel
-// launch per sweep (replayed from a hipGraph).
+// parallel-tempering ensemble, advanced together, a few kernel launches per
+// sweep of all of them (replayed from a hipGraph).
 //
-// Scheduling.  A sweep of one system (nsteps x two stretch halves over its
-// T x W walkers, the swap round, the ladder update, the statistics and the
-// optional record) is one work item, done start to finish by one workgroup:
-// the system's epochs stay resident in LDS (N <= TILE) for all its
-// likelihoods, and no workgroup ever waits for another.  Workgroups pop
-// items from a queue ordered longest first (cost ~ N (k c_kep + c_ep) T W),
-// so the ragged tail of small systems fills in behind the big ones.  The
-// last workgroup to leave resets the queue and advances the sweep counter,
-// so the captured launch replays unchanged.
+// A half-step is two passes.  The prior pass, one workgroup per system, draws
+// the proposals, evaluates their priors and lists those inside the support.
+// The likelihood pass gives every workgroup up to `chunk` listed walkers of one
+// system: their vectors, planet constants and acceptance operands are set up
+// for all of them at once (one lane per walker and planet, instead of one wave
+// per walker with a few lanes busy), then each wave takes walkers on its own.
+// Workgroups run longest system first, so the ragged tail of small systems
+// fills in behind the big ones, and the longest system's walkers spread over
+// the chip.  The swap pass, one workgroup per system, ends the sweep; its last
+// workgroup advances the sweep counter, so the captured launches replay
+// unchanged and no workgroup ever waits for another.
 //
 // Randomness: the counters of the single-system engine with the system index
 // mixed in (system 0 draws exactly what the single-system engine draws).
@@ -24,7 +26,9 @@
 
 using namespace emp;
 
-constexpr int SYS_MAX_TASKS = 512;   // T W / 2 per system (per-task prior and list in LDS)
+constexpr int SYS_MAX_TASKS = 512;   // T W / 2 per system
+constexpr int SYS_PASS = 256;        // threads of the prior and swap passes
+constexpr int SYS_SCRATCH = 24 * 1024;   // working copies of the swap pass: 12 (2 T - 1) W bytes, T W <= 1024
 
 struct SysDev {
     int S, T, W, nsteps;
@@ -43,7 +47,10 @@ struct SysDev {
     long long* accepted;       // [S][T W] by position
     double* tsw_sum;           // [S][T-1] summed over sweeps
     double* smd_sum;           // [S][T-1]
-    unsigned long long* ctl;   // queue head, workgroups finished, sweeps done, likelihoods evaluated
+    unsigned long long* ctl;   // (unused), swap workgroups finished, sweeps done, likelihoods evaluated
+    double* tlp;               // [S][T W/2] ln prior of each task's proposal
+    int* list;                 // [S][T W/2] tasks inside the prior support
+    int* nlive;                // [2][S] how many, per half
     int rec_every, rec_temps;
     int64_t max_rec;
     const int64_t* rxoff;      // [S] first element of system s in one record of h_x
@@ -70,205 +77,272 @@ __device__ __forceinline__ PTView sys_view(const SysDev& sd, int s, int D) {
                    sd.accepted + s * TW);
 }
 
-// Prior of every proposal of one half-step of one system into lp[ntask], in
-// three workgroup-wide steps over `scratch` (bytes of LDS not otherwise in
-// use): the proposals (one thread per task), every (task, term) pair of the
-// prior's summation sequence md.pseq (all loads in flight together), then
-// the sum of each task's terms in sequence order with prior_seq's -inf
-// return (one thread per task), bit-identical to prior_seq.  Ends with a
-// barrier.
-__device__ inline void sys_priors(const ModelDev& md, const PTView& pv, long long sweep, int half, int step,
-                                  int ntask, char* scratch, size_t bytes, double* lp, int nthr) {
+// The prior pass: workgroup (s, c) takes the c-th SYS_PRIOR_TASKS tasks of
+// system s: the proposals (one thread per task), every (task, term) pair of the
+// prior's summation sequence (the system's resolved sequence in LDS, all loads
+// of the walkers' rows in flight together), then the sum of each task's terms in
+// sequence order with prior_seq's -inf return (one thread per task),
+// bit-identical to prior_seq.  The tasks inside the support are appended to the
+// system's list (in any order: the tasks of a half-step are independent); the
+// other half's count is cleared for its next pass.  The term values take
+// `terms` doubles of LDS, a few tasks at a time where a long sequence needs it.
+// Latency-bound; measured against one workgroup per system with the sequence
+// read from global memory for every term: 110 -> 24 us for 512 systems of 8 x 64
+// walkers.
+constexpr int SYS_PRIOR_TASKS = 64;
+__host__ __device__ inline size_t sys_prior_terms(int L) {
+    const size_t want = (size_t)SYS_PRIOR_TASKS * L, cap = 4096;
+    return want < cap ? want : (cap > (size_t)L ? cap : (size_t)L);
+}
+__global__ __launch_bounds__(SYS_PASS) void k_sys_prior(SysDev sd, int half, int step, int nchunk, int terms_cap) {
 #pragma clang fp contract(off)
-    double* z = (double*)scratch;                      // [ntask]
-    int* sk = (int*)(z + ntask);                       // [ntask]
-    int* sj = sk + ntask;                              // [ntask]
-    double* terms = (double*)(sj + ntask);             // 8-byte aligned: z, sk, sj take 16 ntask bytes
-    const int L = md.npseq;
-    const int chunk = (int)min((size_t)ntask, (bytes - (size_t)((char*)terms - scratch)) / (sizeof(double) * L));
-    for (int b = threadIdx.x; b < ntask; b += nthr) {
-        const Proposal pr = pt_propose(pv, sweep, half, step, b);
-        z[b] = pr.z;
-        sk[b] = pr.sk;
-        sj[b] = pr.sj;
+    extern __shared__ __align__(16) char s_dyn[];
+    __shared__ double s_z[SYS_PRIOR_TASKS];
+    __shared__ int s_k[SYS_PRIOR_TASKS], s_j[SYS_PRIOR_TASKS];
+    const int tid = threadIdx.x;
+    const int s = blockIdx.x / nchunk, b0 = (blockIdx.x - s * nchunk) * SYS_PRIOR_TASKS;
+    const ModelDev& md = sys_model(sd, s);
+    const PTView pv = sys_view(sd, s, md.D);
+    const int ntask = sd.T * (sd.W / 2), nt = min(SYS_PRIOR_TASKS, ntask - b0), L = md.npseq;
+    double* terms = (double*)s_dyn;
+    PseqEntry* seq = (PseqEntry*)(terms + terms_cap);
+    int* nlive = sd.nlive + (size_t)half * sd.S + s;
+    if (b0 == 0 && tid == 0) sd.nlive[(size_t)(1 - half) * sd.S + s] = 0;
+    for (int i = tid; i < L; i += SYS_PASS) seq[i] = md.pseq_e[i];
+    if (tid < nt) {
+        const Proposal pr = pt_propose(pv, (long long)sd.ctl[2], half, step, b0 + tid);
+        s_z[tid] = pr.z;
+        s_k[tid] = pr.sk;
+        s_j[tid] = pr.sj;
     }
     __syncthreads();
-    for (int c0 = 0; c0 < ntask; c0 += chunk) {
-        const int cn = min(chunk, ntask - c0);
-        for (int e = threadIdx.x; e < cn * L; e += nthr) {
-            const int bl = e / L, i = e - bl * L, b = c0 + bl;
-            const int q = md.pseq[i];
-            if (q == PSEQ_CHECK) continue;
-            const double* Xk = pv.X + (size_t)sk[b] * pv.D;
-            const double* Xj = pv.X + (size_t)sj[b] * pv.D;
-            double v;
-            if (q >= 0) {
-                v = prior_term(md.prior[q], pt_prop_value(Xk, Xj, z[b], md.inv_free[q]));
+    const int per = min(nt, terms_cap / L);
+    for (int c0 = 0; c0 < nt; c0 += per) {
+        const int cn = min(per, nt - c0);
+        for (int e = tid; e < cn * L; e += SYS_PASS) {
+            const int bl = e / L, i = e - bl * L, r = c0 + bl;
+            const PseqEntry& pe = seq[i];
+            if (pe.kind == 2) continue;
+            const double* Xk = pv.X + (size_t)s_k[r] * pv.D;
+            const double* Xj = pv.X + (size_t)s_j[r] * pv.D;
+            double x;
+            if (pe.kind == 0) {
+                x = pt_prop_value(Xk, Xj, s_z[r], pe.fa);
             } else {
-                const int pb = PSEQ_ECC - q;
-                const int o = md.off_kep + 5 * pb + 3;
-                const int f3 = md.inv_free[o], f4 = md.inv_free[o + 1];
-                const double s3 = f3 >= 0 ? pt_prop_value(Xk, Xj, z[b], f3) : md.fixed_val[o];
-                const double s4 = f4 >= 0 ? pt_prop_value(Xk, Xj, z[b], f4) : md.fixed_val[o + 1];
-                const double x = s3 * s3 + s4 * s4;
-                v = prior_term(md.ecc_prior[pb], x);
+                const double s3 = pe.fa >= 0 ? pt_prop_value(Xk, Xj, s_z[r], pe.fa) : pe.va;
+                const double s4 = pe.fb >= 0 ? pt_prop_value(Xk, Xj, s_z[r], pe.fb) : pe.vb;
+                x = s3 * s3 + s4 * s4;
             }
-            terms[e] = v;
+            terms[e] = prior_term(pe.term, x);
         }
         __syncthreads();
-        for (int bl = threadIdx.x; bl < cn; bl += nthr) {
-            const double* tv = terms + (size_t)bl * L;
-            double s = 0.0;
-            for (int i = 0; i < L; ++i) {
-                if (md.pseq[i] == PSEQ_CHECK) {
-                    if (s == -__builtin_inf()) break;
-                } else {
-                    s += tv[i];
+        if (tid < 64) {                      // whole first wave (per <= 64)
+            const bool own = tid < cn;
+            double lp = 0.0;
+            if (own) {
+                const double* tv = terms + (size_t)tid * L;
+                for (int i = 0; i < L; ++i) {
+                    if (seq[i].kind == 2) {
+                        if (lp == -__builtin_inf()) break;
+                    } else {
+                        lp += tv[i];
+                    }
                 }
+                sd.tlp[(size_t)s * ntask + b0 + c0 + tid] = lp;
             }
-            lp[c0 + bl] = s;
+            const bool live = own && lp > -__builtin_inf();
+            const unsigned long long m = __ballot(live);
+            int base = 0;
+            if (tid == 0 && m) base = atomicAdd(nlive, __popcll(m));
+            base = __builtin_amdgcn_readfirstlane(base);
+            if (live) sd.list[(size_t)s * ntask + base + __popcll(m & ((1ull << tid) - 1ull))] = b0 + c0 + tid;
         }
         __syncthreads();
     }
 }
 
-// One sweep of every system.  NW waves per workgroup, WPT waves per walker;
-// EXT: the instance with the extended model features (needs_ext), used when
-// any system of the batch has them.
-template <int PREC, int WPT, int NW, bool EXT>
-__global__ __launch_bounds__(NW * 64) void k_sys_sweep(SysDev sd) {
-    constexpr int NT = NW * 64, SLOTS = NW / WPT;
-    __shared__ SlotLDS<SLOTS> s_slot[SLOTS];
-    __shared__ TileLDS s_tile;
+// A walker's slot in the likelihood pass: its vector and planet constants are
+// rows of the workgroup's, the rest belongs to the wave (or waves) at work on
+// it.
+template <class KTE>
+struct SlotView {
+    const double* theta;
+    const PlanetC* planet;
+    KTE (*ktab)[KT_N];
+    double *gam, *jit2, *ma_c, *ma_tau, *jit, *acc;
+    double (*cosw)[3];
+    int ktab_mask;             // (lane 0's)
+};
+struct SlotRest {
+    double gam[IMAX], jit2[IMAX], ma_c[IMAX], ma_tau[IMAX], jit[IMAX];
+    double acc[AMAX];
+    double cosw[CMAX][3];
+};
+
+constexpr int sys_vecs(int wpt) { return wpt == 1 ? 4 : 1; }       // walkers at work in a workgroup
+constexpr int SYS_CHUNK = 16;                                       // most walkers per workgroup
+template <int WPT>
+using SysKTE = std::conditional_t<WPT == 1, float2, float4>;       // as the single-system engine's tables
+
+// Dynamic LDS of the likelihood pass: `chunk` vectors and planet rows, and the
+// Kepler tables of the walkers at work.
+__host__ __device__ inline size_t sys_lds(int wpt, int chunk, int Dfull, int K) {
+    const size_t kte = wpt == 1 ? sizeof(SysKTE<1>) : sizeof(SysKTE<2>);
+    return (size_t)sys_vecs(wpt) * K * KT_N * kte + (size_t)chunk * (Dfull * sizeof(double) + K * sizeof(PlanetC));
+}
+
+// The likelihood pass: workgroup (it, c) takes the c-th `chunk` listed tasks of
+// the it-th system in queue order; with INIT instead every walker (the state
+// loaded into slot = position order), whose prior and likelihood it stores.
+// WPT waves per walker; EXT: the instance with the extended model features
+// (model_ext), used when any system of the batch has them.
+// Bound by VALU issue.  Measured against one persistent workgroup per compute
+// unit that did a whole system's sweep at a time (16 walkers in step between
+// barriers, each wave setting up its own walker, the sweep as long as the
+// longest system's): per sweep of 64 / 512 / 2048 systems of 8 x 64 walkers, mixed,
+// 824 -> 151, 1152 -> 645, 3820 -> 2279 us; 512 FP64 1853 -> 731 us.
+template <int PREC, int WPT, bool EXT, bool INIT>
+__global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_waves_per_eu(EXT ? 3 : 5))) void k_sys_lik(SysDev sd, int half, int step, int chunk,
+                                                                     int nchunk) {
+    constexpr int VECS = sys_vecs(WPT), NT = 64 * WPT * VECS;
+    using KTE = SysKTE<WPT>;
+    extern __shared__ __align__(16) char s_dyn[];
+    __shared__ SinCosTab s_tab;
     __shared__ ScanLDS s_scan;
-    __shared__ int s_acc[SLOTS];
-    __shared__ TaskOps s_ops[SLOTS];
+    __shared__ SlotRest s_rest[VECS];
+    __shared__ TaskOps s_ops[SYS_CHUNK];
+    __shared__ double s_z[SYS_CHUNK];
+    __shared__ int s_k[SYS_CHUNK], s_j[SYS_CHUNK], s_acc[VECS];
+    const int tid = threadIdx.x, wave = wave_uniform(tid >> 6), lane = tid & 63;
+    const int it = blockIdx.x / nchunk, q0 = (blockIdx.x - it * nchunk) * chunk;
+    const int s = __builtin_amdgcn_readfirstlane(sd.order[it]);
+    const int ntask = INIT ? sd.T * sd.W : sd.T * (sd.W / 2);
+    const int nl = INIT ? ntask : __builtin_amdgcn_readfirstlane(sd.nlive[(size_t)half * sd.S + s]);
+    if (q0 >= nl) return;                    // the whole workgroup
+    const int nt = min(chunk, nl - q0);
+    const ModelDev& md = sys_model(sd, s);
+    const PTView pv = sys_view(sd, s, md.D);
+    const int Df = md.Dfull, K = md.K;
+    KTE (*ktab)[KT_N] = (KTE (*)[KT_N])s_dyn;
+    double* theta = (double*)(s_dyn + (size_t)VECS * K * KT_N * sizeof(KTE));
+    PlanetC* planet = (PlanetC*)(theta + chunk * Df);
+    tab_load(md, s_tab);
+    if (tid < nt) {
+        if (INIT) {
+            s_z[tid] = 0.0;
+            s_k[tid] = s_j[tid] = q0 + tid;
+        } else {
+            const int b = sd.list[(size_t)s * ntask + q0 + tid];
+            const Proposal pr = pt_propose(pv, (long long)sd.ctl[2], half, step, b);
+            s_z[tid] = pr.z;
+            s_k[tid] = pr.sk;
+            s_j[tid] = pr.sj;
+            s_ops[tid] = pt_task_ops(pv, pr, sd.tlp[(size_t)s * ntask + b], md.D);
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < nt * Df; e += NT) {
+        const int r = e / Df, f = md.inv_free[e - r * Df];
+        double v = md.fixed_val[e - r * Df];
+        if (f >= 0) {
+            const double* Xk = pv.X + (size_t)s_k[r] * pv.D;
+            v = INIT ? Xk[f] : pt_prop_value(Xk, pv.X + (size_t)s_j[r] * pv.D, s_z[r], f);
+        }
+        theta[e] = v;
+    }
+    __syncthreads();
+    for (int e = tid; e < nt * K; e += NT) {
+        const int r = e / K;
+        planet[e] = planet_slot(md, theta + r * Df, e - r * K);
+    }
+    __syncthreads();
+    const int slot = wave / WPT, wsub = wave - slot * WPT;
+    SlotRest& rest = s_rest[slot];
+    // one wave per walker: the waves work without waiting for one another
+    // (two: one walker after the other, the workgroup together)
+    for (int r = slot; r < nt; r += VECS) {
+        vec_sync<WPT>();                     // the previous walker is finished with the slot
+        SlotView<KTE> sl{theta + r * Df, planet + r * K, ktab + slot * K, rest.gam, rest.jit2, rest.ma_c,
+                         rest.ma_tau, rest.jit, rest.acc, rest.cosw, 0};
+        // every wave computes the mask (a register); the LDS values are the same
+        slot_rest(md, sl, lane, lane < K ? kt_flags(sl.planet[lane].ktab != 0, sl.planet[lane].e) : 0);
+        for (int p = wsub; p < K; p += WPT)
+            if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
+        vec_sync<WPT>();
+        double ll = vec_lnl<PREC, WPT, false, false, EXT ? 2 : 0>(md, sl, s_tab, s_scan, true, wsub);
+        if (INIT) {
+            if (wsub == 0 && lane == 0) {
+                const int b = q0 + r;
+                const double lp = prior_seq(md, sl.theta);
+                if (!(ll == ll) || ll == __builtin_inf()) ll = -__builtin_inf();
+                pv.map[b] = b;
+                pv.lnp[b] = lp;
+                pv.lnl[b] = lp > -__builtin_inf() ? ll : -__builtin_inf();
+            }
+            continue;
+        }
+        if (wsub == 0 && lane == 0) s_acc[slot] = pt_decide(pv, s_ops[r], ll);
+        vec_sync<WPT>();
+        if (s_acc[slot]) {
+            double* Xk = pv.X + (size_t)s_ops[r].sk * pv.D;
+            for (int d = wsub * 64 + lane; d < md.D; d += 64 * WPT) Xk[d] = sl.theta[md.free_idx[d]];
+        }
+    }
+    if (!INIT && tid == 0) atomicAdd(&sd.ctl[3], (unsigned long long)nt);
+}
+
+// The end of a sweep of one system: swap round, ladder, statistics, record.
+__global__ __launch_bounds__(SYS_PASS) void k_sys_swap(SysDev sd) {
+    __shared__ __align__(16) char s_scr[SYS_SCRATCH];
     __shared__ double s_bet[64], s_ld[64];
     __shared__ double s_red[64][2];
     __shared__ double s_rate[64], s_smd[64], s_sig[64];
-    __shared__ double s_tlp[SYS_MAX_TASKS];    // prior of each task's proposal
-    __shared__ int s_list[SYS_MAX_TASKS];      // tasks with a finite prior, in order
-    __shared__ int s_wcnt[MAX_WAVES];
-    __shared__ long long s_item;
-    __shared__ unsigned long long s_cnt;
-    const int tid = threadIdx.x, wave = tid >> 6;
-    const int slot = wave / WPT, wsub = wave % WPT;
+    const int tid = threadIdx.x, s = blockIdx.x;
     const long long sweep = (long long)sd.ctl[2];
-    const int T = sd.T, W = sd.W, TW = T * W, ntask = T * (W / 2);
-    tab_load(sys_model(sd, 0), s_tile);      // one table serves every system
-    for (;;) {
-        __syncthreads();             // the previous item is finished with LDS
-        if (tid == 0) {
-            s_item = (long long)atomicAdd(&sd.ctl[0], 1ull);
-            s_cnt = 0ull;
-        }
-        __syncthreads();
-        // uniform by construction; say so, so that the model is read with
-        // scalar loads into scalar registers
-        const int it = __builtin_amdgcn_readfirstlane((int)min(s_item, (long long)sd.S));
-        if (it >= sd.S) break;
-        const int s = __builtin_amdgcn_readfirstlane(sd.order[it]);
-        const ModelDev& md = sys_model(sd, s);
-        const PTView pv = sys_view(sd, s, md.D);
-        const bool res = md.N <= TILE;
-        if (res) tile_load(md, s_tile, 0, md.N);   // published by the first task's barrier
-        for (int st = 0; st < sd.nsteps; ++st)
-            for (int half = 0; half < 2; ++half) {
-                // Priors of all proposals (in the idle slot memory), then only
-                // the proposals inside the prior support take likelihood slots.
-                sys_priors(md, pv, sweep, half, st, ntask, (char*)s_slot, sizeof(s_slot), s_tlp, NT);
-                __syncthreads();
-                const int nlive = compact_live(s_tlp, ntask, s_list, s_wcnt, NT);
-                for (int q0 = 0; q0 < nlive; q0 += SLOTS) {
-                    const int q = q0 + slot;
-                    const int b = q < nlive ? s_list[q] : -1;
-                    pt_half_task<PREC, WPT, EXT>(md, pv, sweep, half, st, b, b >= 0 ? s_tlp[b] : -__builtin_inf(),
-                                            s_slot[slot], s_tile, s_scan, s_acc, s_ops, slot, wsub, res, &s_cnt);
-                }
-                __syncthreads();     // this half's writes before the other half reads them
-            }
-        // Swap round on LDS copies that alias the (now idle) slot scratch.
-        double* L = (double*)s_slot;
-        double* LU = L + TW;
-        int* Mp = (int*)(LU + (T - 1) * W);
-        int* JP = Mp + TW;
-        pt_swap_stage(pv, sweep, L, Mp, LU, JP, NT);
-        for (int e = tid; e < T; e += NT) s_bet[e] = pv.betas[e];
-        __syncthreads();
-        pt_swap_round(pv, sweep, L, Mp, LU, JP, false, s_red, s_bet, NT);
-        for (int e = tid; e < TW; e += NT) pv.map[e] = Mp[e];
-        if (tid < T - 1) {
-            const double r = s_red[tid][0] / W;
-            s_rate[tid] = r;
-            s_smd[tid] = s_red[tid][1] / W;
-            sd.tsw_sum[(size_t)s * (T - 1) + tid] += r;
-            sd.smd_sum[(size_t)s * (T - 1) + tid] += s_red[tid][1] / W;
-        }
-        if (sd.rec_every > 0 && (sweep + 1) % sd.rec_every == 0) {
-            const long long r = (sweep + 1) / sd.rec_every - 1;
-            if (r < sd.max_rec) {
-                const int nw = sd.rec_temps * W, D = md.D;
-                double* hx = sd.h_x + r * sd.rec_x + sd.rxoff[s];
-                for (int e = tid; e < nw * D; e += NT) {
-                    const int w = e / D, d = e - w * D;
-                    hx[e] = pv.X[(size_t)Mp[w] * D + d];
-                }
-                const size_t o = ((size_t)r * sd.S + s) * nw;
-                for (int w = tid; w < nw; w += NT) {
-                    sd.h_lnl[o + w] = pv.lnl[Mp[w]];
-                    sd.h_lnp[o + w] = pv.lnp[Mp[w]];
-                }
-            }
-        }
-        if (pv.adapt_mode == 2) pt_lnl_spread(pv, L, s_sig, NT);
-        __syncthreads();
-        pt_ladder_update(pv, sweep, s_rate, s_smd, s_sig, s_bet, s_ld, NT);
-        if (tid == 0) atomicAdd(&sd.ctl[3], s_cnt);
+    const int T = sd.T, W = sd.W, TW = T * W;
+    const ModelDev& md = sys_model(sd, s);
+    const PTView pv = sys_view(sd, s, md.D);
+    double* L = (double*)s_scr;
+    double* LU = L + TW;
+    int* Mp = (int*)(LU + (T - 1) * W);
+    int* JP = Mp + TW;
+    pt_swap_stage(pv, sweep, L, Mp, LU, JP, SYS_PASS);
+    for (int e = tid; e < T; e += SYS_PASS) s_bet[e] = pv.betas[e];
+    __syncthreads();
+    pt_swap_round(pv, sweep, L, Mp, LU, JP, false, s_red, s_bet, SYS_PASS);
+    for (int e = tid; e < TW; e += SYS_PASS) pv.map[e] = Mp[e];
+    if (tid < T - 1) {
+        const double r = s_red[tid][0] / W;
+        s_rate[tid] = r;
+        s_smd[tid] = s_red[tid][1] / W;
+        sd.tsw_sum[(size_t)s * (T - 1) + tid] += r;
+        sd.smd_sum[(size_t)s * (T - 1) + tid] += s_red[tid][1] / W;
     }
+    if (sd.rec_every > 0 && (sweep + 1) % sd.rec_every == 0) {
+        const long long r = (sweep + 1) / sd.rec_every - 1;
+        if (r < sd.max_rec) {
+            const int nw = sd.rec_temps * W, D = md.D;
+            double* hx = sd.h_x + r * sd.rec_x + sd.rxoff[s];
+            for (int e = tid; e < nw * D; e += SYS_PASS) {
+                const int w = e / D, d = e - w * D;
+                hx[e] = pv.X[(size_t)Mp[w] * D + d];
+            }
+            const size_t o = ((size_t)r * sd.S + s) * nw;
+            for (int w = tid; w < nw; w += SYS_PASS) {
+                sd.h_lnl[o + w] = pv.lnl[Mp[w]];
+                sd.h_lnp[o + w] = pv.lnp[Mp[w]];
+            }
+        }
+    }
+    if (pv.adapt_mode == 2) pt_lnl_spread(pv, L, s_sig, SYS_PASS);
+    __syncthreads();
+    pt_ladder_update(pv, sweep, s_rate, s_smd, s_sig, s_bet, s_ld, SYS_PASS);
     if (tid == 0) {
         __threadfence();
         const unsigned long long f = atomicAdd(&sd.ctl[1], 1ull);
-        if (f == (unsigned long long)gridDim.x - 1) {   // every other workgroup has left
-            sd.ctl[0] = 0ull;
+        if (f == (unsigned long long)gridDim.x - 1) {   // every other workgroup has read the counter
             sd.ctl[1] = 0ull;
             sd.ctl[2] = (unsigned long long)(sweep + 1);
-        }
-    }
-}
-
-// Initial prior and likelihood of every walker (the state loaded into slot =
-// position order), one workgroup per system; the same arithmetic as the
-// batched likelihood kernel with the same waves per walker.
-template <int PREC, int WPT, int NW, bool EXT>
-__global__ __launch_bounds__(NW * 64) void k_sys_init(SysDev sd) {
-    constexpr int NT = NW * 64, SLOTS = NW / WPT;
-    __shared__ SlotLDS<SLOTS> s_slot[SLOTS];
-    __shared__ TileLDS s_tile;
-    __shared__ ScanLDS s_scan;
-    __shared__ double s_lp[SLOTS];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int slot = wave / WPT, wsub = wave % WPT;
-    const int s = blockIdx.x;
-    const ModelDev& md = sys_model(sd, s);
-    const PTView pv = sys_view(sd, s, md.D);
-    const int TW = sd.T * sd.W;
-    SlotLDS<SLOTS>& sl = s_slot[slot];
-    tab_load(md, s_tile);
-    for (int e = tid; e < TW; e += NT) pv.map[e] = e;
-    for (int b0 = 0; b0 < TW; b0 += SLOTS) {
-        const int b = b0 + slot;
-        const bool live = b < TW;
-        __syncthreads();
-        if (live) expand_theta(md, sl, pv.X + (size_t)b * md.D, wsub * 64 + lane, 64 * WPT);
-        __syncthreads();
-        if (live && wsub == 0 && lane == 0) s_lp[slot] = prior_seq(md, sl.theta);
-        slot_prepare<PREC, WPT>(md, sl, s_tile, live, wsub, lane);
-        double v = block_lnl<PREC, WPT, false, false, false, EXT>(md, sl, s_tile, s_scan, live, wsub, nullptr, nullptr);
-        if (live && wsub == 0 && lane == 0) {
-            if (!(v == v) || v == __builtin_inf()) v = -__builtin_inf();
-            const double lp = s_lp[slot];
-            pv.lnp[b] = lp;
-            pv.lnl[b] = lp > -__builtin_inf() ? v : -__builtin_inf();
         }
     }
 }
@@ -288,72 +362,71 @@ struct EmpSystems {
     hipGraphExec_t graph_exec = nullptr;
     EmpSystemsTuning tune{};
     int n_cu = 256;
-    bool ext = false;          // some system needs the extended instance (needs_ext)
+    bool ext = false;          // some system needs the extended instance (model_ext)
+    int max_d = 1, max_k = 1, max_l = 1;   // longest full vector, most planets, longest prior sequence of a system
     int64_t x_total = 0;
     double last_ms = -1.0;
 };
 
-// Static LDS of the sweep kernel's slot array (the swap round's working set
-// must fit in it).
-static size_t slot_bytes(int nw, int wpt) {
-    const int slots = nw / wpt;
-    return (size_t)slots * (slots <= 2 ? sizeof(SlotLDS<2>) : sizeof(SlotLDS<4>));
+#define EMP_SYS_CONFIGS(X) X(0, 1) X(0, 2) X(1, 1) X(1, 2)
+
+// Walkers per likelihood workgroup: two or four for every walker at work in it
+// (a workgroup's set-up serves them all), fewer while the pass has under eight
+// workgroups per compute unit (64 systems of 8 x 64 walkers: 168 / 147 us per
+// sweep at four / two; 512: 650 / 665).
+static int chunk_of(const EmpSystems* p, int64_t tasks) {
+    const int vecs = sys_vecs(p->tune.waves_per_theta);
+    int per = p->tune.waves_per_wg == 16 ? 4 : 2;
+    while (per > 1 && tasks < (int64_t)per * vecs * 8 * p->n_cu) per /= 2;
+    return vecs * per;
 }
-static size_t swap_bytes(int T, int W) { return (size_t)(2 * T - 1) * W * (sizeof(double) + sizeof(int)); }
 
-#define EMP_SYS_CONFIGS(X) X(0, 1, 8) X(0, 1, 16) X(0, 2, 8) X(0, 2, 16) X(1, 1, 8) X(1, 1, 16) X(1, 2, 8) X(1, 2, 16)
-
-template <int PREC, int WPT, int NW>
-static const void* sweep_fn(bool ext) {
-    return ext ? (const void*)&k_sys_sweep<PREC, WPT, NW, true> : (const void*)&k_sys_sweep<PREC, WPT, NW, false>;
+template <bool INIT>
+static int launch_lik(EmpSystems* p, int half, int step) {
+    const EmpSystemsTuning& tu = p->tune;
+    const int prec = p->desc.precision, S = p->desc.n_systems;
+    const int n = p->desc.ntemps * p->desc.nwalkers / (INIT ? 1 : 2), chunk = chunk_of(p, (int64_t)S * n);
+    const int nchunk = (n + chunk - 1) / chunk;
+    const size_t lds = sys_lds(tu.waves_per_theta, chunk, p->max_d, p->max_k);
+    const dim3 grid((unsigned)S * (unsigned)nchunk);
+#define EMP_CASE(P, WP)                                                                                      \
+    if (prec == P && tu.waves_per_theta == WP) {                                                            \
+        const dim3 nt(64 * WP * sys_vecs(WP));                                                               \
+        if (p->ext) hipLaunchKernelGGL((k_sys_lik<P, WP, true, INIT>), grid, nt, lds, p->stream, p->dev, half, step, chunk, nchunk); \
+        else hipLaunchKernelGGL((k_sys_lik<P, WP, false, INIT>), grid, nt, lds, p->stream, p->dev, half, step, chunk, nchunk); \
+        EMP_HIP(hipGetLastError());                                                                         \
+        return EMP_OK;                                                                                      \
+    }
+    EMP_SYS_CONFIGS(EMP_CASE)
+#undef EMP_CASE
+    emp_set_error("unsupported launch configuration (%d waves per walker)", tu.waves_per_theta);
+    return EMP_EINVAL;
 }
 
 static int launch_sweep(EmpSystems* p) {
-    const EmpSystemsTuning& tu = p->tune;
-    const int prec = p->desc.precision;
-    const int grid = std::max(1, std::min(p->desc.n_systems, p->n_cu * tu.wgs_per_cu));
-    p->dev.order = tu.order == 0 ? p->d_order_lpt : p->d_order_input;
-#define EMP_CASE(P, WP, NW)                                                                                \
-    if (prec == P && tu.waves_per_theta == WP && tu.waves_per_wg == NW) {                                 \
-        if (p->ext) hipLaunchKernelGGL((k_sys_sweep<P, WP, NW, true>), dim3(grid), dim3(NW * 64), 0, p->stream, p->dev); \
-        else hipLaunchKernelGGL((k_sys_sweep<P, WP, NW, false>), dim3(grid), dim3(NW * 64), 0, p->stream, p->dev); \
-        EMP_HIP(hipGetLastError());                                                                       \
-        return EMP_OK;                                                                                    \
-    }
-    EMP_SYS_CONFIGS(EMP_CASE)
-#undef EMP_CASE
-    emp_set_error("unsupported launch configuration (%d waves per workgroup, %d per walker)", tu.waves_per_wg,
-                  tu.waves_per_theta);
-    return EMP_EINVAL;
+    const unsigned S = (unsigned)p->desc.n_systems;
+    p->dev.order = p->tune.order == 0 ? p->d_order_lpt : p->d_order_input;
+    for (int st = 0; st < p->desc.nsteps; ++st)
+        for (int half = 0; half < 2; ++half) {
+            const int nc = (p->desc.ntemps * (p->desc.nwalkers / 2) + SYS_PRIOR_TASKS - 1) / SYS_PRIOR_TASKS;
+            const size_t terms = sys_prior_terms(p->max_l), lds = terms * sizeof(double) + p->max_l * sizeof(PseqEntry);
+            hipLaunchKernelGGL(k_sys_prior, dim3(S * (unsigned)nc), dim3(SYS_PASS), lds, p->stream, p->dev, half, st, nc,
+                               (int)terms);
+            EMP_HIP(hipGetLastError());
+            if (int rc = launch_lik<false>(p, half, st)) return rc;
+        }
+    hipLaunchKernelGGL(k_sys_swap, dim3(S), dim3(SYS_PASS), 0, p->stream, p->dev);
+    EMP_HIP(hipGetLastError());
+    return EMP_OK;
 }
 
-static int launch_init(EmpSystems* p) {
-    const EmpSystemsTuning& tu = p->tune;
-    const int prec = p->desc.precision;
-#define EMP_CASE(P, WP, NW)                                                                                           \
-    if (prec == P && tu.waves_per_theta == WP && tu.waves_per_wg == NW) {                                            \
-        if (p->ext) hipLaunchKernelGGL((k_sys_init<P, WP, NW, true>), dim3(p->desc.n_systems), dim3(NW * 64), 0, p->stream, p->dev); \
-        else hipLaunchKernelGGL((k_sys_init<P, WP, NW, false>), dim3(p->desc.n_systems), dim3(NW * 64), 0, p->stream, p->dev); \
-        EMP_HIP(hipGetLastError());                                                                                  \
-        return EMP_OK;                                                                                               \
-    }
-    EMP_SYS_CONFIGS(EMP_CASE)
-#undef EMP_CASE
-    emp_set_error("unsupported launch configuration");
-    return EMP_EINVAL;
-}
-
-static int check_tuning(const EmpSystems* p, const EmpSystemsTuning& t) {
+static int check_tuning(const EmpSystemsTuning& t) {
     if (!(t.waves_per_wg == 8 || t.waves_per_wg == 16) || !(t.waves_per_theta == 1 || t.waves_per_theta == 2)) {
         emp_set_error("waves_per_wg must be 8 or 16 and waves_per_theta 1 or 2");
         return EMP_EINVAL;
     }
     if (t.wgs_per_cu < 1 || t.wgs_per_cu > 4) { emp_set_error("wgs_per_cu must be in [1, 4]"); return EMP_EINVAL; }
     if (t.order != 0 && t.order != 1) { emp_set_error("order must be 0 (longest first) or 1 (input)"); return EMP_EINVAL; }
-    if (swap_bytes(p->desc.ntemps, p->desc.nwalkers) > slot_bytes(t.waves_per_wg, t.waves_per_theta)) {
-        emp_set_error("T x W too large for the LDS swap round of this configuration");
-        return EMP_EUNSUP;
-    }
     return EMP_OK;
 }
 
@@ -439,6 +512,7 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
     }
     std::vector<double> t(nep), y(nep), s2(nep), dt(nep), fixed(npar), sai(nsai);
     std::vector<int> ins(nep), inv(npar), fidx(nfree), bst(nblk), pseq(nseq), saib(nsaib);
+    std::vector<PseqEntry> pseq_e(nseq);
     std::vector<EmpPriorTerm> pri(npar), ecc(necc);
     std::vector<ModelDev> mds(S);
     std::vector<size_t> o_ep(S), o_par(S), o_free(S), o_blk(S), o_ecc(S), o_seq(S), o_sai(S), o_saib(S);
@@ -467,6 +541,7 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
             std::copy(h.bstart.begin(), h.bstart.end(), bst.begin() + b);
             std::copy(h.ecc.begin(), h.ecc.end(), ecc.begin() + c);
             std::copy(h.pseq.begin(), h.pseq.end(), pseq.begin() + g);
+            std::copy(h.pseq_e.begin(), h.pseq_e.end(), pseq_e.begin() + g);
             e += h.t.size(); q += h.inv.size(); f += h.free_idx.size(); b += h.bstart.size(); c += h.ecc.size();
             g += h.pseq.size();
             p->D[s] = h.dev.D;
@@ -489,6 +564,7 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
     double *dt_, *dy, *ds2, *ddt, *dfix, *dsai;
     int *dins, *dinv, *dfidx, *dbst, *dseq, *dsaib;
     EmpPriorTerm *dpri, *decc;
+    PseqEntry* dseq_e;
     double2* dtab;
     std::vector<double2> tab;
     emp_sincos_table(tab);
@@ -496,7 +572,7 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
         (rc = upload(p, dt, &ddt)) || (rc = upload(p, ins, &dins)) || (rc = upload(p, inv, &dinv)) ||
         (rc = upload(p, fixed, &dfix)) || (rc = upload(p, pri, &dpri)) || (rc = upload(p, fidx, &dfidx)) ||
         (rc = upload(p, bst, &dbst)) || (rc = upload(p, ecc, &decc)) || (rc = upload(p, tab, &dtab)) ||
-        (rc = upload(p, pseq, &dseq)) || (rc = upload(p, sai, &dsai)) || (rc = upload(p, saib, &dsaib))) {
+        (rc = upload(p, pseq, &dseq)) || (rc = upload(p, pseq_e, &dseq_e)) || (rc = upload(p, sai, &dsai)) || (rc = upload(p, saib, &dsaib))) {
         emp_systems_destroy(p);
         return rc;
     }
@@ -507,6 +583,7 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
         m.free_idx = dfidx + o_free[s]; m.block_start = dbst + o_blk[s]; m.ecc_prior = decc + o_ecc[s];
         m.sctab = dtab;
         m.pseq = dseq + o_seq[s];
+        m.pseq_e = dseq_e + o_seq[s];
         m.sai = dsai + o_sai[s];
         m.sai_base = dsaib + o_saib[s];
         if (!emp_model_dev_complete(m)) {
@@ -514,7 +591,10 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
             emp_set_error("system %d: a device array of the model is missing", s);
             return EMP_EINVAL;
         }
-        p->ext = p->ext || needs_ext(m);
+        p->ext = p->ext || model_ext(m) > 0;
+        p->max_d = std::max(p->max_d, m.Dfull);
+        p->max_k = std::max(p->max_k, m.K);
+        p->max_l = std::max(p->max_l, m.npseq);
         mds[s] = m;
     }
     // Queue orders: longest first (stable), and the input order.
@@ -534,7 +614,8 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
         (rc = alloc(p, &v.X, (size_t)p->x_total)) || (rc = alloc(p, &v.lnl, STW)) || (rc = alloc(p, &v.lnp, STW)) ||
         (rc = alloc(p, &v.map, STW)) || (rc = alloc(p, &v.betas, (size_t)S * T)) ||
         (rc = alloc(p, &v.accepted, STW)) || (rc = alloc(p, &v.tsw_sum, (size_t)S * std::max(T - 1, 1))) ||
-        (rc = alloc(p, &v.smd_sum, (size_t)S * std::max(T - 1, 1))) || (rc = alloc(p, &v.ctl, 4))) {
+        (rc = alloc(p, &v.smd_sum, (size_t)S * std::max(T - 1, 1))) || (rc = alloc(p, &v.ctl, 4)) ||
+        (rc = alloc(p, &v.tlp, STW / 2)) || (rc = alloc(p, &v.list, STW / 2)) || (rc = alloc(p, &v.nlive, (size_t)2 * S))) {
         emp_systems_destroy(p);
         return rc;
     }
@@ -554,18 +635,14 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
     EMP_TRY(hipMemset(v.accepted, 0, STW * sizeof(long long)));
     EMP_TRY(hipMemset(v.tsw_sum, 0, (size_t)S * std::max(T - 1, 1) * sizeof(double)));
     EMP_TRY(hipMemset(v.smd_sum, 0, (size_t)S * std::max(T - 1, 1) * sizeof(double)));
+    EMP_TRY(hipMemset(v.nlive, 0, 2 * (size_t)S * sizeof(int)));
     EMP_TRY(hipMemset(v.ctl, 0, 4 * sizeof(unsigned long long)));
     EMP_TRY(hipDeviceSynchronize());     // the engine stream does not wait for the null stream
 #undef EMP_TRY
-    // Default launch: 16 waves (16 walkers) per workgroup, one workgroup per
-    // compute unit, longest system first; 8-wave workgroups when the swap
-    // round does not fit.
+    // Default launch: 16 walkers per likelihood workgroup, one wave each, longest
+    // system first.
     p->tune = EmpSystemsTuning{16, 1, 1, 0, -1.0};
-    if (check_tuning(p, p->tune)) {
-        p->tune = EmpSystemsTuning{8, 1, 2, 0, -1.0};
-        if ((rc = check_tuning(p, p->tune))) { emp_systems_destroy(p); return rc; }
-    }
-    if ((rc = launch_init(p))) { emp_systems_destroy(p); return rc; }
+    if ((rc = launch_lik<true>(p, 0, 0))) { emp_systems_destroy(p); return rc; }
     if (hipStreamSynchronize(p->stream) != hipSuccess) {
         rc = emp_hip_fail(hipGetLastError(), "initial evaluation", __FILE__, __LINE__);
         emp_systems_destroy(p);
@@ -628,7 +705,7 @@ extern "C" int emp_systems_last_timing(EmpSystems* p, double* ms_per_sweep) {
 
 extern "C" int emp_systems_set_tuning(EmpSystems* p, const EmpSystemsTuning* t) {
     if (!p || !t) { emp_set_error("null argument"); return EMP_EINVAL; }
-    int rc = check_tuning(p, *t);
+    int rc = check_tuning(*t);
     if (rc) return rc;
     EMP_HIP(hipStreamSynchronize(p->stream));
     p->tune = *t;
@@ -693,28 +770,16 @@ extern "C" int emp_systems_autotune(EmpSystems* p, int32_t trial_sweeps, EmpSyst
     const int nws[2] = {16, 8}, wps[2] = {1, 2};
     for (int order = 0; order < 2 && !rc; ++order)
         for (int a = 0; a < 2 && !rc; ++a)
-            for (int b = 0; b < 2 && !rc; ++b)
-                for (int wpc = 1; wpc <= 4 && !rc; ++wpc) {
-                    EmpSystemsTuning c{nws[a], wps[b], wpc, order, -1.0};
-                    if (check_tuning(p, c)) continue;
-                    // persistent workgroups beyond what a compute unit holds would only queue
-                    int fit = 0;
-                    const void* fn = nullptr;
-                    const int prec = p->desc.precision;
-#define EMP_CASE(P, WP, NW) if (prec == P && c.waves_per_theta == WP && c.waves_per_wg == NW) fn = sweep_fn<P, WP, NW>(p->ext);
-                    EMP_SYS_CONFIGS(EMP_CASE)
-#undef EMP_CASE
-                    if (!fn || hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, fn, c.waves_per_wg * 64, 0) != hipSuccess)
-                        fit = 1;
-                    if (wpc > std::max(fit, 1)) continue;
-                    p->tune = c;
-                    double ms = 0.0;
-                    if ((rc = run_sweeps(p, 1, false, nullptr)) || (rc = run_sweeps(p, trial_sweeps, false, &ms)) ||
-                        (rc = snap_restore(p, sn)))
-                        break;
-                    c.ms_per_sweep = ms;
-                    if (best.ms_per_sweep < 0 || ms < best.ms_per_sweep) best = c;
-                }
+            for (int b = 0; b < 2 && !rc; ++b) {
+                EmpSystemsTuning c{nws[a], wps[b], 1, order, -1.0};
+                p->tune = c;
+                double ms = 0.0;
+                if ((rc = run_sweeps(p, 1, false, nullptr)) || (rc = run_sweeps(p, trial_sweeps, false, &ms)) ||
+                    (rc = snap_restore(p, sn)))
+                    break;
+                c.ms_per_sweep = ms;
+                if (best.ms_per_sweep < 0 || ms < best.ms_per_sweep) best = c;
+            }
     const int rc2 = snap_restore(p, sn);
     snap_free(sn);
     if (rc) { p->tune = keep; return rc; }

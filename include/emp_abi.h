@@ -372,12 +372,13 @@ typedef struct EmpSystemsDesc {
     int64_t max_records;        /* record capacity */
 } EmpSystemsDesc;
 
-/* Launch configuration of the batched sweep kernel, chosen by the autotuner
+/* Launch configuration of the batched likelihood pass, chosen by the autotuner
  * or set by the caller. */
 typedef struct EmpSystemsTuning {
-    int32_t waves_per_wg;       /* 8 or 16 */
+    int32_t waves_per_wg;       /* 8 or 16: walkers a workgroup of one wave per walker takes (2 or 4 per wave; with
+                                 * two waves per walker 2 or 4 in turn) */
     int32_t waves_per_theta;    /* 1 or 2 */
-    int32_t wgs_per_cu;         /* persistent workgroups per compute unit, 1..4 */
+    int32_t wgs_per_cu;         /* 1..4: accepted, no effect (the pass's workgroups are not persistent) */
     int32_t order;              /* 0: longest system first (LPT), 1: input order */
     double ms_per_sweep;        /* measured by the autotuner (output) */
 } EmpSystemsTuning;
@@ -389,8 +390,8 @@ int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDesc* desc, c
                        const double* p0, EmpSystems** out);
 void emp_systems_destroy(EmpSystems* sys);
 
-/* nsweeps sweeps of every system; one kernel launch per sweep (captured once
- * into a hipGraph when use_graph != 0).  Returns after completion. */
+/* nsweeps sweeps of every system; 4 nsteps + 1 kernel launches per sweep (captured
+ * once into a hipGraph when use_graph != 0).  Returns after completion. */
 int emp_systems_run(EmpSystems* sys, int64_t nsweeps, int32_t use_graph);
 
 /* Times every launch configuration that fits for trial_sweeps sweeps each
