@@ -92,6 +92,8 @@ struct EmpPT {
     long long hist_base = 0;     // first sweep whose history the engine holds (a restore from a
                                  // checkpoint without chain rows starts the history there)
     double last_ms_per_sweep = -1.0, last_ms_half = -1.0;
+    double* gather_buf = nullptr;    // device workspace of the state getters
+    size_t gather_cap = 0;
 };
 
 static __host__ __device__ inline PTView view_of(const PTDev& pd) {
@@ -1102,6 +1104,7 @@ extern "C" void emp_pt_destroy(EmpPT* p) {
     drop_graphs(p);
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     for (void* q : p->allocations) (void)hipFree(q);
+    if (p->gather_buf) (void)hipFree(p->gather_buf);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
 }
@@ -1375,29 +1378,27 @@ extern "C" int emp_pt_last_timing(EmpPT* p, double* ms_per_sweep, double* ms_hal
     return EMP_OK;
 }
 
-// Current state in logical order (gathered through the map) on the host.
-static int gather_state(EmpPT* p, std::vector<double>& X, std::vector<double>& l, std::vector<double>& lp) {
+// Current state in logical order (gathered through the map on the device).
+static int gather_state(EmpPT* p, int32_t what, double* out) {
     const PTDev& v = p->dev;
-    const size_t TW = (size_t)v.T * v.W;
-    std::vector<double> Xs(TW * v.D), ls(TW), ps(TW);
-    std::vector<int> mp(TW);
-    EMP_HIP(hipMemcpy(Xs.data(), v.X, Xs.size() * 8, hipMemcpyDeviceToHost));
-    EMP_HIP(hipMemcpy(ls.data(), v.lnl, ls.size() * 8, hipMemcpyDeviceToHost));
-    EMP_HIP(hipMemcpy(ps.data(), v.lnp, ps.size() * 8, hipMemcpyDeviceToHost));
-    EMP_HIP(hipMemcpy(mp.data(), v.map, mp.size() * 4, hipMemcpyDeviceToHost));
-    X.resize(TW * v.D); l.resize(TW); lp.resize(TW);
-    for (size_t w = 0; w < TW; ++w) {
-        const size_t s = (size_t)mp[w];
-        memcpy(&X[w * v.D], &Xs[s * v.D], (size_t)v.D * 8);
-        l[w] = ls[s];
-        lp[w] = ps[s];
-    }
-    return EMP_OK;
+    const int TW = v.T * v.W;
+    const double* src = what == EMP_PT_STATE_X ? v.X : what == EMP_PT_STATE_LNL ? v.lnl : v.lnp;
+    return emp_gather_rows(src, v.map, TW, TW, what == EMP_PT_STATE_X ? v.D : 1, &p->gather_buf, &p->gather_cap,
+                           p->stream, out);
 }
 
 extern "C" int emp_pt_get(EmpPT* p, int32_t what, void* host_out, int64_t cap, int64_t* shape) {
     if (!p || !host_out) { emp_set_error("null argument"); return EMP_EINVAL; }
     const PTDev& v = p->dev;
+    if (what == EMP_PT_STATE_X || what == EMP_PT_STATE_LNL || what == EMP_PT_STATE_LNP) {
+        const int64_t n = (int64_t)v.T * v.W * (what == EMP_PT_STATE_X ? v.D : 1);
+        if (n * (int64_t)sizeof(double) > cap) {
+            emp_set_error("output buffer too small (%lld bytes needed)", (long long)(n * sizeof(double)));
+            return EMP_EINVAL;
+        }
+        if (shape) { shape[0] = v.T; shape[1] = v.W; shape[2] = what == EMP_PT_STATE_X ? v.D : 1; shape[3] = 1; }
+        return gather_state(p, what, (double*)host_out);
+    }
     EMP_HIP(hipStreamSynchronize(p->stream));
     long long done = 0;
     EMP_HIP(hipMemcpy(&done, v.sweep, sizeof(done), hipMemcpyDeviceToHost));
@@ -1409,12 +1410,6 @@ extern "C" int emp_pt_get(EmpPT* p, int32_t what, void* host_out, int64_t cap, i
     int64_t sh[4] = {1, 1, 1, 1};
     const void* src = nullptr;
     size_t elem = sizeof(double);
-    std::vector<double> Xg, lg, pg;
-    if (what == EMP_PT_STATE_X || what == EMP_PT_STATE_LNL || what == EMP_PT_STATE_LNP) {
-        int rc = gather_state(p, Xg, lg, pg);
-        if (rc) return rc;
-    }
-    bool host_src = false;
     switch (what) {
         case EMP_PT_CHAIN:
             if (!v.record) goto norec;
@@ -1426,9 +1421,6 @@ extern "C" int emp_pt_get(EmpPT* p, int32_t what, void* host_out, int64_t cap, i
         case EMP_PT_TSW: sh[0] = S - S0; sh[1] = std::max(v.T - 1, 0); src = v.h_tsw + (size_t)S0 * T1; break;
         case EMP_PT_SMD: sh[0] = S - S0; sh[1] = std::max(v.T - 1, 0); src = v.h_smd + (size_t)S0 * T1; break;
         case EMP_PT_ACCEPTED: sh[0] = v.T; sh[1] = v.W; src = v.accepted; elem = sizeof(long long); break;
-        case EMP_PT_STATE_X: sh[0] = v.T; sh[1] = v.W; sh[2] = v.D; src = Xg.data(); host_src = true; break;
-        case EMP_PT_STATE_LNL: sh[0] = v.T; sh[1] = v.W; src = lg.data(); host_src = true; break;
-        case EMP_PT_STATE_LNP: sh[0] = v.T; sh[1] = v.W; src = pg.data(); host_src = true; break;
         case EMP_PT_STATE_BETAS: sh[0] = v.T; src = v.betas; break;
         case EMP_PT_NSWEEPS: sh[0] = 2; src = v.sweep; elem = sizeof(long long); break;
         case EMP_PT_GRAD_STEPS:
@@ -1440,10 +1432,7 @@ extern "C" int emp_pt_get(EmpPT* p, int32_t what, void* host_out, int64_t cap, i
     {
         const size_t n = (size_t)sh[0] * sh[1] * sh[2] * sh[3];
         if ((int64_t)(n * elem) > cap) { emp_set_error("output buffer too small (%zu bytes needed)", n * elem); return EMP_EINVAL; }
-        if (n) {
-            if (host_src) memcpy(host_out, src, n * elem);
-            else EMP_HIP(hipMemcpy(host_out, src, n * elem, hipMemcpyDeviceToHost));
-        }
+        if (n) EMP_HIP(hipMemcpy(host_out, src, n * elem, hipMemcpyDeviceToHost));
         if (shape) for (int i = 0; i < 4; ++i) shape[i] = sh[i];
         return EMP_OK;
     }
@@ -1636,10 +1625,12 @@ extern "C" int emp_pt_checkpoint(EmpPT* p, const char* path) {
     const PTDev& v = p->dev;
     EMP_HIP(hipStreamSynchronize(p->stream));
     const size_t TW = (size_t)v.T * v.W, T1 = (size_t)std::max(v.T - 1, 1);
-    std::vector<double> X, l, pr, b(v.T), buf;
+    std::vector<double> X(TW * v.D), l(TW), pr(TW), b(v.T), buf;
     std::vector<long long> acc(TW);
-    int rc = gather_state(p, X, l, pr);
-    if (rc) return rc;
+    int rc = 0;
+    if ((rc = gather_state(p, EMP_PT_STATE_X, X.data())) || (rc = gather_state(p, EMP_PT_STATE_LNL, l.data())) ||
+        (rc = gather_state(p, EMP_PT_STATE_LNP, pr.data())))
+        return rc;
     long long cnt[2] = {0, 0};
     EMP_HIP(hipMemcpy(b.data(), v.betas, b.size() * 8, hipMemcpyDeviceToHost));
     EMP_HIP(hipMemcpy(acc.data(), v.accepted, acc.size() * 8, hipMemcpyDeviceToHost));

@@ -9,6 +9,8 @@
 // 0 for a single system, so one system of a batch draws exactly what the
 // single-system engine draws.
 #pragma once
+#include <algorithm>
+
 #include "emp_kernels.h"
 
 namespace emp {
@@ -329,4 +331,43 @@ __device__ inline void pt_ladder_update(const PTView& pv, long long sweep, const
     }
 }
 
+// Reading a state back: rows of src (`width` doubles each) taken through the map,
+// logical walkers [w0, w0 + n) of a list in which every `per` consecutive walkers
+// have slots of their own (one ensemble; the ensembles of a batch), into out.
+__global__ static void k_gather_rows(const double* __restrict__ src, const int* __restrict__ map, long long w0,
+                                     long long n, int per, int width, double* __restrict__ out) {
+    const long long total = n * width;
+    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < total;
+         e += (long long)gridDim.x * blockDim.x) {
+        const long long w = w0 + e / width;
+        out[e] = src[((w / per) * per + map[w]) * width + e % width];
+    }
+}
+
 }  // namespace emp
+
+// Gathers n rows on the device in pieces of at most 32 MiB (the engine's `buf`,
+// grown to the piece once and kept) and copies each to the host: one kernel and
+// one copy where every buffer used to be copied whole and permuted by the host.
+constexpr size_t GATHER_MOST = (size_t)4 << 20;      // doubles
+inline int emp_gather_rows(const double* src, const int* map, long long n, int per, int width, double** buf,
+                           size_t* cap, hipStream_t s, double* host) {
+    const long long piece = std::max<long long>(1, std::min<long long>(n, (long long)(GATHER_MOST / width)));
+    const size_t need = (size_t)piece * width;
+    if (*cap < need) {
+        if (*buf) (void)hipFree(*buf);
+        *buf = nullptr;
+        *cap = 0;
+        EMP_HIP(hipMalloc((void**)buf, need * sizeof(double)));
+        *cap = need;
+    }
+    for (long long w0 = 0; w0 < n; w0 += piece) {
+        const long long m = std::min(piece, n - w0), total = m * width;
+        const unsigned grid = (unsigned)std::min<long long>((total + 255) / 256, 8192);
+        hipLaunchKernelGGL(emp::k_gather_rows, dim3(grid), dim3(256), 0, s, src, map, w0, m, per, width, *buf);
+        EMP_HIP(hipGetLastError());
+        EMP_HIP(hipMemcpyAsync(host + w0 * width, *buf, (size_t)total * sizeof(double), hipMemcpyDeviceToHost, s));
+        EMP_HIP(hipStreamSynchronize(s));    // before the buffer is written again, and before the caller reads
+    }
+    return EMP_OK;
+}

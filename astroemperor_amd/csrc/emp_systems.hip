@@ -366,6 +366,8 @@ struct EmpSystems {
     int max_d = 1, max_k = 1, max_l = 1;   // longest full vector, most planets, longest prior sequence of a system
     int64_t x_total = 0;
     double last_ms = -1.0;
+    double* gather_buf = nullptr;    // device workspace of the state getters
+    size_t gather_cap = 0;
 };
 
 #define EMP_SYS_CONFIGS(X) X(0, 1) X(0, 2) X(1, 1) X(1, 2)
@@ -452,6 +454,7 @@ extern "C" void emp_systems_destroy(EmpSystems* p) {
     if (p->graph_exec) (void)hipGraphExecDestroy(p->graph_exec);
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     for (void* q : p->allocations) (void)hipFree(q);
+    if (p->gather_buf) (void)hipFree(p->gather_buf);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
 }
@@ -794,21 +797,19 @@ extern "C" int emp_systems_autotune(EmpSystems* p, int32_t trial_sweeps, EmpSyst
     return EMP_OK;
 }
 
-// One system's current state in position order.
-static int gather_one(EmpSystems* p, int s, int what, double* out) {
+// The current state of systems [s0, s1) in position order (gathered through the
+// maps on the device).
+static int gather_systems(EmpSystems* p, int s0, int s1, int what, double* out) {
     const SysDev& v = p->dev;
-    const size_t TW = (size_t)v.T * v.W;
-    const int D = p->D[s];
-    std::vector<int> mp(TW);
-    EMP_HIP(hipMemcpy(mp.data(), v.map + s * TW, TW * 4, hipMemcpyDeviceToHost));
-    if (what == EMP_PT_STATE_X) {
-        std::vector<double> xs(TW * D);
-        EMP_HIP(hipMemcpy(xs.data(), v.X + p->xoff[s], xs.size() * 8, hipMemcpyDeviceToHost));
-        for (size_t w = 0; w < TW; ++w) memcpy(out + w * D, &xs[(size_t)mp[w] * D], (size_t)D * 8);
-    } else {
-        std::vector<double> ls(TW);
-        EMP_HIP(hipMemcpy(ls.data(), (what == EMP_PT_STATE_LNL ? v.lnl : v.lnp) + s * TW, TW * 8, hipMemcpyDeviceToHost));
-        for (size_t w = 0; w < TW; ++w) out[w] = ls[mp[w]];
+    const int TW = v.T * v.W;
+    if (what != EMP_PT_STATE_X)
+        return emp_gather_rows((what == EMP_PT_STATE_LNL ? v.lnl : v.lnp) + (size_t)s0 * TW, v.map + (size_t)s0 * TW,
+                               (long long)(s1 - s0) * TW, TW, 1, &p->gather_buf, &p->gather_cap, p->stream, out);
+    for (int s = s0; s < s1; ++s) {
+        const int rc = emp_gather_rows(v.X + p->xoff[s], v.map + (size_t)s * TW, TW, TW, p->D[s], &p->gather_buf,
+                                       &p->gather_cap, p->stream, out);
+        if (rc) return rc;
+        out += (size_t)TW * p->D[s];
     }
     return EMP_OK;
 }
@@ -848,12 +849,7 @@ extern "C" int emp_systems_get(EmpSystems* p, int32_t what, int32_t system, void
             for (int s = s0; s < s1; ++s) n += TW * p->D[s];
             if (system >= 0) { sh[0] = T; sh[1] = W; sh[2] = p->D[system]; } else { sh[0] = (int64_t)n; }
             if (!need(n)) return EMP_EINVAL;
-            double* o = (double*)host_out;
-            for (int s = s0; s < s1; ++s) {
-                int rc = gather_one(p, s, what, o);
-                if (rc) return rc;
-                o += TW * p->D[s];
-            }
+            if (int rc = gather_systems(p, s0, s1, what, (double*)host_out)) return rc;
             break;
         }
         case EMP_PT_STATE_LNL:
@@ -861,10 +857,7 @@ extern "C" int emp_systems_get(EmpSystems* p, int32_t what, int32_t system, void
             n = (size_t)ns * TW;
             if (system >= 0) { sh[0] = T; sh[1] = W; } else { sh[0] = S; sh[1] = T; sh[2] = W; }
             if (!need(n)) return EMP_EINVAL;
-            for (int s = s0; s < s1; ++s) {
-                int rc = gather_one(p, s, what, (double*)host_out + (size_t)(s - s0) * TW);
-                if (rc) return rc;
-            }
+            if (int rc = gather_systems(p, s0, s1, what, (double*)host_out)) return rc;
             break;
         }
         case EMP_PT_ACCEPTED:
