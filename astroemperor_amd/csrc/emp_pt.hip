@@ -124,33 +124,36 @@ __device__ __forceinline__ void record_walker(const PTDev& pd, long long s, int 
     }
 }
 
+// Record the state before this step's moves (nothing has moved since the
+// previous step, or the previous sweep's swap round): walker k of half 0 and its
+// half-1 twin, by one wave (task b of half 0).
+__device__ __forceinline__ void record_pair(const PTDev& pd, int step, int b, int lane) {
+    if (!pd.record || !(step > 0 || *pd.rec_owed)) return;
+    const long long s = *pd.sweep * pd.nsteps + step - 1;
+    if (s < 0 || s >= pd.max_rows) return;
+    const int t = b / pd.W2, k = b % pd.W2;
+    record_walker(pd, s, t * pd.W + k, lane);
+    record_walker(pd, s, t * pd.W + k + pd.W2, lane);
+}
+
+// The swap round's pairings and uniforms depend on (seed, sweep, pair) only: pair
+// e of (T - 1) W.
+__device__ __forceinline__ void draw_swap(const PTDev& pd, const PTView& pv, int e) {
+    if (e >= (pd.T - 1) * pd.W) return;
+    const long long sweep = *pd.sweep;
+    const int h = e / pd.W + 1, i = e - (h - 1) * pd.W;
+    pd.swap_jp[e] = (int)swap_partner(pv, sweep, h, i);
+    pd.swap_lu[e] = swap_logu(pv, sweep, h, i);
+}
+
 __global__ __launch_bounds__(PRIOR_BLOCK) void k_pt_prior(ModelDev md, PTDev pd, int half, int step, int draw_swaps,
                                                           int first) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int b = blockIdx.x * PRIOR_WAVES + wave;
     const PTView pv = view_of(pd);
-    if (first && pd.record && (step > 0 || *pd.rec_owed) && b < pd.T * pd.W2) {
-        // A step's first pass records the state before it (nothing has moved
-        // since): the previous step's, or the previous sweep's after its
-        // swap round.  Walker k of half 0 and its half-1 twin.
-        const long long s = *pd.sweep * pd.nsteps + step - 1;
-        if (s >= 0 && s < pd.max_rows) {
-            const int t = b / pd.W2, k = b % pd.W2;
-            record_walker(pd, s, t * pd.W + k, lane);
-            record_walker(pd, s, t * pd.W + k + pd.W2, lane);
-        }
-    }
-    if (draw_swaps) {
-        // The swap round's pairings and uniforms depend on (seed, sweep, pair)
-        // only; this grid has T W / 2 x 64 threads >= (T - 1) W pairs.
-        const int e = blockIdx.x * PRIOR_BLOCK + threadIdx.x;
-        if (e < (pd.T - 1) * pd.W) {
-            const long long sweep = *pd.sweep;
-            const int h = e / pd.W + 1, i = e - (h - 1) * pd.W;
-            pd.swap_jp[e] = (int)swap_partner(pv, sweep, h, i);
-            pd.swap_lu[e] = swap_logu(pv, sweep, h, i);
-        }
-    }
+    if (first && b < pd.T * pd.W2) record_pair(pd, step, b, lane);
+    // this grid has T W / 2 x 64 threads >= (T - 1) W pairs
+    if (draw_swaps) draw_swap(pd, pv, blockIdx.x * PRIOR_BLOCK + threadIdx.x);
     if (b >= pd.T * pd.W2) return;            // whole waves
     // What does not depend on the random draws is loaded first, so that it
     // is in flight while the counter is read and Philox runs.
@@ -232,6 +235,80 @@ __global__ __launch_bounds__(64 * WPT * vecs_per_wg(WPT)) void k_pt_half(ModelDe
     if (s_acc[slot]) {
         double* Xk = pd.X + (size_t)ops.sk * pd.D;
         for (int d = g; d < md.D; d += G) Xk[d] = sl.theta[md.free_idx[d]];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The whole half-step in one launch, for ensembles whose proposals all fit the
+// chip at once (fuse_half): one workgroup of WPT waves per walker of the moving
+// half draws the proposal, then evaluates its prior (wave 0), its planets'
+// constants (wave 1) and its acceptance operands (the last wave) side by side,
+// and leaves if the proposal lies outside the support.  The same values as
+// k_pt_prior and k_pt_half, bit for bit.  A launch of this size is bound by
+// latency: the second launch, the record and the row between the passes cost
+// more than the workgroups that leave.
+// ---------------------------------------------------------------------------
+template <int PREC, int WPT, int EXT>
+__global__ __launch_bounds__(64 * WPT) void k_pt_step(ModelDev md, PTDev pd, int half, int step, int draw_swaps,
+                                                     int first) {
+    static_assert(WPT >= 2, "one workgroup per walker, at least two waves");
+    __shared__ SlotLDS<1> sl;
+    __shared__ SinCosTab s_tab;
+    __shared__ ScanLDS s_scan;
+    __shared__ TaskOps s_ops;
+    __shared__ int s_acc;
+    const int wave = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63, g = threadIdx.x, b = blockIdx.x;
+    const PTView pv = view_of(pd);
+    // What does not depend on the random draws is loaded first, so that it
+    // is in flight while the counter is read and Philox runs.
+    const int t = b / pd.W2, k = half * pd.W2 + b % pd.W2;
+    const int sk = pd.map[t * pd.W + k];
+    const double beta = pd.betas[t], lnl_old = pd.lnl[sk], lnp_old = pd.lnp[sk];
+    const Proposal pr = pt_propose(pv, *pd.sweep, half, step, b);
+    const double* Xk = pd.X + (size_t)pr.sk * pd.D;
+    const double* Xj = pd.X + (size_t)pr.sj * pd.D;
+    for (int q = g; q < md.Dfull; q += 64 * WPT) {
+        const int f = md.inv_free[q];
+        sl.theta[q] = f >= 0 ? pt_prop_value(Xk, Xj, pr.z, f) : md.fixed_val[q];
+    }
+    tab_load(md, s_tab);
+    if (draw_swaps) draw_swap(pd, pv, b * 64 * WPT + g);     // (T W / 2 x 64 WPT threads)
+    // every walker of the moving half is written only by its own workgroup, after this
+    if (first && wave == WPT - 1) record_pair(pd, step, b, lane);
+    __syncthreads();
+    if (wave == WPT - 1 && lane == 0) {
+        s_ops.t = pr.t;
+        s_ops.k = pr.k;
+        s_ops.sk = pr.sk;
+        s_ops.beta = beta;
+        s_ops.lz = (double)(pd.D - 1) * log(pr.z);
+        s_ops.to = beta == 0.0 ? 0.0 : beta * lnl_old;
+        s_ops.logu = log(pr.uacc);
+    }
+    if (wave == 1) slot_setup(md, sl, lane);
+    if (wave == 0) {
+        const double lp = prior_vector_wave(md, sl.theta, lane);
+        if (lane == 0) {
+            s_ops.lp = lp;
+            s_ops.dp = lp - lnp_old;
+        }
+    }
+    __syncthreads();
+    if (!(s_ops.lp > -__builtin_inf())) return;              // the whole workgroup
+    for (int p = wave; p < md.K; p += WPT)
+        if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
+    __syncthreads();
+    const double ll = vec_lnl<PREC, WPT, false, false, EXT>(md, sl, s_tab, s_scan, true, wave);
+    if (g == 0) {
+        atomicAdd((unsigned long long*)(pd.sweep + 1), 1ull);
+        s_acc = pt_decide(pv, s_ops, ll);
+        // an accepted stretch move leaves the slot's gradient out of date
+        if (pd.lg_stale && s_acc) pd.lg_stale[s_ops.sk] = 1;
+    }
+    __syncthreads();
+    if (s_acc) {
+        double* Xw = pd.X + (size_t)s_ops.sk * pd.D;
+        for (int d = g; d < md.D; d += 64 * WPT) Xw[d] = sl.theta[md.free_idx[d]];
     }
 }
 
@@ -430,13 +507,7 @@ __global__ __launch_bounds__(SWAP_BLOCK) void k_pt_swap(PTDev pd) {
 // The swap round's randoms for a sweep without stretch half-steps (the
 // gradient-move sweep).
 __global__ void k_pt_swap_draw(PTDev pd) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (pd.T - 1) * pd.W) return;
-    const PTView pv = view_of(pd);
-    const long long sweep = *pd.sweep;
-    const int h = e / pd.W + 1, i = e - (h - 1) * pd.W;
-    pd.swap_jp[e] = (int)swap_partner(pv, sweep, h, i);
-    pd.swap_lu[e] = swap_logu(pv, sweep, h, i);
+    draw_swap(pd, view_of(pd), blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // History row of the state before step `step` of the current sweep (step 0:
@@ -945,9 +1016,51 @@ static int launch_lik(EmpPT* p, int half, int step, hipEvent_t e0 = nullptr, hip
     return EMP_EINVAL;
 }
 
-static int launch_half(EmpPT* p, int half, int step, int draw_swaps, int first = 0) {
-    const int rc = launch_prior(p, half, step, draw_swaps, first);
-    return rc ? rc : launch_lik(p, half, step);
+template <int PREC, int WPT>
+static void launch_step_t(const ModelDev& md, const PTDev& pd, int half, int step, int draw_swaps, int first,
+                          hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+    const dim3 grid((unsigned)(pd.T * pd.W2)), nt(64 * WPT);
+#define EMP_STEP(E)                                                                                                  \
+    do {                                                                                                             \
+        if (e0) hipExtLaunchKernelGGL((k_pt_step<PREC, WPT, E>), grid, nt, 0, s, e0, e1, 0, md, pd, half, step, draw_swaps, first); \
+        else hipLaunchKernelGGL((k_pt_step<PREC, WPT, E>), grid, nt, 0, s, md, pd, half, step, draw_swaps, first);   \
+    } while (0)
+    switch (model_ext(md)) {
+        case 0: EMP_STEP(0); break;
+        case 1: EMP_STEP(1); break;
+        default: EMP_STEP(2);
+    }
+#undef EMP_STEP
+}
+
+// One launch per half-step (k_pt_step) while every workgroup of it is resident
+// at once: at most FUSE_WAVES waves per SIMD (its registers allow six or seven).
+// Stretch sweeps with two launches per half-step against one: 5 x 100 walkers, 1
+// planet x 256 epochs, FP64, 36.1 -> 25.5 us; 10 x 256, 3 x 1530, mixed, 76.9 ->
+// 67.5 us (FP64 79.1 -> 68.6); 8 x 200, 2 x 400, 48.8 -> 40.9 us; 6 x 60, 5 x 3000,
+// 63.5 -> 55.4 us.  Beyond, the workgroups whose proposal lies outside the
+// support would queue before the others.
+constexpr int FUSE_WAVES = 6;
+static bool fuse_half(const EmpPT* p) {
+    return p->wpt >= 2 && (int64_t)p->dev.T * p->dev.W2 * p->wpt <= (int64_t)FUSE_WAVES * 4 * p->model->n_cu;
+}
+
+// One half-step; with events, those of its likelihood launch (or of its only
+// one).
+static int launch_half(EmpPT* p, int half, int step, int draw_swaps, int first = 0, hipEvent_t e0 = nullptr,
+                       hipEvent_t e1 = nullptr) {
+    if (!fuse_half(p)) {
+        const int rc = launch_prior(p, half, step, draw_swaps, first);
+        return rc ? rc : launch_lik(p, half, step, e0, e1);
+    }
+    const ModelDev& md = p->model->dev;
+    const int prec = p->desc.precision, w = p->wpt;
+#define EMP_CASE(P, W) if (prec == P && w == W) { launch_step_t<P, W>(md, p->dev, half, step, draw_swaps, first, p->stream, e0, e1); EMP_HIP(hipGetLastError()); return EMP_OK; }
+    EMP_CASE(0, 2) EMP_CASE(0, 4) EMP_CASE(0, 8)
+    EMP_CASE(1, 2) EMP_CASE(1, 4) EMP_CASE(1, 8)
+#undef EMP_CASE
+    emp_set_error("bad precision/wpt");
+    return EMP_EINVAL;
 }
 
 // Swap round (with ladder and sweep counter): the end of every sweep,
@@ -1248,9 +1361,8 @@ extern "C" int emp_pt_time_halfstep(EmpPT* p, int32_t n, double* ms_avg) {
     for (int64_t sw = 0; sw < ns && !rc; ++sw) {
         for (int st = 0; st < p->desc.nsteps && !rc; ++st)
             for (int h = 0; h < 2 && !rc; ++h) {
-                rc = launch_prior(p, h, st, h == 1 && st == p->desc.nsteps - 1, h == 0);
-                if (rc) break;
-                rc = k < n ? launch_lik(p, h, st, ev[2 * k], ev[2 * k + 1]) : launch_lik(p, h, st);
+                rc = launch_half(p, h, st, h == 1 && st == p->desc.nsteps - 1, h == 0, k < n ? ev[2 * k] : nullptr,
+                                 k < n ? ev[2 * k + 1] : nullptr);
                 ++k;
             }
         if (!rc) rc = launch_tail(p);
