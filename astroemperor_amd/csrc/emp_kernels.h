@@ -41,22 +41,49 @@ __device__ inline double prior_term(const EmpPriorTerm& p, double x) {
     }
 }
 
-__device__ inline double prior_seq(const ModelDev& md, const double* th) {
+// Sum of a vector's prior terms by one whole wave, as if term by term: each
+// block's free parameters, a return if the sum is -inf at the block's end, then
+// the block's derived eccentricity prior.  The lanes evaluate the terms of that
+// sequence in parallel, with their loads in flight together (term(entry, i): the
+// value of sequence entry i), then the terms are added up in sequence order (a
+// scalar read of each lane), with the -inf return where a ballot marks a block's
+// end, so that every caller forms the same bits.
+template <class F>
+__device__ __forceinline__ double prior_wave(const ModelDev& md, int lane, F term) {
 #pragma clang fp contract(off)
     double lp = 0.0;
-    for (int b = 0; b < md.nblocks; ++b) {
-        for (int j = md.block_start[b]; j < md.block_start[b + 1]; ++j) {
-            if (md.inv_free[j] < 0) continue;
-            lp += prior_term(md.prior[j], th[j]);
+    for (int i0 = 0; i0 < md.npseq; i0 += 64) {
+        const int i = i0 + lane;
+        double v = 0.0;
+        int kind = 0;
+        if (i < md.npseq) {
+            const PseqEntry& pe = md.pseq_e[i];
+            kind = pe.kind;
+            if (kind != 2) v = term(pe, i);
         }
-        if (lp == -__builtin_inf()) return lp;
-        if (b < md.K && md.ecc_prior[b].kind != EMP_PRIOR_NONE) {
-            const double* s = th + md.off_kep + 5 * b;
-            double x = s[3] * s[3] + s[4] * s[4];
-            lp += prior_term(md.ecc_prior[b], x);
+        const unsigned long long chk = __ballot(i < md.npseq && kind == 2);
+        const int n = min(64, md.npseq - i0);
+        for (int k = 0; k < n; ++k) {
+            if ((chk >> k) & 1ull) {
+                if (lp == -__builtin_inf()) return lp;
+            } else {
+                lp += readlane_f64(v, k);
+            }
         }
     }
     return lp;
+}
+
+// Prior of a full parameter vector (fixed values in place).
+__device__ inline double prior_vector_wave(const ModelDev& md, const double* th, int lane) {
+    return prior_wave(md, lane, [&](const PseqEntry& pe, int i) {
+#pragma clang fp contract(off)
+        const int q = md.pseq[i];
+        if (pe.kind == 0) return prior_term(pe.term, th[q]);
+        const double* sc = th + md.off_kep + 5 * (PSEQ_ECC - q) + 3;
+        const double x = sc[0] * sc[0] + sc[1] * sc[1];
+        return prior_term(pe.term, x);
+    });
 }
 
 // Planet p's constants of the full parameter vector th.

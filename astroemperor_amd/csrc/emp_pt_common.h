@@ -76,38 +76,6 @@ __device__ __forceinline__ double pt_prop_value(const double* Xk, const double* 
     return __builtin_fma(z, Xk[f] - Xj[f], Xj[f]);
 }
 
-// Sum of a vector's prior terms by one whole wave, in the order of prior_seq:
-// the lanes evaluate the terms of the summation sequence in parallel, with their
-// loads in flight together (term(entry, i): the value of sequence entry i), then
-// the terms are added up in sequence order (a scalar read of each lane) with
-// prior_seq's -inf return at the block ends, which a ballot marks, so the sum is
-// bit-identical.
-template <class F>
-__device__ __forceinline__ double prior_wave(const ModelDev& md, int lane, F term) {
-#pragma clang fp contract(off)
-    double lp = 0.0;
-    for (int i0 = 0; i0 < md.npseq; i0 += 64) {
-        const int i = i0 + lane;
-        double v = 0.0;
-        int kind = 0;
-        if (i < md.npseq) {
-            const PseqEntry& pe = md.pseq_e[i];
-            kind = pe.kind;
-            if (kind != 2) v = term(pe, i);
-        }
-        const unsigned long long chk = __ballot(i < md.npseq && kind == 2);
-        const int n = min(64, md.npseq - i0);
-        for (int k = 0; k < n; ++k) {
-            if ((chk >> k) & 1ull) {
-                if (lp == -__builtin_inf()) return lp;
-            } else {
-                lp += readlane_f64(v, k);
-            }
-        }
-    }
-    return lp;
-}
-
 // Prior of a proposal, read straight from the two walkers' rows.
 __device__ inline double prior_proposal_wave(const ModelDev& md, const double* Xk, const double* Xj, double z,
                                              int lane) {
@@ -117,18 +85,6 @@ __device__ inline double prior_proposal_wave(const ModelDev& md, const double* X
         const double s3 = pe.fa >= 0 ? pt_prop_value(Xk, Xj, z, pe.fa) : pe.va;
         const double s4 = pe.fb >= 0 ? pt_prop_value(Xk, Xj, z, pe.fb) : pe.vb;
         const double x = s3 * s3 + s4 * s4;
-        return prior_term(pe.term, x);
-    });
-}
-
-// Prior of a full parameter vector (fixed values in place).
-__device__ inline double prior_vector_wave(const ModelDev& md, const double* th, int lane) {
-    return prior_wave(md, lane, [&](const PseqEntry& pe, int i) {
-#pragma clang fp contract(off)
-        const int q = md.pseq[i];
-        if (pe.kind == 0) return prior_term(pe.term, th[q]);
-        const double* sc = th + md.off_kep + 5 * (PSEQ_ECC - q) + 3;
-        const double x = sc[0] * sc[0] + sc[1] * sc[1];
         return prior_term(pe.term, x);
     });
 }

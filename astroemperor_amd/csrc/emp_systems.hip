@@ -81,8 +81,8 @@ __device__ __forceinline__ PTView sys_view(const SysDev& sd, int s, int D) {
 // system s: the proposals (one thread per task), every (task, term) pair of the
 // prior's summation sequence (the system's resolved sequence in LDS, all loads
 // of the walkers' rows in flight together), then the sum of each task's terms in
-// sequence order with prior_seq's -inf return (one thread per task),
-// bit-identical to prior_seq.  The tasks inside the support are appended to the
+// sequence order with prior_wave's -inf return (one thread per task),
+// bit-identical to prior_wave.  The tasks inside the support are appended to the
 // system's list (in any order: the tasks of a half-step are independent); the
 // other half's count is cleared for its next pass.  The term values take
 // `terms` doubles of LDS, a few tasks at a time where a long sequence needs it.
@@ -271,9 +271,9 @@ __global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_wav
         vec_sync<WPT>();
         double ll = vec_lnl<PREC, WPT, false, false, EXT ? 2 : 0>(md, sl, s_tab, s_scan, true, wsub);
         if (INIT) {
+            const double lp = prior_vector_wave(md, sl.theta, lane);
             if (wsub == 0 && lane == 0) {
                 const int b = q0 + r;
-                const double lp = prior_seq(md, sl.theta);
                 if (!(ll == ll) || ll == __builtin_inf()) ll = -__builtin_inf();
                 pv.map[b] = b;
                 pv.lnp[b] = lp;
