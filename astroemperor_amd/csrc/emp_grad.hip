@@ -1268,10 +1268,11 @@ static void launch_grad_t(const ModelDev& md, const double* th, int64_t B, int64
 // 84 / 86 / 168 / 238 (7 planets with MA(1), mixed: 135 / 139 / 223 / 361
 // against 172 / 166 / 320 / 536).
 constexpr int GRAD1_NW = 2;
-// Below this many epochs the two-pass kernel used to be the default: a batch
-// whose eps rows would not fit the allocation-free entry point's scratch stays
-// refused there.
-constexpr int NOALLOC_TWO_PASS_N = 1024;
+// Below this many epochs the default kernel is one that a caller may still
+// replace by the two-pass one after scratch was set aside for it: a batch whose
+// eps rows would not fit the allocation-free entry point's scratch is refused
+// there, and the gradient move holds the rows (emp_grad_scratch_reserve).
+constexpr int TWO_PASS_RESERVE_N = 1024;
 
 static bool use_grad1(const EmpModel* m) {
     const ModelDev& md = m->dev;
@@ -1298,6 +1299,15 @@ extern "C" int emp_model_set_grad_kernel(EmpModel* m, int32_t which) {
 // otherwise.
 size_t emp_grad_scratch_doubles(const EmpModel* m, int64_t B) {
     return (m->dev.ma_active && !use_grad1(m)) ? (size_t)B * (size_t)m->dev.N : 0;
+}
+
+// Doubles to set aside where the scratch is fixed before the kernel is: what a
+// launch needs now, and below TWO_PASS_RESERVE_N epochs also what it would need
+// after a switch of the default to the two-pass kernel.
+size_t emp_grad_scratch_reserve(const EmpModel* m, int64_t B) {
+    if (m->grad_kernel == EMP_GRAD_KERNEL_AUTO && m->dev.ma_active && m->dev.N < TWO_PASS_RESERVE_N)
+        return (size_t)B * (size_t)m->dev.N;
+    return emp_grad_scratch_doubles(m, B);
 }
 
 // The MA adjoint's scratch, model-owned, grown (never shrunk) on demand.
@@ -1339,6 +1349,16 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
     if (use_grad1(m)) {
         const ModelDev& md = m->dev;
         if (precision != 0 && precision != 1) { emp_set_error("bad precision"); return EMP_EINVAL; }
+        // a grid holds fewer than 2^32 threads: larger batches in pieces
+        constexpr int64_t PIECE = (int64_t)1 << 24;
+        if (B > PIECE) {
+            for (int64_t b = 0; b < B; b += PIECE) {
+                const int rc = emp_launch_grad_ws(m, th + b * ld, std::min(PIECE, B - b), ld, lnl + b, grad + b * md.D,
+                                                  eps_scratch, s, precision, stale ? stale + b : nullptr, wpt);
+                if (rc) return rc;
+            }
+            return EMP_OK;
+        }
 #define EMP_CASE1(P, E, A, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, GRAD1_NW, M, T>), dim3((unsigned)B), dim3(64 * GRAD1_NW), 0, s, md, th, B, ld, lnl, grad, nf, stale)
 #define EMP_CASE1M(P, E, A, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, GRAD1_FEW, T); else if (md.K <= 6) EMP_CASE1(P, E, A, 6, T); else EMP_CASE1(P, E, A, KMAX, T); }
 #define EMP_CASE1A(P, E, T) { if (md.ma_active) EMP_CASE1M(P, E, true, T) else EMP_CASE1M(P, E, false, T) }
@@ -1439,9 +1459,7 @@ extern "C" int emp_lnl_grad_batch_noalloc(EmpModel* m, const double* theta, int6
         return EMP_EINVAL;
     }
     if (flags & ~EMP_GRAD_MIXED) { emp_set_error("unknown flags 0x%x", (unsigned)flags); return EMP_EINVAL; }
-    size_t need = emp_grad_scratch_doubles(m, B);
-    if (m->grad_kernel == EMP_GRAD_KERNEL_AUTO && m->dev.ma_active && m->dev.N < NOALLOC_TWO_PASS_N)
-        need = (size_t)B * (size_t)m->dev.N;
+    const size_t need = emp_grad_scratch_reserve(m, B);
     if (need > EMP_NOALLOC_SCRATCH_DOUBLES) {
         emp_set_error("batch of %lld vectors needs %zu doubles of scratch; the allocation-free entry point holds %zu",
                       (long long)B, need, (size_t)EMP_NOALLOC_SCRATCH_DOUBLES);

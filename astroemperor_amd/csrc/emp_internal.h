@@ -162,3 +162,4 @@ int emp_launch_grad_ws(const EmpModel* m, const double* d_theta, int64_t B, int6
 int emp_pick_grad_wpt(const EmpModel* m, int64_t B);
 // Doubles of scratch one adjoint launch over B vectors needs.
 size_t emp_grad_scratch_doubles(const EmpModel* m, int64_t B);
+size_t emp_grad_scratch_reserve(const EmpModel* m, int64_t B);
