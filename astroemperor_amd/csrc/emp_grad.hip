@@ -785,70 +785,59 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
 // Bound by VALU issue (104 to 112 instructions per planet-epoch against the
 // 205 of one epoch per lane with five sums per planet reduced in every tile;
 // the VALU issues in about 70% of the cycles).  Measured before and after:
-// 8192 vectors of 7 planets x 10^4 epochs, MA(1), mixed, 3.76 -> 2.46 ms; 16,384
-// of 5 planets x 2000 epochs, FP64 (with its table start), 1.16 -> 0.58 ms, a
-// third of that from grouping the epochs by instrument (emp_model_host).
+// 8192 vectors of 7 planets x 10^4 epochs, MA(1), mixed, 3.76 -> 2.36 ms; 16,384
+// of 5 planets x 2000 epochs, FP64 (with its table start), 1.16 -> 0.53 ms, a
+// good part of that from grouping the epochs by instrument (emp_model_host).
 // ---------------------------------------------------------------------------
+
+// The wave's sums in LDS of the terms that lanes add to as they go, in
+// 2^cl copies (lane mod 2^cl): 64 lanes adding to one address take the LDS some
+// 260 cycles, and the lanes of a wave often share an instrument.  `pairs` sums
+// with an R state each (offsets; the MA sets' coefficients, then their
+// timescales where these are free; acceleration), the totals first, then the R
+// states (only with the MA), then the jitters' sums, which have none.
+// Measured with one copy and with this: 8192 vectors of 1500 epochs and
+// 1 planet, 4 instruments, FP64, 177 -> 98 us, with MA(1) per instrument 239 -> 166;
+// 3 planets x 3000 epochs with MA(1) per instrument, mixed, 509 -> 424, with a
+// global one 485 -> 430.
+struct InsLayout {
+    int sets, pairs, rows;      // MA sets; sums with an R state; all rows (of 2^cl doubles) of one wave
+    __host__ __device__ explicit InsLayout(const ModelDev& md) {
+        sets = !md.ma_active ? 0 : md.ma_global ? 1 : md.I;
+        pairs = md.I + (md.ma_wfixed ? 1 : 2) * sets + md.acc;
+        rows = (md.ma_active ? 2 : 1) * pairs + md.I;
+    }
+    __host__ __device__ int mac(const ModelDev& md) const { return md.I; }
+    __host__ __device__ int mat(const ModelDev& md) const { return md.I + sets; }
+    __host__ __device__ int acc(const ModelDev& md) const { return pairs - md.acc; }
+    __host__ __device__ int jit(const ModelDev& md) const { return rows - md.I; }
+};
 
 // Per-lane sums of the per-instrument terms (offset, jitter, MA(1)
 // coefficient and timescale) of the lane's epochs, the offset and MA sums
-// with their R states; added to the wave's LDS totals and R states when the
+// with their R states; added to the wave's sums in LDS (InsLayout) when the
 // lane's instrument changes (the MA sums are keyed by instrument, or by 0 for
-// a global MA).
+// a global MA).  hasR: the wave has R states that are not all zero.
 struct InsAcc1 {
     int k = -1, km = -1;
     double off = 0.0, offR = 0.0, jit = 0.0, mac = 0.0, macR = 0.0, mat = 0.0, matR = 0.0;
-    template <int EXT>
-    __device__ __forceinline__ void flush_ins(double* tot, double* rst) {
-        using GW = GradWave<EXT>;
+    // copy: the lane's copy of the wave's first row
+    __device__ __forceinline__ void flush_ins(const ModelDev& md, const InsLayout& il, double* copy, int cl, bool hasR) {
         if (k < 0) return;
-        atomicAdd(&tot[GW::OFF + k], off);
-        atomicAdd(&rst[GW::OFF + k], offR);
-        atomicAdd(&tot[GW::JIT + k], jit);
+        atomicAdd(&copy[k << cl], off);
+        if (hasR) atomicAdd(&copy[(il.pairs + k) << cl], offR);
+        atomicAdd(&copy[(il.jit(md) + k) << cl], jit);
         off = offR = jit = 0.0;
     }
-    template <int EXT>
-    __device__ __forceinline__ void flush_ma(double* tot, double* rst) {
-        using GW = GradWave<EXT>;
+    __device__ __forceinline__ void flush_ma(const ModelDev& md, const InsLayout& il, double* copy, int cl, bool hasR) {
         if (km < 0) return;
-        atomicAdd(&tot[GW::MAC + km * GW::QM], mac);
-        atomicAdd(&rst[GW::MAC + km * GW::QM], macR);
-        atomicAdd(&tot[GW::MAT + km * GW::QM], mat);
-        atomicAdd(&rst[GW::MAT + km * GW::QM], matR);
+        atomicAdd(&copy[(il.mac(md) + km) << cl], mac);
+        if (hasR) atomicAdd(&copy[(il.pairs + il.mac(md) + km) << cl], macR);
+        if (!md.ma_wfixed) {
+            atomicAdd(&copy[(il.mat(md) + km) << cl], mat);
+            if (hasR) atomicAdd(&copy[(il.pairs + il.mat(md) + km) << cl], matR);
+        }
         mac = macR = mat = matR = 0.0;
-    }
-    // The end of the pass: the lanes that share an instrument are summed over
-    // the wave (in a fixed order) and added by one lane, one instrument after
-    // the other, instead of 64 atomics on the same few addresses.  Whole wave
-    // active.
-    template <int EXT>
-    __device__ __forceinline__ void flush_all(bool ma, double* tot, double* rst, int lane) {
-        using GW = GradWave<EXT>;
-        unsigned long long left = __ballot(k >= 0);
-        while (left) {
-            const int kk = __builtin_amdgcn_readlane(k, (int)__builtin_ctzll(left));
-            const bool in = k == kk;
-            const double so = wave_sum(in ? off : 0.0), sj = wave_sum(in ? jit : 0.0);
-            const double sr = ma ? wave_sum(in ? offR : 0.0) : 0.0;
-            if (lane == 0) {
-                tot[GW::OFF + kk] += so;
-                rst[GW::OFF + kk] += sr;
-                tot[GW::JIT + kk] += sj;
-            }
-            left &= ~__ballot(in);
-        }
-        if (!ma) return;
-        left = __ballot(km >= 0);
-        while (left) {
-            const int kk = __builtin_amdgcn_readlane(km, (int)__builtin_ctzll(left));
-            const bool in = km == kk;
-            const double sc = wave_sum(in ? mac : 0.0), st = wave_sum(in ? mat : 0.0);
-            if (lane == 0) {
-                tot[GW::MAC + kk * GW::QM] += sc;
-                tot[GW::MAT + kk * GW::QM] += st;
-            }
-            left &= ~__ballot(in);
-        }
     }
     // The move to the next tile, whose map is (tA, tB).
     __device__ __forceinline__ void move(double tA, double tB) {
@@ -859,14 +848,14 @@ struct InsAcc1 {
         macR *= tA;
         matR *= tA;
     }
-    template <int EXT>
-    __device__ __forceinline__ void to(int kk, int kkm, double* tot, double* rst) {
+    __device__ __forceinline__ void to(const ModelDev& md, const InsLayout& il, int kk, int kkm, double* copy, int cl,
+                                       bool ma, bool hasR) {
         if (kk != k) {
-            flush_ins<EXT>(tot, rst);
+            flush_ins(md, il, copy, cl, hasR);
             k = kk;
         }
-        if (kkm != km) {
-            flush_ma<EXT>(tot, rst);
+        if (ma && kkm != km) {
+            flush_ma(md, il, copy, cl, hasR);
             km = kkm;
         }
     }
@@ -876,10 +865,9 @@ struct InsAcc1 {
 // the compiler keeps those of all planets in registers over the tiles.
 __device__ __forceinline__ void reload_lds() { asm volatile("" ::: "memory"); }
 
-template <int EXT, int NW>
+template <int NW>
 struct Grad1LDS {
-    double rst[NW][GradWave<EXT>::N];    // R states of the per-instrument sums (per wave)
-    double natR[NW][WN_N];               // R states of the planet and acceleration sums (per wave)
+    double natR[NW][WN_ACC];             // R states of the planets' sums (per wave)
     double2 fwd[2][NW], suf[2][NW];      // per segment: its forward and suffix maps (double-buffered)
     double first[2][NW];                 // its first epoch's multiplier
 };
@@ -891,22 +879,23 @@ struct Grad1LDS {
 // time of periastron (model_tp), a template parameter so that no planet-epoch
 // branches on it.  `stale` as in k_lnl_grad.
 // Waves per SIMD that an instance is compiled for: as many as its registers
-// allow with little or no spilling (KM 4 / 6 / 8: 115 / 128 / 154 VGPRs without
-// the moving average; with it 128, 165 and 168, the last with 34 spilled, which
-// still beats 198 VGPRs at two waves per SIMD, 2.49 against 2.82 ms).
+// allow with little spilling (KM 4 / 6 / 8: 107 / 128 / 156 VGPRs without the
+// moving average; with it 128, 168 and 168, the first and the last with 22 and
+// 47 spilled, which still beats two waves per SIMD at KM 8, 2.49 against 2.82 ms).
 constexpr int GRAD1_FEW = 4;
 constexpr int grad1_occ(bool ma, int km) { return km <= 4 || (km <= 6 && !ma) ? 4 : 3; }
 template <int PREC, int EXT, bool MA, int NW, int KM, bool TP>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_occ(MA, KM)))) void k_lnl_grad1(
     ModelDev md, const double* __restrict__ theta, int64_t B, int64_t ld, double* __restrict__ out_lnl,
-    double* __restrict__ out_grad, unsigned long long* nonfinite, int* stale) {
+    double* __restrict__ out_grad, unsigned long long* nonfinite, int* stale, int cl) {
     constexpr int NT = 64 * NW, NE = 2, TILE1 = NT * NE;
     constexpr bool POST = EXT >= 1, tp = TP;
     using GW = GradWave<EXT>;
     __shared__ SlotLDSt<float4, KM> sl;
     __shared__ GradLDS gl;
     __shared__ GradWaveLDS<EXT, NW> s_gw;
-    __shared__ Grad1LDS<EXT, NW> s_g1;
+    __shared__ Grad1LDS<NW> s_g1;
+    extern __shared__ double s_ins[];   // [NW][rows << cl]: the sums of InsLayout
     __shared__ SinCosTab s_tab;
     __shared__ ScanLDS s_scan;
     const int wave = wave_uniform(threadIdx.x >> 6), lane = threadIdx.x & 63, g = threadIdx.x;
@@ -917,10 +906,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
     for (int j = g; j < KMAX * 5; j += NT) (&gl.nat[0][0])[j] = 0.0;
     double* wacc = s_gw.acc[wave];
     double* wnat = s_gw.nat[wave];
-    double* wrst = s_g1.rst[wave];
     double* wnatR = s_g1.natR[wave];
-    for (int j = lane; j < GW::N; j += 64) wacc[j] = wrst[j] = 0.0;
-    for (int j = lane; j < WN_N; j += 64) wnat[j] = wnatR[j] = 0.0;
+    const InsLayout il(md);
+    double* wins = s_ins + wave * (il.rows << cl);
+    double* copy = wins + (lane & ((1 << cl) - 1));
+    for (int j = lane; j < GW::N; j += 64) wacc[j] = 0.0;
+    for (int j = lane; j < WN_N; j += 64) wnat[j] = 0.0;
+    for (int j = lane; j < WN_ACC; j += 64) wnatR[j] = 0.0;
+    for (int j = lane; j < il.rows << cl; j += 64) wins[j] = 0.0;
     for (int j = g; j <= SC_N; j += NT) s_tab.v[j] = md.sctab[j];
     __syncthreads();
     if (wave == 0) slot_setup(md, sl, lane);
@@ -944,6 +937,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
     int pexp = 0;
     double carry = 0.0;                 // eps of the last epoch so far
     int parity = 0, rot = wave;         // rot: the tile's segment this wave takes
+    bool hasR = false;                  // the wave's R states are not all zero
     InsAcc1 ia;
     double tnx[NE];                     // the next tile's times, loaded a tile ahead
 #pragma unroll
@@ -1119,27 +1113,33 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
             // data can give): it reduces the B parts alone.  With |a| <= 1/3,
             // every wave of a tile but the last is such a wave.
             needA = __any(__builtin_fabs(wA[0]) > 0x1p-100 || __builtin_fabs(wA[1]) > 0x1p-100);
-            // the sums this wave already holds in LDS, and the lane's own,
-            // move to the next tile
-            for (int e = lane; e < GW::COS; e += 64) {
-                const double R0 = wrst[e];
-                wacc[e] = __builtin_fma(tB, R0, wacc[e]);
-                wrst[e] = tA * R0;
+            // The sums this wave already holds in LDS, and the lane's own, move
+            // to the next tile; a tile whose map's |A| is below 2^-100 (most
+            // are) leaves no R state, by the same measure.
+            if (hasR) {
+                hasR = __any(__builtin_fabs(tA) > 0x1p-100);
+                const double rA = hasR ? tA : 0.0;
+                for (int e = lane; e < il.pairs << cl; e += 64) {
+                    const double R0 = wins[(il.pairs << cl) + e];
+                    wins[e] = __builtin_fma(tB, R0, wins[e]);
+                    wins[(il.pairs << cl) + e] = rA * R0;
+                }
+                for (int e = lane; e < md.K * 5; e += 64) {
+                    const double R0 = wnatR[e];
+                    wnat[e] = __builtin_fma(tB, R0, wnat[e]);
+                    wnatR[e] = rA * R0;
+                }
+                ia.move(rA, tB);
             }
-            for (int e = lane; e < WN_N; e += 64) {
-                const double R0 = wnatR[e];
-                wnat[e] = __builtin_fma(tB, R0, wnat[e]);
-                wnatR[e] = tA * R0;
-            }
-            ia.move(tA, tB);
+            hasR = hasR || needA;
         }
         // The per-instrument sums of the lane's epochs.
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
             if (!valid[i]) continue;
-            ia.to<EXT>(k[i], md.ma_global ? 0 : k[i], wacc, wrst);
+            ia.to(md, il, k[i], md.ma_global ? 0 : k[i], copy, cl, ma, hasR);
             ia.off += wB[i];
-            ia.offR += wA[i];
+            if (needA) ia.offR += wA[i];
             if (md.has_jit) ia.jit = __builtin_fma(sl.jit[k[i]], ef[i] * ef[i] * ie[i] * ie[i] - ie[i], ia.jit);
             if (ma) {
                 // d a / d (c, tau) times the previous eps (none at a segment start)
@@ -1148,12 +1148,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
                     const double wgt = md.ma_wfixed ? dtc[i] : exp(-dtc[i] / sl.ma_tau[k[i]]);
                     const double hc = em[i] * wgt;                      // lambda = -w
                     ia.mac = __builtin_fma(wB[i], hc, ia.mac);
-                    ia.macR = __builtin_fma(wA[i], hc, ia.macR);
+                    if (needA) ia.macR = __builtin_fma(wA[i], hc, ia.macR);
                     if (!md.ma_wfixed) {
                         const double tau = sl.ma_tau[k[i]];
                         const double ht = hc * (sl.ma_c[k[i]] * dtc[i] / (tau * tau));
                         ia.mat = __builtin_fma(wB[i], ht, ia.mat);
-                        ia.matR = __builtin_fma(wA[i], ht, ia.matR);
+                        if (needA) ia.matR = __builtin_fma(wA[i], ht, ia.matR);
                     }
                 }
             }
@@ -1209,8 +1209,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
                     }
                 }
             }
-            wave_reduce_add4(b4, md.acc, wnat + WN_ACC, ri4);
-            if (needA) wave_reduce_add4(a4, md.acc, wnatR + WN_ACC, ri4);
+#pragma unroll
+            for (int q = 0; q < AMAX; ++q)
+                if (q < md.acc) {
+                    atomicAdd(&copy[(il.acc(md) + q) << cl], b4[q]);
+                    if (needA) atomicAdd(&copy[(il.pairs + il.acc(md) + q) << cl], a4[q]);
+                }
         }
         parity ^= 1;
     }
@@ -1226,7 +1230,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
             const double v4 = wave_sum(acc1[p]);
             if (lane == 0) wnat[5 * p + 4] += v4;
         }
-    ia.flush_all<EXT>(ma, wacc, wrst, lane);
+    // The copies of the wave's sums (R states have nothing left to meet).
+    ia.flush_ins(md, il, copy, cl, false);
+    ia.flush_ma(md, il, copy, cl, false);
+    wave_sync();
+    for (int r = lane; r < il.pairs + md.I; r += 64) {
+        const double* c = wins + ((r < il.pairs ? r : il.jit(md) + r - il.pairs) << cl);
+        double v = 0.0;
+        for (int q = 0; q < 1 << cl; ++q) v += c[q];
+        if (r >= il.pairs) wacc[GW::JIT + r - il.pairs] = v;
+        else if (r >= il.acc(md)) wnat[WN_ACC + r - il.acc(md)] = v;
+        else if (r >= md.I + il.sets) wacc[GW::MAT + (r - il.mat(md)) * GW::QM] = v;
+        else if (r >= md.I) wacc[GW::MAC + (r - md.I) * GW::QM] = v;
+        else wacc[GW::OFF + r] = v;
+    }
     double ldet = log(prod) + (double)pexp * LN2;
     chi = wave_sum(chi);
     ldet = wave_sum(ldet);
@@ -1268,6 +1285,9 @@ static void launch_grad_t(const ModelDev& md, const double* th, int64_t B, int64
 // 84 / 86 / 168 / 238 (7 planets with MA(1), mixed: 135 / 139 / 223 / 361
 // against 172 / 166 / 320 / 536).
 constexpr int GRAD1_NW = 2;
+// LDS for the copies of the waves' sums (InsLayout) that keeps the KM = 8
+// instances' 6 workgroups per CU (160 KB, 20 KB of each without the copies).
+constexpr size_t GRAD1_INS_BYTES = 5632;
 // Below this many epochs the default kernel is one that a caller may still
 // replace by the two-pass one after scratch was set aside for it: a batch whose
 // eps rows would not fit the allocation-free entry point's scratch is refused
@@ -1359,7 +1379,12 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
             }
             return EMP_OK;
         }
-#define EMP_CASE1(P, E, A, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, GRAD1_NW, M, T>), dim3((unsigned)B), dim3(64 * GRAD1_NW), 0, s, md, th, B, ld, lnl, grad, nf, stale)
+        // Eight copies of the wave's sums, fewer where many instruments would cost occupancy.
+        const int rows = GRAD1_NW * InsLayout(md).rows;
+        int cl = 3;
+        while (cl && (rows << cl) * sizeof(double) > GRAD1_INS_BYTES) --cl;
+        const size_t lds = (size_t)(rows << cl) * sizeof(double);
+#define EMP_CASE1(P, E, A, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, GRAD1_NW, M, T>), dim3((unsigned)B), dim3(64 * GRAD1_NW), lds, s, md, th, B, ld, lnl, grad, nf, stale, cl)
 #define EMP_CASE1M(P, E, A, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, GRAD1_FEW, T); else if (md.K <= 6) EMP_CASE1(P, E, A, 6, T); else EMP_CASE1(P, E, A, KMAX, T); }
 #define EMP_CASE1A(P, E, T) { if (md.ma_active) EMP_CASE1M(P, E, true, T) else EMP_CASE1M(P, E, false, T) }
 #define EMP_CASE1T(P, E) { if (model_tp(md)) EMP_CASE1A(P, E, true) else EMP_CASE1A(P, E, false) }
