@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include <hip/hip_ext.h>
@@ -630,10 +631,8 @@ __global__ __launch_bounds__(MOM_BLOCK) void k_pt_lnl_moments(PTDev pd, long lon
 constexpr uint32_t LG_TAG = 0x20000000u;
 constexpr uint32_t MOVE_TAG = 0x10000000u;
 constexpr int LG_BLOCK = 1024;
-constexpr int LG_CHUNK = 64;
-constexpr int LG_NP = MAXD * (MAXD + 1) / 2;
-constexpr int LG_PAIRS = (LG_NP + LG_BLOCK - 1) / LG_BLOCK;
-constexpr int LG_STAGE = (LG_CHUNK * MAXD + LG_BLOCK - 1) / LG_BLOCK;
+constexpr int LG_WAVES = LG_BLOCK / 64;
+constexpr int LG_PANEL = 4;          // columns per step of the factorisation
 constexpr double LG_RIDGE = 1e-6;
 
 __device__ __forceinline__ U4 lg_draw(const PTDev& pd, long long sweep, int half, int step, int t, int k, uint32_t r) {
@@ -660,34 +659,99 @@ __device__ __forceinline__ double lg_bcast(const double v[2], int k) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// (L^T g)_j for the two parameters j = lane, lane + 64 of this lane.
-__device__ inline void lg_lt_times(const double* L2, const double g[2], int D, int lane, double v[2]) {
-    v[0] = v[1] = 0.0;
-    for (int k = 0; k < D; ++k) {
-        const double gk = lg_bcast(g, k);
-        for (int h = 0; h < 2; ++h) {
-            const int j = lane + 64 * h;
-            if (j < D) v[h] = __builtin_fma(L2[(size_t)k * D + j], gk, v[h]);
+// v_j += sum_k M[k][j] x_k for the parameters j = lane, lane + 64 of this lane,
+// k in order.  The rows are loaded eight ahead: a row at a time the pass waits
+// for D loads one after the other (the proposals of 8 x 400 walkers of 45
+// parameters 34 -> 19 us).
+__device__ inline void lg_times(const double* M, const double x[2], int D, int lane, double v[2]) {
+    const int j0 = min(lane, D - 1), j1 = min(lane + 64, D - 1);
+    auto rows = [&](int k0, auto n) {
+        double a[decltype(n)::value], b[decltype(n)::value];
+#pragma unroll
+        for (int q = 0; q < n; ++q) {
+            a[q] = M[(size_t)(k0 + q) * D + j0];
+            b[q] = D > 64 ? M[(size_t)(k0 + q) * D + j1] : 0.0;
         }
-    }
+#pragma unroll
+        for (int q = 0; q < n; ++q) {
+            const double xk = lg_bcast(x, k0 + q);
+            v[0] = __builtin_fma(a[q], xk, v[0]);
+            if (D > 64) v[1] = __builtin_fma(b[q], xk, v[1]);
+        }
+    };
+    int k = 0;
+    for (; k + 8 <= D; k += 8) rows(k, std::integral_constant<int, 8>());
+    for (; k < D; ++k) rows(k, std::integral_constant<int, 1>());
+    if (lane >= D) v[0] = 0.0;
+    if (lane + 64 >= D) v[1] = 0.0;
+}
+
+// d <- L^-1 d for the parameters j = lane, lane + 64 of this lane by forward
+// substitution, one column (L1[k][j] = L_jk) at a time, the columns loaded eight
+// ahead.  The quotient by the diagonal is formed from its reciprocal and one
+// residual, as accurate as a division and off the serial chain but for three
+// operations.
+__device__ inline void lg_solve(const double* L1, int D, int lane, double d[2]) {
+    const int j0 = min(lane, D - 1), j1 = min(lane + 64, D - 1);
+    const double diag[2] = {L1[(size_t)j0 * D + j0], D > 64 ? L1[(size_t)j1 * D + j1] : 1.0};
+    const double inv[2] = {1.0 / diag[0], 1.0 / diag[1]};
+    auto cols = [&](int k0, auto n) {
+        double a[decltype(n)::value], b[decltype(n)::value];
+#pragma unroll
+        for (int q = 0; q < n; ++q) {
+            a[q] = L1[(size_t)(k0 + q) * D + j0];
+            b[q] = D > 64 ? L1[(size_t)(k0 + q) * D + j1] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < n; ++q) {
+            const int k = k0 + q;
+            const double dk = lg_bcast(d, k), lk = lg_bcast(diag, k), ik = lg_bcast(inv, k);
+            const double r0 = dk * ik, rk = __builtin_fma(__builtin_fma(-r0, lk, dk), ik, r0);
+            d[0] = lane == k ? rk : lane > k && lane < D ? __builtin_fma(-a[q], rk, d[0]) : d[0];
+            if (D > 64) d[1] = lane + 64 == k ? rk : lane + 64 > k && lane + 64 < D ? __builtin_fma(-b[q], rk, d[1]) : d[1];
+        }
+    };
+    int k = 0;
+    for (; k + 8 <= D; k += 8) cols(k, std::integral_constant<int, 8>());
+    for (; k < D; ++k) cols(k, std::integral_constant<int, 1>());
 }
 
 // Covariance of the complementary half at each temperature and its Cholesky
-// factor; one workgroup of 1024 threads per temperature.  The walkers are
-// staged through LDS in chunks (the next chunk's rows are loaded into
-// registers while the current one is summed); the covariance and its
-// factorisation stay in LDS as a packed lower triangle (row i starts at
-// i (i + 1) / 2).  Each thread owns the same entries in both phases.  The
-// factorisation is right-looking on the unscaled columns,
-// A_ik -= A_ij A_kj / A_jj for j < k <= i, with one barrier per column; the
-// columns are scaled by 1 / sqrt(A_jj) at the end.  Deterministic: every sum
-// runs in a fixed order.  Block 0 of the first half-step of the sweep also
-// counts the likelihoods of the current-position gradient launch.
+// factor; one workgroup of 16 waves per temperature.  The covariance is a
+// contraction over the walkers, on FP64 matrix instructions (16 x 16 tiles of
+// the lower triangle, four walkers each): a lane loads parameter 16 t + lane mod
+// 16 of walker lane / 16, which is the operand of a tile's rows and of its
+// columns alike, straight from the walkers' rows.  ND: column tiles.  Up to 64
+// parameters (ND <= 4) every wave takes all tiles for its share of the walkers;
+// beyond (ND = 6, 8), four waves share the tiles of each quarter of the walkers.
+// The waves' parts are added in a fixed order, so the factor is a function of
+// the positions alone.  The walkers are taken relative to the first of them, so
+// that a parameter without spread has a variance of exactly zero.
+// The factorisation stays in LDS as a packed lower triangle (row i starts at
+// i (i + 1) / 2): right-looking on the unscaled columns, A_ik -= A_ij A_kj / A_jj
+// for j < k <= i, four columns per step (each thread brings its rows' panel
+// entries up to date itself, so a step costs one round trip to LDS and two
+// barriers instead of four of each); the columns are scaled by 1 / sqrt(A_jj) at
+// the end.  Bound by latency: walker loads, the partial sums, D / 4 steps.
+// Measured against a thread per entry that read two LDS values per
+// multiply-add and a barrier per column: 16 x 1024 walkers of 50 parameters 103
+// -> 50 us, 8 x 400 of 45 49 -> 27 us, 5 x 100 of 9 17 -> 10 us.  (Panels of 16
+// columns by one wave with matrix updates of the rest gained nothing more.)
+// Block 0 of the first half-step of the sweep also counts the likelihoods of
+// the current-position gradient launch.
+typedef double lg_v4 __attribute__((ext_vector_type(4)));
+
+template <int ND>
 __global__ __launch_bounds__(LG_BLOCK) void k_lg_precond(PTDev pd, int half, int step) {
-    __shared__ double s_x[LG_CHUNK][MAXD];
-    __shared__ double s_a[LG_NP];
-    __shared__ double s_mean[MAXD], s_diag[MAXD];
+    constexpr int DP = 16 * ND, NP = DP * (DP + 1) / 2;
+    constexpr bool ALL = ND <= 4;                               // a wave takes every tile
+    constexpr int NT = ND * (ND + 1) / 2, WT = ALL ? NT : (NT + 3) / 4, BUF = ALL ? 4 : 1;
+    constexpr int PAIRS = (NP + LG_BLOCK - 1) / LG_BLOCK;
+    __shared__ double s_a[BUF][NP];
+    __shared__ double s_part[LG_WAVES][DP];
+    __shared__ double s_mean[DP], s_diag[DP];
     const int t = blockIdx.x, D = pd.D, W2 = pd.W2, tid = threadIdx.x;
+    const int wave = wave_uniform(tid >> 6), lane = tid & 63;
     const int* cmap = pd.map + t * pd.W + (1 - half) * W2;
     double* A = pd.lg_L2 + (size_t)t * D * D;
     double* L1 = pd.lg_L1 + (size_t)t * D * D;
@@ -695,80 +759,114 @@ __global__ __launch_bounds__(LG_BLOCK) void k_lg_precond(PTDev pd, int half, int
         atomicAdd((unsigned long long*)(pd.sweep + 1), (unsigned long long)pd.T * pd.W);
     const int np = D * (D + 1) / 2;
     // this thread's entries p = tid + m LG_BLOCK of the packed triangle, as i << 16 | j
-    int pij[LG_PAIRS];
+    int pij[PAIRS];
     {
         int i = 0, j = tid;
         while (j > i) { j -= i + 1; ++i; }
 #pragma unroll
-        for (int m = 0; m < LG_PAIRS; ++m) {
+        for (int m = 0; m < PAIRS; ++m) {
             pij[m] = i << 16 | j;
             j += LG_BLOCK;
             while (j > i) { j -= i + 1; ++i; }
         }
     }
-    double pre[LG_STAGE];
-    auto fetch = [&](int w0) {
-        const int nw = min(LG_CHUNK, W2 - w0);
-#pragma unroll
-        for (int r = 0; r < LG_STAGE; ++r) {
-            const int e = tid + r * LG_BLOCK;
-            if (e < nw * D) {
-                const int w = e / D, j = e - w * D;
-                pre[r] = pd.X[(size_t)cmap[w0 + w] * D + j];
-            }
+    const double* first = pd.X + (size_t)cmap[0] * D;
+    // mean: each wave sums every 16th walker, then the waves in order
+    {
+        const int c0 = min(lane, D - 1), c1 = min(lane + 64, D - 1);
+        const double f0 = first[c0], f1 = first[c1];
+        double m0 = 0.0, m1 = 0.0;
+#pragma unroll 4
+        for (int w = wave; w < W2; w += LG_WAVES) {
+            const double* row = pd.X + (size_t)cmap[w] * D;
+            m0 += row[c0] - f0;
+            if (!ALL) m1 += row[c1] - f1;
         }
-    };
-    auto stage = [&](int w0, bool centre) {
-        const int nw = min(LG_CHUNK, W2 - w0);
-#pragma unroll
-        for (int r = 0; r < LG_STAGE; ++r) {
-            const int e = tid + r * LG_BLOCK;
-            if (e < nw * D) {
-                const int w = e / D, j = e - w * D;
-                s_x[w][j] = centre ? pre[r] - s_mean[j] : pre[r];
-            }
+        if (lane < DP) s_part[wave][lane] = m0;
+        if (!ALL) s_part[wave][lane + 64] = m1;
+        __syncthreads();
+        if (tid < D) {
+            double sum = 0.0;
+            for (int w = 0; w < LG_WAVES; ++w) sum += s_part[w][tid];
+            s_mean[tid] = first[tid] + sum / (double)W2;
         }
-    };
-    // mean (thread j < D sums column j over the walkers in order)
-    double sum = 0.0;
-    fetch(0);
-    for (int w0 = 0; w0 < W2; w0 += LG_CHUNK) {
-        const int nw = min(LG_CHUNK, W2 - w0);
         __syncthreads();
-        stage(w0, false);
-        if (w0 + LG_CHUNK < W2) fetch(w0 + LG_CHUNK);
-        __syncthreads();
-        if (tid < D)
-            for (int w = 0; w < nw; ++w) sum += s_x[w][tid];
     }
-    if (tid < D) s_mean[tid] = sum / (double)W2;
     // lower triangle of the covariance
-    double acc[LG_PAIRS];
+    {
+        const int lc = lane & 15, kq = lane >> 4;
+        const int share = ALL ? wave : wave >> 2, nshare = ALL ? LG_WAVES : LG_WAVES / 4, g = ALL ? 0 : wave & 3;
+        constexpr int GS = ALL ? 1 : 4;
+        double mt[ND];
+        int col[ND];
 #pragma unroll
-    for (int m = 0; m < LG_PAIRS; ++m) acc[m] = 0.0;
-    fetch(0);
-    for (int w0 = 0; w0 < W2; w0 += LG_CHUNK) {
-        const int nw = min(LG_CHUNK, W2 - w0);
-        __syncthreads();
-        stage(w0, true);
-        if (w0 + LG_CHUNK < W2) fetch(w0 + LG_CHUNK);
-        __syncthreads();
+        for (int q = 0; q < ND; ++q) {
+            col[q] = min(16 * q + lc, D - 1);
+            mt[q] = s_mean[col[q]];
+        }
+        lg_v4 acc[WT];
 #pragma unroll
-        for (int m = 0; m < LG_PAIRS; ++m) {
-            if (tid + m * LG_BLOCK < np) {
-                const int i = pij[m] >> 16, j = pij[m] & 0xffff;
-                double a = acc[m];
-                for (int w = 0; w < nw; ++w) a = __builtin_fma(s_x[w][i], s_x[w][j], a);
-                acc[m] = a;
+        for (int m = 0; m < WT; ++m) acc[m] = lg_v4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+        for (int w0 = 4 * share; w0 < W2; w0 += 4 * nshare) {
+            const int w = w0 + kq;
+            const double* row = pd.X + (size_t)cmap[min(w, W2 - 1)] * D;
+            double x[ND];
+#pragma unroll
+            for (int q = 0; q < ND; ++q) {
+                const double v = row[col[q]] - mt[q];
+                x[q] = w < W2 && 16 * q + lc < D ? v : 0.0;
+            }
+            if (ALL) {
+#pragma unroll
+                for (int ti = 0; ti < ND; ++ti)
+#pragma unroll
+                    for (int tj = 0; tj <= ti; ++tj) {
+                        lg_v4& c = acc[ti * (ti + 1) / 2 + tj];
+                        c = __builtin_amdgcn_mfma_f64_16x16x4f64(x[ti], x[tj], c, 0, 0, 0);
+                    }
+            } else {
+                // the four waves of a share take a tile in turn
+#pragma unroll
+                for (int ti = 0; ti < ND; ++ti)
+#pragma unroll
+                    for (int tj = 0; tj <= ti; ++tj) {
+                        const int q = ti * (ti + 1) / 2 + tj;
+                        if ((q & 3) == g) acc[q >> 2] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[ti], x[tj], acc[q >> 2], 0, 0, 0);
+                    }
             }
         }
-    }
+        // the parts of waves 4 r .. 4 r + 3 in round r: four triangles (or four waves' tiles of one)
+        double* part = s_a[ALL ? wave & 3 : 0];
+        for (int r = 0; r < 4; ++r) {
+            if (wave >> 2 == r) {
 #pragma unroll
-    for (int m = 0; m < LG_PAIRS; ++m) {
+                for (int ti = 0; ti < ND; ++ti)
+#pragma unroll
+                    for (int tj = 0; tj <= ti; ++tj) {
+                        const int q = ti * (ti + 1) / 2 + tj;
+                        if (GS == 1 || (q & 3) == g) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {       // lane / 16 + 4 e, lane mod 16 of the tile
+                                const int i = 16 * ti + kq + 4 * e, j = 16 * tj + lc;
+                                const int p = i * (i + 1) / 2 + j;
+                                if (j <= i) part[p] = r ? part[p] + acc[q / GS][e] : acc[q / GS][e];
+                            }
+                        }
+                    }
+            }
+            __syncthreads();
+        }
+    }
+    double* sa = s_a[0];
+#pragma unroll
+    for (int m = 0; m < PAIRS; ++m) {
         const int p = tid + m * LG_BLOCK;
         if (p < np) {
-            const double c = acc[m] / (double)W2;
-            s_a[p] = c;
+            double c = sa[p];
+            for (int q = 1; q < BUF; ++q) c += s_a[q % BUF][p];
+            c /= (double)W2;
+            sa[p] = c;
             if ((pij[m] >> 16) == (pij[m] & 0xffff)) s_diag[pij[m] >> 16] = c;
         }
     }
@@ -780,30 +878,72 @@ __global__ __launch_bounds__(LG_BLOCK) void k_lg_precond(PTDev pd, int half, int
         pd.lg_act[t * D + i] = act ? 1 : 0;
         const int ri = i * (i + 1) / 2;
         if (act) {
-            s_a[ri + i] = s_diag[i] * (1.0 + LG_RIDGE);
+            sa[ri + i] = s_diag[i] * (1.0 + LG_RIDGE);
         } else {
-            for (int k = 0; k < i; ++k) s_a[ri + k] = 0.0;
-            for (int r = i + 1; r < D; ++r) s_a[r * (r + 1) / 2 + i] = 0.0;
-            s_a[ri + i] = 1.0;
+            for (int k = 0; k < i; ++k) sa[ri + k] = 0.0;
+            for (int r = i + 1; r < D; ++r) sa[r * (r + 1) / 2 + i] = 0.0;
+            sa[ri + i] = 1.0;
         }
     }
     bool fail = false;
-    for (int j = 0; j < D; ++j) {
+    for (int j0 = 0; j0 < D; j0 += LG_PANEL) {
         __syncthreads();
-        const double piv = s_a[j * (j + 1) / 2 + j];    // final since step j - 1; same value in every thread
-        if (!(piv > 0.0) || !(piv < __builtin_inf())) {
-            fail = true;
-            break;
-        }
-        const double inv = 1.0 / piv;
+        // the panel's own triangle, and 1 / pivot of its columns; the same in every thread
+        double pan[LG_PANEL][LG_PANEL], inv[LG_PANEL];
 #pragma unroll
-        for (int m = 0; m < LG_PAIRS; ++m) {
+        for (int r = 0; r < LG_PANEL; ++r)
+#pragma unroll
+            for (int q = 0; q <= r; ++q) {
+                const int i = min(j0 + r, D - 1);
+                pan[r][q] = sa[i * (i + 1) / 2 + j0 + q];       // past the last column: values that nothing uses
+            }
+#pragma unroll
+        for (int q = 0; q < LG_PANEL; ++q) {
+            const bool in = j0 + q < D;
+            const double piv = pan[q][q];
+            if (in && (!(piv > 0.0) || !(piv < __builtin_inf()))) fail = true;
+            inv[q] = 1.0 / piv;
+#pragma unroll
+            for (int r = q + 1; r < LG_PANEL; ++r)
+#pragma unroll
+                for (int c = q + 1; c <= r; ++c)
+                    pan[r][c] = __builtin_fma(-(pan[r][q] * inv[q]), pan[c][q], pan[r][c]);
+        }
+        if (fail) break;
+        double upd[PAIRS];
+#pragma unroll
+        for (int m = 0; m < PAIRS; ++m) {
             const int p = tid + m * LG_BLOCK;
             const int i = pij[m] >> 16, k = pij[m] & 0xffff;
-            if (p < np && k > j) {
-                const double lij = s_a[i * (i + 1) / 2 + j] * inv;
-                s_a[p] = __builtin_fma(-lij, s_a[k * (k + 1) / 2 + j], s_a[p]);
+            if (p < np && k > j0) {
+                const int last = np - 1;
+                double ai[LG_PANEL], ak[LG_PANEL], v = sa[p];
+#pragma unroll
+                for (int q = 0; q < LG_PANEL; ++q) {
+                    ai[q] = sa[min(i * (i + 1) / 2 + j0 + q, last)];
+                    ak[q] = sa[min(k * (k + 1) / 2 + j0 + q, last)];
+                }
+#pragma unroll
+                for (int q = 0; q < LG_PANEL; ++q) {
+                    if (j0 + q < k) {
+                        const double li = ai[q] * inv[q];
+                        v = __builtin_fma(-li, ak[q], v);
+                        const double lk = ak[q] * inv[q];
+#pragma unroll
+                        for (int r = q + 1; r < LG_PANEL; ++r) {
+                            ai[r] = __builtin_fma(-li, pan[r][q], ai[r]);
+                            ak[r] = __builtin_fma(-lk, pan[r][q], ak[r]);
+                        }
+                    }
+                }
+                upd[m] = v;
             }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < PAIRS; ++m) {
+            const int p = tid + m * LG_BLOCK;
+            if (p < np && (pij[m] & 0xffff) > j0) sa[p] = upd[m];
         }
     }
     __syncthreads();
@@ -813,12 +953,23 @@ __global__ __launch_bounds__(LG_BLOCK) void k_lg_precond(PTDev pd, int half, int
         if (fail) {
             if (i == k) v = s_diag[i] > 0.0 ? sqrt(s_diag[i]) : 1.0;
         } else if (k <= i) {
-            const double dk = sqrt(s_a[k * (k + 1) / 2 + k]);
-            v = i == k ? dk : s_a[i * (i + 1) / 2 + k] / dk;
+            const double dk = sqrt(sa[k * (k + 1) / 2 + k]);
+            v = i == k ? dk : sa[i * (i + 1) / 2 + k] / dk;
         }
         A[e] = v;
         L1[(size_t)k * D + i] = v;
     }
+}
+
+static void launch_precond(const PTDev& d, int half, int step, hipStream_t s) {
+#define EMP_PRE(N) hipLaunchKernelGGL(k_lg_precond<N>, dim3((unsigned)d.T), dim3(LG_BLOCK), 0, s, d, half, step)
+    if (d.D <= 16) EMP_PRE(1);
+    else if (d.D <= 32) EMP_PRE(2);
+    else if (d.D <= 48) EMP_PRE(3);
+    else if (d.D <= 64) EMP_PRE(4);
+    else if (d.D <= 96) EMP_PRE(6);
+    else EMP_PRE(8);
+#undef EMP_PRE
 }
 
 // Proposal of every walker of the moving half (one wave per walker), its
@@ -851,7 +1002,7 @@ __global__ __launch_bounds__(PRIOR_BLOCK) void k_lg_propose(ModelDev md, PTDev p
     }
     const bool drift = __ballot(!fin) == 0ull;
     double v[2] = {0.0, 0.0};
-    if (drift) lg_lt_times(L2, gv, D, lane, v);
+    if (drift) lg_times(L2, gv, D, lane, v);        // L^T g
     double u[2] = {0.0, 0.0}, lq = 0.0;
     for (int h = 0; h < 2; ++h) {
         const int j = lane + 64 * h;
@@ -863,13 +1014,7 @@ __global__ __launch_bounds__(PRIOR_BLOCK) void k_lg_propose(ModelDev md, PTDev p
     }
     lq = wave_sum(lq);
     double dy[2] = {0.0, 0.0};
-    for (int kk = 0; kk < D; ++kk) {
-        const double uk = lg_bcast(u, kk);
-        for (int h = 0; h < 2; ++h) {
-            const int j = lane + 64 * h;
-            if (j < D) dy[h] = __builtin_fma(L1[(size_t)kk * D + j], uk, dy[h]);
-        }
-    }
+    lg_times(L1, u, D, lane, dy);                   // L u
     double y[2];
     for (int h = 0; h < 2; ++h) {
         const int j = lane + 64 * h;
@@ -921,16 +1066,8 @@ __global__ __launch_bounds__(PRIOR_BLOCK) void k_lg_accept(PTDev pd, int half, i
     }
     const bool drift = __ballot(!fin) == 0ull;
     double v[2] = {0.0, 0.0};
-    if (drift) lg_lt_times(L2, gv, D, lane, v);
-    // r = L^-1 (x - y) by forward substitution, one column at a time
-    for (int kk = 0; kk < D; ++kk) {
-        const double rk = lg_bcast(dv, kk) / L1[(size_t)kk * D + kk];
-        for (int h = 0; h < 2; ++h) {
-            const int j = lane + 64 * h;
-            if (j == kk) dv[h] = rk;
-            else if (j > kk && j < D) dv[h] = __builtin_fma(-L1[(size_t)kk * D + j], rk, dv[h]);
-        }
-    }
+    if (drift) lg_times(L2, gv, D, lane, v);        // L^T g
+    lg_solve(L1, D, lane, dv);                      // r = L^-1 (x - y)
     // reverse proposal: xi' = r / eps - (eps / 2) beta L^T g(y)
     const double eps = pd.lg_eps[t];
     double lq = 0.0;
@@ -1116,7 +1253,7 @@ static int launch_grad_sweep(EmpPT* p, hipEvent_t* ev = nullptr) {
     for (int st = 0; st < p->desc.nsteps; ++st)
         for (int h = 0; h < 2; ++h) {
             if (h == 0 && st > 0 && (rc = launch_record(p, 2, st))) return rc;
-            hipLaunchKernelGGL(k_lg_precond, dim3((unsigned)d.T), dim3(LG_BLOCK), 0, p->stream, d, h, st);
+            launch_precond(d, h, st, p->stream);
             EMP_HIP(hipGetLastError());
             hipLaunchKernelGGL(k_lg_propose, dim3(tgrid), dim3(PRIOR_BLOCK), 0, p->stream, md, d, h, st);
             EMP_HIP(hipGetLastError());
