@@ -326,14 +326,18 @@ __global__ static void k_gather_rows(const double* __restrict__ src, const int* 
 constexpr size_t GATHER_MOST = (size_t)4 << 20;      // doubles
 inline int emp_gather_rows(const double* src, const int* map, long long n, int per, int width, double** buf,
                            size_t* cap, hipStream_t s, double* host) {
-    const long long piece = std::max<long long>(1, std::min<long long>(n, (long long)(GATHER_MOST / width)));
-    const size_t need = (size_t)piece * width;
-    if (*cap < need) {
+    long long piece = std::max<long long>(1, std::min<long long>(n, (long long)(GATHER_MOST / width)));
+    if (*cap < (size_t)piece * width) {
         if (*buf) (void)hipFree(*buf);
         *buf = nullptr;
         *cap = 0;
-        EMP_HIP(hipMalloc((void**)buf, need * sizeof(double)));
-        *cap = need;
+        hipError_t e;       // smaller pieces where the device's memory is nearly full
+        while ((e = hipMalloc((void**)buf, (size_t)piece * width * sizeof(double))) == hipErrorOutOfMemory && piece > 1) {
+            (void)hipGetLastError();
+            piece = (piece + 1) / 2;
+        }
+        EMP_HIP(e);
+        *cap = (size_t)piece * width;
     }
     for (long long w0 = 0; w0 < n; w0 += piece) {
         const long long m = std::min(piece, n - w0), total = m * width;
