@@ -174,7 +174,7 @@ struct PlanetC {
     double bq, ibq;  // sqrt(1 - e^2) and its reciprocal (for gradients)
     int tp_mode;
     int bad;         // NaN-producing parameter set (reference would give NaN)
-    int ktab;        // mixed path: this planet's per-vector Kepler table is built and used
+    int ktab;        // this planet's per-vector Kepler table is built and used
 };
 
 // Builds PlanetC from the 5 block parameters, following the reference's

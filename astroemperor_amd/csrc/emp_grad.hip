@@ -782,9 +782,10 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
 // random walk).  The waves take the tile's segments in turn (rotated by one
 // every tile), so that this work falls on every SIMD alike.
 //
-// Bound by VALU issue (104 to 112 instructions per planet-epoch against the
-// 205 of one epoch per lane with five sums per planet reduced in every tile;
-// the VALU issues in about 70% of the cycles).  Measured before and after:
+// Bound by VALU issue (7 planets, MA(1): 126 instructions per planet-epoch mixed
+// and 137 FP64, the epochs' share included, against the 205 and 263 of one epoch
+// per lane with five sums per planet reduced in every tile; the VALU issues in
+// about 70% of the cycles).  Measured before and after:
 // 8192 vectors of 7 planets x 10^4 epochs, MA(1), mixed, 3.76 -> 2.36 ms; 16,384
 // of 5 planets x 2000 epochs, FP64 (with its table start), 1.16 -> 0.53 ms, a
 // good part of that from grouping the epochs by instrument (emp_model_host).
@@ -875,9 +876,9 @@ struct Grad1LDS {
 // Single-pass adjoint (above).  EXT: 0 plain models, 1 with the terms added
 // after the MA.  MA: the model may have a moving average.  NW waves per
 // workgroup (one vector), tiles of 128 NW epochs.  KM: the instance holds up to
-// KM planets' values and sums in registers (8 and 4 VGPRs per planet).  TP: the model's planets are parameterised by the
-// time of periastron (model_tp), a template parameter so that no planet-epoch
-// branches on it.  `stale` as in k_lnl_grad.
+// KM planets' values and sums in registers (8 and 4 VGPRs per planet).  TP: the
+// model's planets are parameterised by the time of periastron (model_tp), a
+// template parameter so that no planet-epoch branches on it.  `stale` as in k_lnl_grad.
 // Waves per SIMD that an instance is compiled for: as many as its registers
 // allow with little spilling (KM 4 / 6 / 8: 107 / 128 / 156 VGPRs without the
 // moving average; with it 128, 168 and 168, the first and the last with 22 and
@@ -1346,7 +1347,7 @@ static int ensure_grad_scratch(EmpModel* m, int64_t B) {
     return EMP_OK;
 }
 
-// Waves per vector of the adjoint kernel for a batch of B.  Four by default:
+// Waves per vector of the two-pass kernel for a batch of B.  Four by default:
 // with one or two waves per vector a workgroup holds four or eight slots of
 // LDS and the kernel's registers allow three or four waves per SIMD, with
 // four both allow four to six (measured on 8192 vectors of 7 planets x 10^4

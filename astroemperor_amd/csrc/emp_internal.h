@@ -16,10 +16,10 @@ constexpr int IMAX = 16;         // instruments per model
 constexpr int AMAX = 4;          // acceleration order
 constexpr int CMAX = 3;          // cosine terms per model (a sinusoid, a magnetic cycle's two)
 constexpr int SAIMAX = 32;       // stellar-activity columns per model
-constexpr int BLOCK = 512;       // threads per workgroup (8 waves)
+constexpr int BLOCK = 512;       // threads per workgroup (8 waves) of the two-pass adjoint and the model dump
 constexpr int NWAVES = BLOCK / 64;
 constexpr int MAX_WAVES = 16;    // largest workgroup any kernel launches (1024 threads)
-constexpr int TILE = 512;        // epochs staged in LDS per tile
+constexpr int TILE = 512;        // epochs that the two-pass adjoint stages in LDS per tile
 // Prior sequence entries: j >= 0 the prior of (free) full parameter j;
 // PSEQ_ECC - b the derived eccentricity prior of Keplerian block b;
 // PSEQ_CHECK: return -inf if the sum is -inf (the end of a block's own terms).
@@ -160,6 +160,7 @@ int emp_launch_grad_ws(const EmpModel* m, const double* d_theta, int64_t B, int6
                        double* d_grad, double* eps_scratch, hipStream_t s, int precision = EMP_FP64,
                        int* stale = nullptr, int wpt = 0);
 int emp_pick_grad_wpt(const EmpModel* m, int64_t B);
-// Doubles of scratch one adjoint launch over B vectors needs.
+// Doubles of scratch one adjoint launch over B vectors needs, and those to set
+// aside for it where the kernel may be switched afterwards.
 size_t emp_grad_scratch_doubles(const EmpModel* m, int64_t B);
 size_t emp_grad_scratch_reserve(const EmpModel* m, int64_t B);

@@ -14,11 +14,11 @@ namespace emp {
 
 constexpr double LN2 = 0.69314718055994530942;
 
-// Prior of one full parameter vector, sequentially and in the reference's
-// order so that the sum is bit-identical to the generated my_prior
-// (emp/emp.py:182-254): per block, add each free parameter's prior, return
-// -inf as soon as a block leaves the sum at -inf, then add the block's
-// derived eccentricity prior.
+// One prior term at x, by the reference's templates (support/priors/*.prior).
+// The sums of terms run in the order of the generated my_prior
+// (emp/emp.py:182-254), so that they are bit-identical to it: per block, add
+// each free parameter's prior, return -inf as soon as a block leaves the sum at
+// -inf, then add the block's derived eccentricity prior.
 __device__ inline double prior_term(const EmpPriorTerm& p, double x) {
 #pragma clang fp contract(off)
     if (!(x >= p.lo && x <= p.hi)) return -__builtin_inf();

@@ -5,7 +5,7 @@ the star's ``my_likelihood``/``my_prior`` (emp/emp.py:576-593) and runs
 ``run_mcmc`` (support/endit_reddemcee.scr:3).  A survey of S stars is S such
 runs.  :class:`SystemsPT` runs all of them at once on the device: S models
 (any mix of epochs, instruments, planets and free parameters) with the same
-T x W ensemble shape, one kernel launch per sweep for the whole batch.
+T x W ensemble shape, each pass of a sweep one kernel launch for the whole batch.
 
 Per system the moves are those of :class:`~astroemperor_amd.sampler.PTSampler`
 (stretch halves, hottest-first adjacent swaps, ladder adaptation in every mode),

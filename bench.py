@@ -38,9 +38,11 @@ METRIC = "PT sweeps/s + lnL evals/s, FP32-mixed vs FP64 on 1 GPU at |ΔlnL|<1e-6
 #                      (two sin/cos pairs, one reciprocal)
 #   per epoch        : 6 arithmetic + 2 elementary (reciprocal, log)
 #   per MA epoch     : 3 arithmetic + 1 elementary (exp)
-# FP64 path: everything at FP64 rates.  Mixed path: the 24 arithmetic and 4
-# of the 5 elementary ops of the Kepler term at FP32 rates, the rest FP64.
-OPS_KEP = {"fp64": 24 + 3 + 20 * 5, "mixed": 24 * 0.5 + 3 + 4 * 4 + 20 * 1}
+# Both paths start Kepler's equation from FP32: 4 of the 5 elementary ops at
+# FP32 rates.  FP64 path: the 24 arithmetic at FP64 rates; mixed path: at FP32
+# rates; the rest FP64.  (While the FP64 path's start was FP64 throughout, all 5
+# were priced at FP64 rates there, 127 ops.)
+OPS_KEP = {"fp64": 24 + 3 + 4 * 4 + 20 * 1, "mixed": 24 * 0.5 + 3 + 4 * 4 + 20 * 1}
 OPS_EPOCH = 6 + 20 * 2
 OPS_MA = 3 + 20 * 1
 # The adjoint (lnL and its gradient) of one vector: the value above once,
@@ -58,16 +60,16 @@ PEAK_FP64_TFLOPS = 78.6       # MI355X FP64 vector, FMA = 2 flops
 # each scaled by what the same counter reads for a plain 256 MiB device copy
 # (FETCH_SIZE 131,084 KiB: factor 2.00; WRITE_SIZE 262,144 KiB: 1.00).  Keys:
 # (workload, kernel, precision); values (FETCH_SIZE, WRITE_SIZE).  Source:
-# profiles/hbm_traffic_k_pt_half_k_lnl_grad1_k_sys_sweep.md.
+# profiles/hbm_traffic_half_step_adjoint_systems.md.
 TRAFFIC_KIB = {
-    ("c5", "k_pt_half", "mixed"): (3371.8, 1457.1),       # k_pt_half<1, 4>, 8192 proposals
-    ("c5", "k_pt_half", "fp64"): (3894.2, 1334.2),        # k_pt_half<0, 8>
-    ("c5", "k_lnl_grad", "mixed"): (4968.9, 6669.2),      # k_lnl_grad1<1, 0, 4, false>, 8192 vectors
-    ("c5", "k_lnl_grad", "fp64"): (5035.4, 6670.8),       # k_lnl_grad1<0, 0, 4, false>
-    ("c2", "k_pt_half", "mixed"): (593.6, 84.5),          # k_pt_half<1, 8>, 1280 proposals
-    ("c2", "k_pt_half", "fp64"): (585.6, 84.5),           # k_pt_half<0, 8>
-    ("c3", "k_sys_sweep", "mixed"): (193728.0, 139875.8),  # k_sys_sweep<1, 1, 16>, 4096 systems
-    ("c3", "k_sys_sweep", "fp64"): (194613.8, 135634.8),   # k_sys_sweep<0, 1, 16>
+    ("c5", "k_pt_half", "mixed"): (4201.5, 1471.4),       # k_pt_half<1, 4, 0>, 8192 proposals
+    ("c5", "k_pt_half", "fp64"): (4224.9, 1471.4),        # k_pt_half<0, 4, 0>
+    ("c5", "k_lnl_grad", "mixed"): (10389.6, 94609.6),    # k_lnl_grad1<1, 0, true, 2, 8, false>, 8192 vectors
+    ("c5", "k_lnl_grad", "fp64"): (10472.4, 95612.1),     # k_lnl_grad1<0, 0, true, 2, 8, false>
+    ("c2", "k_pt_step", "mixed"): (1199.0, 471.4),        # k_pt_step<1, 4, 0>, 1280 proposals
+    ("c2", "k_pt_step", "fp64"): (1208.7, 481.4),         # k_pt_step<0, 4, 0>
+    ("c3", "k_sys sweep", "mixed"): (975874.0, 163064.8),  # 2 k_sys_prior, 2 k_sys_lik<1, 1>, k_sys_swap, 4096 systems
+    ("c3", "k_sys sweep", "fp64"): (976013.6, 163037.0),   # the same with k_sys_lik<0, 1>
 }
 FETCH_SCALE, WRITE_SCALE = 2.00, 1.00
 
@@ -287,7 +289,7 @@ def run_c2(seed, steps, warmup, half_launches=40):
                      "lnl_evaluated_per_s": round((n1 - n0) / wall, 1),
                      "in_support_fraction": round((n1 - n0) / (steps * T * W * nsteps), 4),
                      "waves_per_walker": wpt,
-                     "roofline": roofline("k_pt_half", prec, flops_per_theta(m, prec) * ev, ms_half,
+                     "roofline": roofline("k_pt_step", prec, flops_per_theta(m, prec) * ev, ms_half,
                                           {"lnl_evaluated_per_launch": round(ev, 1),
                                            "proposals_per_launch": T * W // 2}, "c2")}
         if prec == "mixed":
@@ -303,7 +305,7 @@ def run_c2(seed, steps, warmup, half_launches=40):
 
 def run_systems(n_systems, steps, warmup, seed, precisions=("mixed", "fp64"), trial_sweeps=2):
     """Batched uneven systems (synth.c3): every system's own 8 x 64 PT
-    ensemble advanced by one persistent kernel launch per sweep, replayed
+    ensemble advanced by the same prior, likelihood and swap launches, replayed
     from a hipGraph, launch shape from the autotuner."""
     from astroemperor_amd import SystemsPT, synth
     from oracle.emp_oracle import OracleModel
@@ -345,7 +347,7 @@ def run_systems(n_systems, steps, warmup, seed, precisions=("mixed", "fp64"), tr
                      "ms_per_sweep_events": round(ev_ms, 4),
                      "lnl_evals_per_s": round(props / wall, 1), "lnl_evaluated_per_s": round((n1 - n0) / wall, 1),
                      "in_support_fraction": round(frac_eval, 4), "tuning": tune, "create_s": round(create_s, 2),
-                     "roofline": roofline("k_sys_sweep", prec, flops, ev_ms, None, "c3")}
+                     "roofline": roofline("k_sys sweep", prec, flops, ev_ms, None, "c3")}
         print(f"[bench] systems {prec}: {steps / wall:.2f} sweeps/s ({props / wall / 1e6:.1f} M lnL/s), "
               f"tuning {tune}", file=sys.stderr, flush=True)
         states[prec] = s
