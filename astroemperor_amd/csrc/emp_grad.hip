@@ -171,24 +171,23 @@ __device__ __forceinline__ void wave_reduce_add4(const double (&v)[4], int n, do
 }
 
 // Adds w = dlnL/dS_n times the derivatives of the terms added after the MA
-// at epoch n (time t, instrument k).
+// at epoch n (time t, instrument k): entry e of the cosine terms' sums, then of
+// the activity coefficients' (from 3 CMAX on) at acc[e << cl].
 template <int EXT, class SL>
 __device__ __forceinline__ void post_accumulate(const ModelDev& md, const SL& sl, const SinCosTab& tab, double t,
-                                                int n, int k, double w, double* wacc) {
-    using GW = GradWave<EXT>;
+                                                int n, int k, double w, double* acc, int cl) {
     if (md.sai_w) {
         const int b0 = md.sai_base[k], nc = md.sai_base[k + 1] - b0;
-        for (int c = 0; c < nc; ++c) atomicAdd(&wacc[GW::SAI + b0 + c], w * md.sai[(size_t)c * md.N + n]);
+        for (int c = 0; c < nc; ++c) atomicAdd(&acc[(3 * CMAX + b0 + c) << cl], w * md.sai[(size_t)c * md.N + n]);
     }
-    double* acc = wacc + GW::COS;
     for (int c = 0; c < md.n_cos; ++c) {
         const double r = reduce_2pi(cos_phase(sl, c, t));
         double sn, cs;
         sincos_tab(tab, __builtin_fabs(r), sn, cs);
         const double dph = -sl.cosw[c][0] * (r < 0.0 ? -sn : sn);
-        atomicAdd(&acc[3 * c + 0], w * cs);
-        atomicAdd(&acc[3 * c + 1], w * dph);
-        atomicAdd(&acc[3 * c + 2], w * dph * t);
+        atomicAdd(&acc[(3 * c + 0) << cl], w * cs);
+        atomicAdd(&acc[(3 * c + 1) << cl], w * dph);
+        atomicAdd(&acc[(3 * c + 2) << cl], w * dph * t);
     }
 }
 
@@ -409,7 +408,7 @@ __device__ __forceinline__ double ma_chunk_w(const ModelDev& md, const SL& sl, c
     ia.to<EXT>(k, wacc);
     ia.off += w;
     if (md.has_jit) ia.jit = __builtin_fma(sl.jit[k], ef * ef * ie * ie - ie, ia.jit);
-    if (POST && has_post(md)) post_accumulate<EXT>(md, sl, tl.tab, t, tb + j, k, -u, wacc);
+    if (POST && has_post(md)) post_accumulate<EXT>(md, sl, tl.tab, t, tb + j, k, -u, wacc + GradWave<EXT>::COS, 0);
     if (maq) {
         // d a_{n,c} / d phi_c = -exp(-dt / tau_c), d a_{n,c} / d tau_c = a_{n,c} dt / tau_c^2
         const int n = tb + j, set = md.ma_global ? 0 : k;
@@ -478,7 +477,7 @@ __device__ __forceinline__ double plain_w(const ModelDev& md, const SL& sl, cons
     ia.to<EXT>(k, wacc);
     ia.off += w;
     if (md.has_jit) ia.jit = __builtin_fma(sl.jit[k], w * w - ie, ia.jit);
-    if (POST && has_post(md)) post_accumulate<EXT>(md, sl, tl.tab, t, tb + j, k, w, wacc);
+    if (POST && has_post(md)) post_accumulate<EXT>(md, sl, tl.tab, t, tb + j, k, w, wacc + GradWave<EXT>::COS, 0);
     return w;
 }
 
@@ -796,22 +795,27 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
 // 260 cycles, and the lanes of a wave often share an instrument.  `pairs` sums
 // with an R state each (offsets; the MA sets' coefficients, then their
 // timescales where these are free; acceleration), the totals first, then the R
-// states (only with the MA), then the jitters' sums, which have none.
+// states (only with the MA), then the sums that have none: the jitters' and, in
+// the order of GradWave, those of the terms after the MA.
 // Measured with one copy and with this: 8192 vectors of 1500 epochs and
 // 1 planet, 4 instruments, FP64, 177 -> 98 us, with MA(1) per instrument 239 -> 166;
 // 3 planets x 3000 epochs with MA(1) per instrument, mixed, 509 -> 424, with a
-// global one 485 -> 430.
+// global one 485 -> 430; with a sinusoid, whose sums every epoch of every lane
+// adds to, 1 planet x 1500 epochs 561 -> 135, 5 x 3000 1365 -> 593.
 struct InsLayout {
     int sets, pairs, rows;      // MA sets; sums with an R state; all rows (of 2^cl doubles) of one wave
-    __host__ __device__ explicit InsLayout(const ModelDev& md) {
+    int npost;                  // rows of the terms after the MA
+    __host__ __device__ InsLayout(const ModelDev& md, bool has_post) {
+        npost = !has_post ? 0 : 3 * CMAX + (md.sai_w ? SAIMAX : 0);
         sets = !md.ma_active ? 0 : md.ma_global ? 1 : md.I;
         pairs = md.I + (md.ma_wfixed ? 1 : 2) * sets + md.acc;
-        rows = (md.ma_active ? 2 : 1) * pairs + md.I;
+        rows = (md.ma_active ? 2 : 1) * pairs + md.I + npost;
     }
     __host__ __device__ int mac(const ModelDev& md) const { return md.I; }
     __host__ __device__ int mat(const ModelDev& md) const { return md.I + sets; }
     __host__ __device__ int acc(const ModelDev& md) const { return pairs - md.acc; }
-    __host__ __device__ int jit(const ModelDev& md) const { return rows - md.I; }
+    __host__ __device__ int post() const { return rows - npost; }
+    __host__ __device__ int jit(const ModelDev& md) const { return post() - md.I; }
 };
 
 // Per-lane sums of the per-instrument terms (offset, jitter, MA(1)
@@ -908,7 +912,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
     double* wacc = s_gw.acc[wave];
     double* wnat = s_gw.nat[wave];
     double* wnatR = s_g1.natR[wave];
-    const InsLayout il(md);
+    const InsLayout il(md, POST && has_post(md));
     double* wins = s_ins + wave * (il.rows << cl);
     double* copy = wins + (lane & ((1 << cl) - 1));
     for (int j = lane; j < GW::N; j += 64) wacc[j] = 0.0;
@@ -1063,7 +1067,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
                 pexp += __builtin_amdgcn_frexp_exp(prod);
                 prod = __builtin_amdgcn_frexp_mant(prod);
                 if (POST && has_post(md))
-                    post_accumulate<EXT>(md, sl, s_tab, t[i], n0 + i, k[i], ef[i] * ie[i], wacc);
+                    post_accumulate<EXT>(md, sl, s_tab, t[i], n0 + i, k[i], ef[i] * ie[i],
+                                         copy + (il.post() << cl), cl);
             }
         }
         // dlnL/dmu = wB + wA Lambda; lambda = lB + lA Lambda; (tA, tB) the tile's map.
@@ -1235,11 +1240,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
     ia.flush_ins(md, il, copy, cl, false);
     ia.flush_ma(md, il, copy, cl, false);
     wave_sync();
-    for (int r = lane; r < il.pairs + md.I; r += 64) {
+    const int nsum = il.pairs + md.I + il.npost;
+    for (int r = lane; r < nsum; r += 64) {
         const double* c = wins + ((r < il.pairs ? r : il.jit(md) + r - il.pairs) << cl);
         double v = 0.0;
         for (int q = 0; q < 1 << cl; ++q) v += c[q];
-        if (r >= il.pairs) wacc[GW::JIT + r - il.pairs] = v;
+        if (POST && r >= il.pairs + md.I) wacc[GW::COS + r - il.pairs - md.I] = v;
+        else if (r >= il.pairs) wacc[GW::JIT + r - il.pairs] = v;
         else if (r >= il.acc(md)) wnat[WN_ACC + r - il.acc(md)] = v;
         else if (r >= md.I + il.sets) wacc[GW::MAT + (r - il.mat(md)) * GW::QM] = v;
         else if (r >= md.I) wacc[GW::MAC + (r - md.I) * GW::QM] = v;
@@ -1381,7 +1388,7 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
             return EMP_OK;
         }
         // Eight copies of the wave's sums, fewer where many instruments would cost occupancy.
-        const int rows = GRAD1_NW * InsLayout(md).rows;
+        const int rows = GRAD1_NW * InsLayout(md, has_post(md)).rows;
         int cl = 3;
         while (cl && (rows << cl) * sizeof(double) > GRAD1_INS_BYTES) --cl;
         const size_t lds = (size_t)(rows << cl) * sizeof(double);
