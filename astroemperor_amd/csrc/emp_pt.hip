@@ -783,7 +783,7 @@ __global__ __launch_bounds__(LG_BLOCK) void k_lg_precond(PTDev pd, int half, int
             if (!ALL) m1 += row[c1] - f1;
         }
         if (lane < DP) s_part[wave][lane] = m0;
-        if (!ALL) s_part[wave][lane + 64] = m1;
+        if (!ALL && lane + 64 < DP) s_part[wave][lane + 64] = m1;      // rows of DP sums: 96 or 128
         __syncthreads();
         if (tid < D) {
             double sum = 0.0;
