@@ -303,16 +303,15 @@ __device__ __forceinline__ void sincos_tab_f(const SinCosTab& tb, float Ef, doub
 }
 
 // x^(2/3) for x >= 0 to FP32 accuracy (hardware log2 / exp2, ~3e-7
-// relative): the Markley starter's cube root (see kepler_fp64_E).
+// relative): the Markley starter's cube root (see kepler_fp64).
 __device__ __forceinline__ double pow23_start(double x) {
     const float xf = (float)x;
     return xf > 0.0f ? (double)__builtin_amdgcn_exp2f(0.6666667f * __builtin_amdgcn_logf(xf)) : 0.0;
 }
 
 // ----------------------------------------------------------------------------
-// FP64 Kepler solve without a table (Markley 1995; PREC 0 above KT_EMAX or for
-// short series, see planet_sc).  Input: M reduced to [-pi, pi].  Output:
-// sin E, cos E.
+// FP64 Kepler solve without a table (Markley 1995; PREC 0 where planet_slot sets
+// no table).  Input: M reduced to [-pi, pi].  Output: sin E, cos E.
 // ----------------------------------------------------------------------------
 __device__ __forceinline__ void kepler_fp64(double M, const PlanetC& pc, const SinCosTab& tb, double& sE,
                                             double& cE) {
@@ -386,6 +385,11 @@ constexpr double KT_H = PI_D / (KT_N - 1);
 constexpr double KT_ENEWTON = 0.5;
 constexpr double KT_EH64 = 0.75;
 constexpr double KT_EMAX = 0.95;
+// Largest mean anomaly (before its reduction) of a planet with a table.
+// reduce_2pi leaves |M| up to 1.2e-16 of it above pi, here 5e-7 rad; a start is
+// in the sin/cos table's range up to 6.1e-3 rad beyond [0, pi].  (From 1e16 on
+// the reduced M is any number.)
+constexpr double KT_MMAX = 4294967296.0;
 // A planet's Kepler path on the mixed path, as flags: the start from the
 // table (else the FP32 Markley starter), an FP32 Halley step after it, and
 // an FP64 Halley step (else an FP64 Newton step).  Markley: H32 | H64;

@@ -69,6 +69,7 @@ struct ModelDev {
     const double2* sctab;             // [SC_N + 1] (sin, cos) of k pi / SC_N
     double lnl_const;                 // -0.5 ln(2 pi) N
     double t0;                        // X_[0] (acceleration origin)
+    double tmax;                      // largest |t|
 };
 
 // Per-slot LDS scratch of the likelihood kernels.  KTE: the entry of the

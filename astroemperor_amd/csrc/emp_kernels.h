@@ -86,10 +86,14 @@ __device__ inline double prior_vector_wave(const ModelDev& md, const double* th,
     });
 }
 
-// Planet p's constants of the full parameter vector th.
+// Planet p's constants of the full parameter vector th.  The table is for mean
+// anomalies that reduce to [0, pi] and eccentricities of an orbit: its start goes
+// into the sin/cos table's index unclamped.  Any other planet takes Markley's
+// start, which is clamped.
 __device__ __forceinline__ PlanetC planet_slot(const ModelDev& md, const double* th, int p) {
     PlanetC pc = planet_setup(th + md.off_kep + 5 * p, md.param, md.use_c);
-    pc.ktab = md.N >= KT_MIN_EPOCHS && pc.e <= KT_EMAX;
+    const double reach = __builtin_fabs(pc.freq) * (md.tmax + __builtin_fabs(pc.tp)) + __builtin_fabs(pc.phase);
+    pc.ktab = md.N >= KT_MIN_EPOCHS && !pc.bad && pc.e <= KT_EMAX && reach <= KT_MMAX;
     return pc;
 }
 

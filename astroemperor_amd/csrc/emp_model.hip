@@ -445,6 +445,8 @@ int emp_model_host(const EmpModelDesc* d, ModelHost* h) {
     md.lnl_const = -0.5 * std::log(2.0 * M_PI) * (double)N;
     md.npseq = (int)h->pseq.size();
     md.t0 = d->t[0];
+    md.tmax = 0.0;
+    for (int i = 0; i < N; ++i) md.tmax = std::fmax(md.tmax, std::fabs(d->t[i]));
     // Fixed MA timescales (the usual setup): the weight exp(-dt / tau) of
     // every epoch is the same for all parameter vectors; compute it once.
     md.ma_wfixed = 0;
