@@ -234,6 +234,14 @@ __device__ __forceinline__ double cos_phase(const SL& sl, int c, double t) {
     return sl.cosw[c][1] * t + sl.cosw[c][2];
 }
 
+// |r| of a reduced phase r, held in the sin/cos table's range (half a step past
+// pi): a phase beyond FP64's resolution does not reduce to [0, pi].  NaN stays.
+__device__ __forceinline__ double cos_arg(double r) {
+    constexpr double MOST = PI_D + 0.49 * SC_H;
+    const double a = __builtin_fabs(r);
+    return a > MOST ? MOST : a;
+}
+
 // Terms added after the moving average: in the reference's block order
 // StellarActivity, Sinusoid and MagneticCycle follow MOAV (emp/emp.py:
 // 2628-2650), so the MA residuals do not contain them.
@@ -264,7 +272,7 @@ __device__ __forceinline__ double epoch_post(const ModelDev& md, const SL& sl, c
 #pragma unroll 1
     for (int c = 0; c < md.n_cos; ++c) {
         double sn, cs;
-        sincos_tab(tb, __builtin_fabs(reduce_2pi(cos_phase(sl, c, t))), sn, cs);
+        sincos_tab(tb, cos_arg(reduce_2pi(cos_phase(sl, c, t))), sn, cs);
         v = __builtin_fma(sl.cosw[c][0], cs, v);
     }
     return v;
