@@ -174,7 +174,7 @@ struct PlanetC {
     double bq, ibq;  // sqrt(1 - e^2) and its reciprocal (for gradients)
     int tp_mode;
     int bad;         // NaN-producing parameter set (reference would give NaN)
-    int ktab;        // this planet's per-vector Kepler table is built and used
+    int ktab;        // this planet's per-vector Kepler table is built and used (2: KT_F_FULL applies)
 };
 
 // Builds PlanetC from the 5 block parameters, following the reference's
@@ -390,23 +390,41 @@ constexpr double KT_EMAX = 0.95;
 // in the sin/cos table's range up to 6.1e-3 rad beyond [0, pi].  (From 1e16 on
 // the reduced M is any number.)
 constexpr double KT_MMAX = 4294967296.0;
-// A planet's Kepler path on the mixed path, as flags: the start from the
-// table (else the FP32 Markley starter), an FP32 Halley step after it, and
-// an FP64 Halley step (else an FP64 Newton step).  Markley: H32 | H64;
-// table: up to KT_ENEWTON TABLE, up to KT_EH64 TABLE | H64, up to KT_EMAX
-// TABLE | H32 | H64.
-constexpr int KT_F_TABLE = 1, KT_F_H32 = 2, KT_F_H64 = 4;
-__device__ __forceinline__ int kt_flags(bool table, double e) {
-    if (!table) return KT_F_H32 | KT_F_H64;
-    return KT_F_TABLE | (e > KT_EH64 ? KT_F_H32 : 0) | (e > KT_ENEWTON ? KT_F_H64 : 0);
+// A planet's Kepler path as flags: the start from the table (else Markley's, in
+// FP32 on the mixed path, in FP64 on the FP64 path), an FP32 Halley step after it,
+// and the larger FP64 step (mixed: Halley, else Newton; FP64: the cubic term of
+// kepler_fp64_tab, only without H32).  Markley: H32 | H64; table: up to KT_ENEWTON
+// TABLE, up to KT_EH64 TABLE | H64, up to KT_EMAX TABLE | H32 | H64.  FULL (a
+// series shorter than KT_SHORT): the mixed path takes the steps to FP64 accuracy,
+// Halley after a start that is within 7.3e-7 rad (kt_path).
+constexpr int KT_F_TABLE = 1, KT_F_H32 = 2, KT_F_H64 = 4, KT_F_FULL = 8;
+__device__ __forceinline__ int kt_flags(int ktab, double e) {
+    if (!ktab) return KT_F_H32 | KT_F_H64;
+    return KT_F_TABLE | (e > KT_EH64 ? KT_F_H32 : 0) | (e > KT_ENEWTON ? KT_F_H64 : 0) | (ktab > 1 ? KT_F_FULL : 0);
+}
+// The slot's mask as the path reads it: on the mixed path a planet with FULL gets
+// H64, and H32 too where it had H64 (above KT_ENEWTON).
+template <int PREC>
+__device__ __forceinline__ int kt_path(int kmask) {
+    if (PREC == 0) return kmask;
+    const unsigned m = (unsigned)kmask, full = (m >> 1) & 0x44444444u;
+    return (int)(m | full | ((m & full) >> 1));
 }
 // Planet p's flags from SlotLDS::ktab_mask (four bits per planet).
 __device__ __forceinline__ int kt_mode(int kmask, int p) { return (int)(((unsigned)kmask >> (4 * p)) & 7u); }
 // Building a table costs a wave one FP32 Kepler solve (64 nodes, one per lane),
 // less than the extra operations of a start without it over one chunk of 64
-// epochs: sweeps of 512 systems of 50 to 2000 epochs (median 200) take 727 / 674 /
-// 650 us with tables from 256 / 128 / 64 epochs on (mixed), 865 / 754 / 718 FP64.
+// epochs: sweeps of 512 systems of 50 to 2000 epochs (median 200) take 727 / 701
+// us with tables from 256 / 64 epochs on (mixed), 865 / 754 / 718 from 256 / 128 /
+// 64 (FP64).
 constexpr int KT_MIN_EPOCHS = 64;
+// Below this many epochs the mixed path solves Kepler's equation to FP64 accuracy
+// (KT_F_FULL), as its Markley start and Halley steps did there before it took the
+// table: against the FP64 path a planet's term is 2.3e-16 K rms and 2.2e-15 K at
+// most apart (e <= 0.95), where the cheaper steps of longer series leave 2.2e-14
+// and 3e-13 K (Newton, e <= 0.5) and 4.7e-16 and 1.8e-14 K (Halley alone, up to
+// 0.75).  It costs the sweeps above 650 -> 701 us.
+constexpr int KT_SHORT = 256;
 
 // The cubic Hermite interpolant on [M_j, M_j+1] in Horner form: with
 // d = E_j+1 - E_j and the scaled slopes s0 = h E'_j, s1 = h E'_j+1,

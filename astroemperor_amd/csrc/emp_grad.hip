@@ -666,7 +666,7 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
     tab_load(md, s_tile.tab);
     __syncthreads();
     slot_prepare_wg<WPT>(md, sl, live, wsub, lane);
-    const int kmask = wave_uniform(sl.ktab_mask);
+    const int kmask = kt_path<PREC>(wave_uniform(sl.ktab_mask));
     const bool tp = model_tp(md);
 
     const bool ma = md.ma_active;
@@ -926,7 +926,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(grad1_o
     for (int p = wave; p < md.K; p += NW)       // the per-vector Kepler tables, one planet per wave
         if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
     __syncthreads();
-    const int kmask = wave_uniform(sl.ktab_mask);
+    const int kmask = kt_path<PREC>(wave_uniform(sl.ktab_mask));
     const int ri5 = red5_index(lane), ri4 = red4_index(lane);    // the sums a lane holds after a reduction
 
     const bool ma = MA && md.ma_active;

@@ -83,7 +83,7 @@ struct SlotLDSt {
     double acc[AMAX];
     double cosw[CMAX][3];      // per cosine term: (amplitude, angular frequency, phase)
     KTE ktab[KP][KT_N];        // per planet, the Kepler table
-    int ktab_mask;             // bits 4 p .. 4 p + 2: planet p's Kepler path flags (kt_flags)
+    int ktab_mask;             // bits 4 p .. 4 p + 3: planet p's Kepler path flags (kt_flags)
 };
 
 // The slot of a workgroup that holds `SLOTS` of them: the interval tables

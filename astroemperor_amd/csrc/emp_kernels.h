@@ -93,7 +93,8 @@ __device__ inline double prior_vector_wave(const ModelDev& md, const double* th,
 __device__ __forceinline__ PlanetC planet_slot(const ModelDev& md, const double* th, int p) {
     PlanetC pc = planet_setup(th + md.off_kep + 5 * p, md.param, md.use_c);
     const double reach = __builtin_fabs(pc.freq) * (md.tmax + __builtin_fabs(pc.tp)) + __builtin_fabs(pc.phase);
-    pc.ktab = md.N >= KT_MIN_EPOCHS && !pc.bad && pc.e <= KT_EMAX && reach <= KT_MMAX;
+    const bool table = md.N >= KT_MIN_EPOCHS && !pc.bad && pc.e <= KT_EMAX && reach <= KT_MMAX;
+    pc.ktab = !table ? 0 : md.N < KT_SHORT ? 2 : 1;
     return pc;
 }
 
@@ -103,7 +104,7 @@ template <class SL>
 __device__ __forceinline__ void slot_rest(const ModelDev& md, SL& sl, int lane, int kf) {
     // the whole wave calls these: flag bit b of planet p to mask bit 4 p + b
     unsigned m = 0;
-    for (int b = 0; b < 3; ++b) {
+    for (int b = 0; b < 4; ++b) {
         const unsigned long long bits = __ballot((kf >> b) & 1);
         for (int p = 0; p < KMAX; ++p) m |= (unsigned)((bits >> p) & 1ull) << (4 * p + b);
     }
@@ -146,7 +147,7 @@ __device__ inline void slot_setup(const ModelDev& md, SL& sl, int lane) {
     int kf = 0;
     if (lane < md.K) {
         const PlanetC pc = planet_slot(md, sl.theta, lane);
-        kf = kt_flags(pc.ktab != 0, pc.e);
+        kf = kt_flags(pc.ktab, pc.e);
         sl.planet[lane] = pc;
     }
     slot_rest(md, sl, lane, kf);
@@ -201,7 +202,7 @@ constexpr int vecs_per_wg(int wpt) { return wpt == 1 ? 4 : 1; }
 __host__ __device__ __forceinline__ bool model_tp(const ModelDev& md) { return md.param == 3 || md.param == 4; }
 
 // Model value (planets + offset + acceleration) of the lane's NE epochs.
-// kmask: the slot's SlotLDS::ktab_mask as a wave-uniform scalar.
+// kmask: the slot's SlotLDS::ktab_mask as a wave-uniform scalar (kt_path).
 template <int PREC, int NE, class SL>
 __device__ __forceinline__ void epoch_mu(const ModelDev& md, const SL& sl, const SinCosTab& tb, const double (&t)[NE],
                                          const int (&k)[NE], int kmask, double (&mu)[NE]) {
@@ -647,7 +648,7 @@ __device__ double vec_lnl(const ModelDev& md, const SL& sl, const SinCosTab& tab
     const int lane = threadIdx.x & 63;
     const int wave = wave_uniform(threadIdx.x >> 6);
     constexpr int G = 64 * WPT;
-    const int kmask = wave_uniform(sl.ktab_mask);
+    const int kmask = kt_path<PREC>(wave_uniform(sl.ktab_mask));
     double chi = 0.0, prod = 1.0;
     int pexp = 0;
     double carry = 0.0;

@@ -200,7 +200,7 @@ __host__ __device__ inline size_t sys_lds(int wpt, int chunk, int Dfull, int K) 
 // unit that did a whole system's sweep at a time (16 walkers in step between
 // barriers, each wave setting up its own walker, the sweep as long as the
 // longest system's): per sweep of 64 / 512 / 2048 systems of 8 x 64 walkers, mixed,
-// 824 -> 151, 1152 -> 645, 3820 -> 2279 us; 512 FP64 1853 -> 731 us.
+// 824 -> 152, 1152 -> 701, 3820 -> 2457 us; 512 FP64 1853 -> 728 us.
 template <int PREC, int WPT, bool EXT, bool INIT>
 __global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_waves_per_eu(EXT ? 3 : 5))) void k_sys_lik(SysDev sd, int half, int step, int chunk,
                                                                      int nchunk) {
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_wav
         SlotView<KTE> sl{theta + r * Df, planet + r * K, ktab + slot * K, rest.gam, rest.jit2, rest.ma_c,
                          rest.ma_tau, rest.jit, rest.acc, rest.cosw, 0};
         // every wave computes the mask (a register); the LDS values are the same
-        slot_rest(md, sl, lane, lane < K ? kt_flags(sl.planet[lane].ktab != 0, sl.planet[lane].e) : 0);
+        slot_rest(md, sl, lane, lane < K ? kt_flags(sl.planet[lane].ktab, sl.planet[lane].e) : 0);
         for (int p = wsub; p < K; p += WPT)
             if (sl.planet[p].ktab) ktab_fill(sl.planet[p], lane, sl.ktab[p][lane]);
         vec_sync<WPT>();
@@ -374,8 +374,8 @@ struct EmpSystems {
 
 // Walkers per likelihood workgroup: two or four for every walker at work in it
 // (a workgroup's set-up serves them all), fewer while the pass has under eight
-// workgroups per compute unit (64 systems of 8 x 64 walkers: 168 / 147 us per
-// sweep at four / two; 512: 650 / 665).
+// workgroups per compute unit (512 systems of 8 x 64 walkers: 701 / 713 us per
+// sweep at four / two; 64, with the mixed path's cheaper steps: 168 / 147).
 static int chunk_of(const EmpSystems* p, int64_t tasks) {
     const int vecs = sys_vecs(p->tune.waves_per_theta);
     int per = p->tune.waves_per_wg == 16 ? 4 : 2;
