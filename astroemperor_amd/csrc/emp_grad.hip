@@ -659,7 +659,11 @@ __global__ __launch_bounds__(BLOCK) void k_lnl_grad(ModelDev md, const double* _
     if (live) expand_theta(md, sl, theta + b * ld, g, G);
     for (int j = g; j < MAXD; j += G) gl.g[j] = 0.0;
     for (int j = g; j < KMAX * 5; j += G) (&gl.nat[0][0])[j] = 0.0;
-    double* wacc = s_gw.acc[wave];
+    // From the thread's index, not the uniform wave number: with an address that is
+    // the same in every lane the compiler turns each atomic sum into a loop over
+    // the wave's lanes (a magnetic cycle's gradients with MA(2), 6 planets x 878
+    // epochs, one vector 66 -> 102 us).
+    double* wacc = s_gw.acc[threadIdx.x >> 6];
     double* wnat = s_gw.nat[wave];
     for (int j = lane; j < GW::N; j += 64) wacc[j] = 0.0;
     for (int j = lane; j < WN_N; j += 64) wnat[j] = 0.0;
