@@ -1297,6 +1297,16 @@ static void launch_grad_t(const ModelDev& md, const double* th, int64_t B, int64
 // 84 / 86 / 168 / 238 (7 planets with MA(1), mixed: 135 / 139 / 223 / 361
 // against 172 / 166 / 320 / 536).
 constexpr int GRAD1_NW = 2;
+// Four with the moving average while the batch has at most three vectors per
+// compute unit: the launch is then one vector's chain of tiles long, and four
+// waves halve the tiles.  FP64 at 2 / 4 waves per vector: 7 planets x 1747 epochs
+// with a global MA(1), 200 / 768 / 1024 vectors 76 / 51, 92 / 74 and 96 / 102 us;
+// 2 x 10^4 with MA(1) per instrument 197 / 113, 236 / 159 and 243 / 189 us; 6 x
+// 300, 26 / 18, 29 / 24 and 31 / 33 us.
+constexpr int GRAD1_NW_FEW = 4;
+static int grad1_waves(const EmpModel* m, int64_t B) {
+    return m->dev.ma_active && B <= 3 * (int64_t)m->n_cu ? GRAD1_NW_FEW : GRAD1_NW;
+}
 // LDS for the copies of the waves' sums (InsLayout) that keeps the KM = 8
 // instances' 6 workgroups per CU (160 KB, 20 KB of each without the copies).
 constexpr size_t GRAD1_INS_BYTES = 5632;
@@ -1391,14 +1401,15 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
             }
             return EMP_OK;
         }
+        const int nw = grad1_waves(m, B);
         // Eight copies of the wave's sums, fewer where many instruments would cost occupancy.
-        const int rows = GRAD1_NW * InsLayout(md, has_post(md)).rows;
+        const int rows = nw * InsLayout(md, has_post(md)).rows;
         int cl = 3;
-        while (cl && (rows << cl) * sizeof(double) > GRAD1_INS_BYTES) --cl;
+        while (cl && (rows << cl) * sizeof(double) > GRAD1_INS_BYTES * (nw / GRAD1_NW)) --cl;
         const size_t lds = (size_t)(rows << cl) * sizeof(double);
-#define EMP_CASE1(P, E, A, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, GRAD1_NW, M, T>), dim3((unsigned)B), dim3(64 * GRAD1_NW), lds, s, md, th, B, ld, lnl, grad, nf, stale, cl)
-#define EMP_CASE1M(P, E, A, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, GRAD1_FEW, T); else if (md.K <= 6) EMP_CASE1(P, E, A, 6, T); else EMP_CASE1(P, E, A, KMAX, T); }
-#define EMP_CASE1A(P, E, T) { if (md.ma_active) EMP_CASE1M(P, E, true, T) else EMP_CASE1M(P, E, false, T) }
+#define EMP_CASE1(P, E, A, W, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, W, M, T>), dim3((unsigned)B), dim3(64 * W), lds, s, md, th, B, ld, lnl, grad, nf, stale, cl)
+#define EMP_CASE1M(P, E, A, W, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, W, GRAD1_FEW, T); else if (md.K <= 6) EMP_CASE1(P, E, A, W, 6, T); else EMP_CASE1(P, E, A, W, KMAX, T); }
+#define EMP_CASE1A(P, E, T) { if (!md.ma_active) EMP_CASE1M(P, E, false, GRAD1_NW, T) else if (nw == GRAD1_NW) EMP_CASE1M(P, E, true, GRAD1_NW, T) else EMP_CASE1M(P, E, true, GRAD1_NW_FEW, T) }
 #define EMP_CASE1T(P, E) { if (model_tp(md)) EMP_CASE1A(P, E, true) else EMP_CASE1A(P, E, false) }
         if (precision == 0) { if (has_post(md)) EMP_CASE1T(0, 1) else EMP_CASE1T(0, 0) }
         else { if (has_post(md)) EMP_CASE1T(1, 1) else EMP_CASE1T(1, 0) }
