@@ -1385,8 +1385,9 @@ int emp_pick_grad_wpt(const EmpModel* m, int64_t B) {
 }
 
 int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t ld, double* lnl, double* grad,
-                       double* eps_scratch, hipStream_t s, int precision, int* stale, int wpt) {
+                       double* eps_scratch, hipStream_t s, int precision, int* stale, int wpt, int64_t shape) {
     if (B <= 0) return EMP_OK;
+    if (shape <= 0) shape = B;
     unsigned long long* nf = m->d_nonfinite;
     if (use_grad1(m)) {
         const ModelDev& md = m->dev;
@@ -1396,12 +1397,12 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
         if (B > PIECE) {
             for (int64_t b = 0; b < B; b += PIECE) {
                 const int rc = emp_launch_grad_ws(m, th + b * ld, std::min(PIECE, B - b), ld, lnl + b, grad + b * md.D,
-                                                  eps_scratch, s, precision, stale ? stale + b : nullptr, wpt);
+                                                  eps_scratch, s, precision, stale ? stale + b : nullptr, wpt, shape);
                 if (rc) return rc;
             }
             return EMP_OK;
         }
-        const int nw = grad1_waves(m, B);
+        const int nw = grad1_waves(m, shape);
         // Eight copies of the wave's sums, fewer where many instruments would cost occupancy.
         const int rows = nw * InsLayout(md, has_post(md)).rows;
         int cl = 3;
@@ -1421,7 +1422,7 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
         return EMP_OK;
     }
     if (m->dev.ma_active && !eps_scratch) { emp_set_error("moving-average gradient needs a scratch buffer"); return EMP_EINVAL; }
-    if (wpt <= 0) wpt = emp_pick_grad_wpt(m, B);
+    if (wpt <= 0) wpt = emp_pick_grad_wpt(m, shape);
 #define EMP_CASE(P, W) if (precision == P && wpt == W) launch_grad_t<P, W>(m->dev, th, B, ld, lnl, grad, nf, eps_scratch, stale, s); else
     EMP_CASE(0, 1) EMP_CASE(0, 2) EMP_CASE(0, 4) EMP_CASE(0, 8)
     EMP_CASE(1, 1) EMP_CASE(1, 2) EMP_CASE(1, 4) EMP_CASE(1, 8) { emp_set_error("bad precision/wpt"); return EMP_EINVAL; }

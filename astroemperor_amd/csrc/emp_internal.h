@@ -156,10 +156,12 @@ int emp_launch_grad(EmpModel* m, const double* d_theta, int64_t B, int64_t ld, d
 // The same with a caller-owned scratch of B x N doubles (used only when the
 // moving average is active); allocates nothing, so it may be captured.
 // stale (optional, per vector): only vectors flagged 1 are computed, and their
-// flags are cleared.  wpt: waves per vector (0: emp_pick_grad_wpt).
+// flags are cleared.  wpt: waves per vector of the two-pass kernel (0:
+// emp_pick_grad_wpt).  shape: the batch whose launch shape to take (0: B); a
+// vector's results are the same bits in batches of one shape.
 int emp_launch_grad_ws(const EmpModel* m, const double* d_theta, int64_t B, int64_t ld, double* d_lnl,
                        double* d_grad, double* eps_scratch, hipStream_t s, int precision = EMP_FP64,
-                       int* stale = nullptr, int wpt = 0);
+                       int* stale = nullptr, int wpt = 0, int64_t shape = 0);
 int emp_pick_grad_wpt(const EmpModel* m, int64_t B);
 // Doubles of scratch one adjoint launch over B vectors needs, and those to set
 // aside for it where the kernel may be switched afterwards.

@@ -85,8 +85,9 @@ struct EmpPT {
     hipGraphExec_t graph_run[5] = {};         // 2, 4, 8, 16, 32 stretch sweeps in one graph
     double w_stretch = 1.0, w_grad = 0.0;     // move weights (one move per sweep)
     int wpt = 1;
-    int grad_wpt = 2;            // waves per vector of the adjoint launches (one shape for both, so a
-                                 // slot's gradient does not depend on which launch computed it)
+    int grad_wpt = 2;            // waves per vector of the two-pass adjoint's launches (both adjoints take one
+                                 // shape for positions and proposals, so that a slot's gradient does not
+                                 // depend on which launch computed it)
     size_t swap_lds = 0;         // dynamic LDS of the swap kernel, 0 = global-memory instance
     size_t swap_lds_fit = 0;     // what the LDS instance needs when the ensemble fits, else 0
     long long host_sweeps = 0;   // mirror of the device counter
@@ -1248,7 +1249,7 @@ static int launch_grad_sweep(EmpPT* p, hipEvent_t* ev = nullptr) {
     int rc = launch_record(p, 1);
     if (rc) return rc;
     rc = emp_launch_grad_ws(p->model, d.X, TW, d.D, d.lg_l, d.lg_g, d.lg_scr, p->stream, p->desc.precision,
-                            d.lg_stale, p->grad_wpt);
+                            d.lg_stale, p->grad_wpt, tasks);
     if (rc) return rc;
     for (int st = 0; st < p->desc.nsteps; ++st)
         for (int h = 0; h < 2; ++h) {
@@ -1260,7 +1261,7 @@ static int launch_grad_sweep(EmpPT* p, hipEvent_t* ev = nullptr) {
             hipEvent_t* e = ev ? ev + 2 * (2 * st + h) : nullptr;
             if (e) EMP_HIP(hipEventRecord(e[0], p->stream));
             rc = emp_launch_grad_ws(p->model, d.lg_Xp, tasks, d.D, d.lg_lp, d.lg_gp, d.lg_scr, p->stream,
-                                    p->desc.precision, nullptr, p->grad_wpt);
+                                    p->desc.precision, nullptr, p->grad_wpt, tasks);
             if (rc) return rc;
             if (e) EMP_HIP(hipEventRecord(e[1], p->stream));
             hipLaunchKernelGGL(k_lg_accept, dim3(tgrid), dim3(PRIOR_BLOCK), 0, p->stream, d, h, st);
