@@ -82,6 +82,8 @@ struct EmpPT {
     hipStream_t stream = nullptr;
     hipGraphExec_t graph_exec = nullptr;      // stretch sweep
     hipGraphExec_t graph_grad = nullptr;      // gradient-move sweep
+    int graph_grad_kernel = 0;                // the adjoint kernel (EMP_GRAD_KERNEL_*) it was captured with
+    size_t lg_scr_cap = 0;                    // doubles behind dev.lg_scr
     hipGraphExec_t graph_run[5] = {};         // 2, 4, 8, 16, 32 stretch sweeps in one graph
     double w_stretch = 1.0, w_grad = 0.0;     // move weights (one move per sweep)
     int wpt = 1;
@@ -1321,6 +1323,25 @@ static int alloc(EmpPT* p, T** out, size_t n) {
     return EMP_OK;
 }
 
+// Before gradient sweeps: the model's adjoint kernel may have been switched
+// (emp_model_set_grad_kernel) since the sweep was captured or its scratch was
+// allocated.
+static int sync_grad_kernel(EmpPT* p) {
+    PTDev& d = p->dev;
+    if (!(p->w_grad > 0.0) || !d.lg_g) return EMP_OK;
+    if (p->graph_grad && p->graph_grad_kernel != p->model->grad_kernel) {
+        EMP_HIP(hipGraphExecDestroy(p->graph_grad));
+        p->graph_grad = nullptr;
+    }
+    p->graph_grad_kernel = p->model->grad_kernel;
+    const size_t need = emp_grad_scratch_doubles(p->model, (int64_t)d.T * d.W);
+    if (need > p->lg_scr_cap) {
+        if (int rc = alloc(p, &d.lg_scr, need)) return rc;
+        p->lg_scr_cap = need;
+    }
+    return EMP_OK;
+}
+
 // Every slot's gradient is recomputed by the next gradient sweep (after a
 // state was loaded or restored; no-op while the gradient move was never on).
 static int mark_all_stale(EmpPT* p) {
@@ -1442,6 +1463,7 @@ extern "C" int emp_pt_run(EmpPT* p, int64_t nsweeps, int32_t use_graph) {
         return EMP_EINVAL;
     }
     if (nsweeps == 0) return EMP_OK;
+    if (int rc = sync_grad_kernel(p)) return rc;
     hipEvent_t e0, e1;
     EMP_HIP(hipEventCreate(&e0));
     EMP_HIP(hipEventCreate(&e1));
@@ -1528,6 +1550,7 @@ extern "C" int emp_pt_time_halfstep(EmpPT* p, int32_t n, double* ms_avg) {
 extern "C" int emp_pt_time_gradstep(EmpPT* p, int32_t n, double* ms_avg) {
     if (!p || n < 1 || !ms_avg) { emp_set_error("bad argument"); return EMP_EINVAL; }
     if (!(p->w_grad > 0.0) || !p->dev.lg_g) { emp_set_error("the gradient move is not enabled"); return EMP_EINVAL; }
+    if (int rc = sync_grad_kernel(p)) return rc;
     const int per = 2 * p->desc.nsteps;
     const int64_t ns = ((int64_t)n + per - 1) / per;
     if (p->host_sweeps + ns > p->dev.max_sweeps) {
@@ -1798,6 +1821,7 @@ extern "C" int emp_pt_set_moves(EmpPT* p, const EmpMoveDesc* moves, int32_t n) {
             v.lg_stale = nullptr;
             return rc;
         }
+        p->lg_scr_cap = emp_grad_scratch_reserve(m, (int64_t)TW);
         p->grad_wpt = emp_pick_grad_wpt(m, (int64_t)T2);
         if ((rc = mark_all_stale(p))) return rc;
         EMP_HIP(hipStreamSynchronize(p->stream));

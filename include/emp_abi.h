@@ -179,8 +179,9 @@ int emp_model_set_waves_per_theta(EmpModel* model, int32_t waves_per_theta);
  *     (B x N doubles of scratch), then the epochs in reverse;
  *   EMP_GRAD_KERNEL_SINGLE_PASS: one pass, no scratch; EMP_EUNSUP for MA
  *     orders above 1.
- * A gradient move enabled before a change keeps the scratch it allocated:
- * switch before emp_pt_set_moves. */
+ * A gradient move enabled before a change follows it: its next run captures
+ * its sweeps again and, if the scratch of emp_pt_set_moves is too small,
+ * allocates the kernel's. */
 #define EMP_GRAD_KERNEL_AUTO 0
 #define EMP_GRAD_KERNEL_TWO_PASS 1
 #define EMP_GRAD_KERNEL_SINGLE_PASS 2
