@@ -1389,19 +1389,21 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
     if (B <= 0) return EMP_OK;
     if (shape <= 0) shape = B;
     unsigned long long* nf = m->d_nonfinite;
+    // A grid holds fewer than 2^32 threads: larger batches in pieces (one vector
+    // takes 128 threads of the single-pass kernel there, up to 512 of the other,
+    // whose scratch rows a piece uses again after the one before it).
+    const int64_t PIECE = (int64_t)1 << (use_grad1(m) ? 24 : 22);
+    if (B > PIECE) {
+        for (int64_t b = 0; b < B; b += PIECE) {
+            const int rc = emp_launch_grad_ws(m, th + b * ld, std::min(PIECE, B - b), ld, lnl + b, grad + b * m->dev.D,
+                                              eps_scratch, s, precision, stale ? stale + b : nullptr, wpt, shape);
+            if (rc) return rc;
+        }
+        return EMP_OK;
+    }
     if (use_grad1(m)) {
         const ModelDev& md = m->dev;
         if (precision != 0 && precision != 1) { emp_set_error("bad precision"); return EMP_EINVAL; }
-        // a grid holds fewer than 2^32 threads: larger batches in pieces
-        constexpr int64_t PIECE = (int64_t)1 << 24;
-        if (B > PIECE) {
-            for (int64_t b = 0; b < B; b += PIECE) {
-                const int rc = emp_launch_grad_ws(m, th + b * ld, std::min(PIECE, B - b), ld, lnl + b, grad + b * md.D,
-                                                  eps_scratch, s, precision, stale ? stale + b : nullptr, wpt, shape);
-                if (rc) return rc;
-            }
-            return EMP_OK;
-        }
         const int nw = grad1_waves(m, shape);
         // Eight copies of the wave's sums, fewer where many instruments would cost occupancy.
         const int rows = nw * InsLayout(md, has_post(md)).rows;

@@ -224,9 +224,11 @@ int emp_launch_lnl(const EmpModel* m, const double* d_theta, int64_t B, int64_t 
     if (B <= 0) return EMP_OK;
     const ModelDev& md = m->dev;
     if (wpt <= 0) wpt = emp_pick_wpt(m, B);
+    constexpr int64_t PIECE = (int64_t)1 << 22;      // a grid holds fewer than 2^32 threads, a vector takes up to 512
 #define EMP_CASE(P, W)                                                                 \
     if (precision == P && wpt == W) {                                                  \
-        launch_lnl_t<P, W>(md, d_theta, B, ld, d_lnl, m->d_nonfinite, s);              \
+        for (int64_t b = 0; b < B; b += PIECE)                                         \
+            launch_lnl_t<P, W>(md, d_theta + b * ld, std::min(PIECE, B - b), ld, d_lnl + b, m->d_nonfinite, s); \
         EMP_HIP(hipGetLastError());                                                    \
         return EMP_OK;                                                                 \
     }
