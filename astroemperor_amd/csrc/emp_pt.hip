@@ -1656,7 +1656,7 @@ static int gather_state(EmpPT* p, int32_t what, double* out) {
     const PTDev& v = p->dev;
     const int TW = v.T * v.W;
     const double* src = what == EMP_PT_STATE_X ? v.X : what == EMP_PT_STATE_LNL ? v.lnl : v.lnp;
-    return emp_gather_rows(src, v.map, TW, TW, what == EMP_PT_STATE_X ? v.D : 1, &p->gather_buf, &p->gather_cap,
+    return emp_gather_rows(p->model->device, src, v.map, TW, TW, what == EMP_PT_STATE_X ? v.D : 1, &p->gather_buf, &p->gather_cap,
                            p->stream, out);
 }
 
@@ -1769,6 +1769,8 @@ extern "C" int emp_pt_lnl_moments(EmpPT* p, int64_t discard, double* mean, doubl
     const long long R0 = std::min<long long>(p->hist_base * v.nsteps, S);
     if (discard < 0 || R0 + discard >= S) { emp_set_error("discard must lie in [0, %lld) rows", S - R0); return EMP_EINVAL; }
     discard += R0;
+    const DeviceScope scope(p->model->device);
+    EMP_HIP(scope.err);
     double* d = nullptr;
     EMP_HIP(hipMalloc(&d, 3 * (size_t)v.T * sizeof(double)));
     hipLaunchKernelGGL(k_pt_lnl_moments, dim3((unsigned)v.T), dim3(MOM_BLOCK), 0, p->stream, v, (long long)discard, S,

@@ -320,12 +320,34 @@ __global__ static void k_gather_rows(const double* __restrict__ src, const int* 
 
 }  // namespace emp
 
+// An engine's device as the current one for a scope, for callers that read its
+// state with another device current: memory is allocated on the current device.
+struct DeviceScope {
+    int before = -1;
+    hipError_t err;
+    explicit DeviceScope(int device) {
+        int now = -1;
+        err = hipGetDevice(&now);
+        if (err == hipSuccess && now != device) {
+            err = hipSetDevice(device);
+            if (err == hipSuccess) before = now;
+        }
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+    ~DeviceScope() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
 // Gathers n rows on the device in pieces of at most 32 MiB (the engine's `buf`,
 // grown to the piece once and kept) and copies each to the host: one kernel and
 // one copy where every buffer used to be copied whole and permuted by the host.
 constexpr size_t GATHER_MOST = (size_t)4 << 20;      // doubles
-inline int emp_gather_rows(const double* src, const int* map, long long n, int per, int width, double** buf,
+inline int emp_gather_rows(int device, const double* src, const int* map, long long n, int per, int width, double** buf,
                            size_t* cap, hipStream_t s, double* host) {
+    const DeviceScope scope(device);
+    EMP_HIP(scope.err);
     long long piece = std::max<long long>(1, std::min<long long>(n, (long long)(GATHER_MOST / width)));
     if (*cap < (size_t)piece * width) {
         if (*buf) (void)hipFree(*buf);

@@ -361,7 +361,7 @@ struct EmpSystems {
     hipStream_t stream = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     EmpSystemsTuning tune{};
-    int n_cu = 256;
+    int n_cu = 256, device = 0;
     bool ext = false;          // some system needs the extended instance (model_ext)
     int max_d = 1, max_k = 1, max_l = 1;   // longest full vector, most planets, longest prior sequence of a system
     int64_t x_total = 0;
@@ -512,6 +512,7 @@ extern "C" int emp_systems_create(const EmpModelDesc* models, const EmpSystemsDe
             return EMP_EHIP;
         }
         p->n_cu = prop.multiProcessorCount;
+        p->device = dev;
     }
     std::vector<double> t(nep), y(nep), s2(nep), dt(nep), fixed(npar), sai(nsai);
     std::vector<int> ins(nep), inv(npar), fidx(nfree), bst(nblk), pseq(nseq), saib(nsaib);
@@ -803,10 +804,10 @@ static int gather_systems(EmpSystems* p, int s0, int s1, int what, double* out) 
     const SysDev& v = p->dev;
     const int TW = v.T * v.W;
     if (what != EMP_PT_STATE_X)
-        return emp_gather_rows((what == EMP_PT_STATE_LNL ? v.lnl : v.lnp) + (size_t)s0 * TW, v.map + (size_t)s0 * TW,
+        return emp_gather_rows(p->device, (what == EMP_PT_STATE_LNL ? v.lnl : v.lnp) + (size_t)s0 * TW, v.map + (size_t)s0 * TW,
                                (long long)(s1 - s0) * TW, TW, 1, &p->gather_buf, &p->gather_cap, p->stream, out);
     for (int s = s0; s < s1; ++s) {
-        const int rc = emp_gather_rows(v.X + p->xoff[s], v.map + (size_t)s * TW, TW, TW, p->D[s], &p->gather_buf,
+        const int rc = emp_gather_rows(p->device, v.X + p->xoff[s], v.map + (size_t)s * TW, TW, TW, p->D[s], &p->gather_buf,
                                        &p->gather_cap, p->stream, out);
         if (rc) return rc;
         out += (size_t)TW * p->D[s];
