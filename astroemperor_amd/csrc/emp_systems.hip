@@ -77,7 +77,7 @@ __device__ __forceinline__ PTView sys_view(const SysDev& sd, int s, int D) {
                    sd.accepted + s * TW);
 }
 
-// The prior pass: workgroup (s, c) takes the c-th SYS_PRIOR_TASKS tasks of
+// The prior pass: workgroup (s, c) (from system s0 on) takes the c-th SYS_PRIOR_TASKS tasks of
 // system s: the proposals (one thread per task), every (task, term) pair of the
 // prior's summation sequence (the system's resolved sequence in LDS, all loads
 // of the walkers' rows in flight together), then the sum of each task's terms in
@@ -94,13 +94,13 @@ __host__ __device__ inline size_t sys_prior_terms(int L) {
     const size_t want = (size_t)SYS_PRIOR_TASKS * L, cap = 4096;
     return want < cap ? want : (cap > (size_t)L ? cap : (size_t)L);
 }
-__global__ __launch_bounds__(SYS_PASS) void k_sys_prior(SysDev sd, int half, int step, int nchunk, int terms_cap) {
+__global__ __launch_bounds__(SYS_PASS) void k_sys_prior(SysDev sd, int s0, int half, int step, int nchunk, int terms_cap) {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) char s_dyn[];
     __shared__ double s_z[SYS_PRIOR_TASKS];
     __shared__ int s_k[SYS_PRIOR_TASKS], s_j[SYS_PRIOR_TASKS];
     const int tid = threadIdx.x;
-    const int s = blockIdx.x / nchunk, b0 = (blockIdx.x - s * nchunk) * SYS_PRIOR_TASKS;
+    const int sl = blockIdx.x / nchunk, s = s0 + sl, b0 = (blockIdx.x - sl * nchunk) * SYS_PRIOR_TASKS;
     const ModelDev& md = sys_model(sd, s);
     const PTView pv = sys_view(sd, s, md.D);
     const int ntask = sd.T * (sd.W / 2), nt = min(SYS_PRIOR_TASKS, ntask - b0), L = md.npseq;
@@ -192,7 +192,7 @@ __host__ __device__ inline size_t sys_lds(int wpt, int chunk, int Dfull, int K) 
 }
 
 // The likelihood pass: workgroup (it, c) takes the c-th `chunk` listed tasks of
-// the it-th system in queue order; with INIT instead every walker (the state
+// system it0 + it in queue order; with INIT instead every walker (the state
 // loaded into slot = position order), whose prior and likelihood it stores.
 // WPT waves per walker; EXT: the instance with the extended model features
 // (model_ext), used when any system of the batch has them.
@@ -202,7 +202,7 @@ __host__ __device__ inline size_t sys_lds(int wpt, int chunk, int Dfull, int K) 
 // longest system's): per sweep of 64 / 512 / 2048 systems of 8 x 64 walkers, mixed,
 // 824 -> 152, 1152 -> 701, 3820 -> 2457 us; 512 FP64 1853 -> 728 us.
 template <int PREC, int WPT, bool EXT, bool INIT>
-__global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_waves_per_eu(EXT ? 3 : 5))) void k_sys_lik(SysDev sd, int half, int step, int chunk,
+__global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_waves_per_eu(EXT ? 3 : 5))) void k_sys_lik(SysDev sd, int it0, int half, int step, int chunk,
                                                                      int nchunk) {
     constexpr int VECS = sys_vecs(WPT), NT = 64 * WPT * VECS;
     using KTE = SysKTE<WPT>;
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(64 * WPT * sys_vecs(WPT)) __attribute__((amdgpu_wav
     __shared__ int s_k[SYS_CHUNK], s_j[SYS_CHUNK], s_acc[VECS];
     const int tid = threadIdx.x, wave = wave_uniform(tid >> 6), lane = tid & 63;
     const int it = blockIdx.x / nchunk, q0 = (blockIdx.x - it * nchunk) * chunk;
-    const int s = __builtin_amdgcn_readfirstlane(sd.order[it]);
+    const int s = __builtin_amdgcn_readfirstlane(sd.order[it0 + it]);
     const int ntask = INIT ? sd.T * sd.W : sd.T * (sd.W / 2);
     const int nl = INIT ? ntask : __builtin_amdgcn_readfirstlane(sd.nlive[(size_t)half * sd.S + s]);
     if (q0 >= nl) return;                    // the whole workgroup
@@ -383,6 +383,10 @@ static int chunk_of(const EmpSystems* p, int64_t tasks) {
     return vecs * per;
 }
 
+// Systems per launch of `nchunk` workgroups of `nthr` threads each: a grid holds
+// fewer than 2^32 threads.
+static int systems_per_launch(int nchunk, int nthr) { return (int)(((int64_t)1 << 31) / ((int64_t)nchunk * nthr)); }
+
 template <bool INIT>
 static int launch_lik(EmpSystems* p, int half, int step) {
     const EmpSystemsTuning& tu = p->tune;
@@ -390,13 +394,16 @@ static int launch_lik(EmpSystems* p, int half, int step) {
     const int n = p->desc.ntemps * p->desc.nwalkers / (INIT ? 1 : 2), chunk = chunk_of(p, (int64_t)S * n);
     const int nchunk = (n + chunk - 1) / chunk;
     const size_t lds = sys_lds(tu.waves_per_theta, chunk, p->max_d, p->max_k);
-    const dim3 grid((unsigned)S * (unsigned)nchunk);
+    const int most = systems_per_launch(nchunk, 64 * tu.waves_per_theta * sys_vecs(tu.waves_per_theta));
 #define EMP_CASE(P, WP)                                                                                      \
     if (prec == P && tu.waves_per_theta == WP) {                                                            \
         const dim3 nt(64 * WP * sys_vecs(WP));                                                               \
-        if (p->ext) hipLaunchKernelGGL((k_sys_lik<P, WP, true, INIT>), grid, nt, lds, p->stream, p->dev, half, step, chunk, nchunk); \
-        else hipLaunchKernelGGL((k_sys_lik<P, WP, false, INIT>), grid, nt, lds, p->stream, p->dev, half, step, chunk, nchunk); \
-        EMP_HIP(hipGetLastError());                                                                         \
+        for (int s0 = 0; s0 < S; s0 += most) {                                                              \
+            const dim3 grid((unsigned)std::min(most, S - s0) * (unsigned)nchunk);                            \
+            if (p->ext) hipLaunchKernelGGL((k_sys_lik<P, WP, true, INIT>), grid, nt, lds, p->stream, p->dev, s0, half, step, chunk, nchunk); \
+            else hipLaunchKernelGGL((k_sys_lik<P, WP, false, INIT>), grid, nt, lds, p->stream, p->dev, s0, half, step, chunk, nchunk); \
+            EMP_HIP(hipGetLastError());                                                                     \
+        }                                                                                                    \
         return EMP_OK;                                                                                      \
     }
     EMP_SYS_CONFIGS(EMP_CASE)
@@ -406,18 +413,21 @@ static int launch_lik(EmpSystems* p, int half, int step) {
 }
 
 static int launch_sweep(EmpSystems* p) {
-    const unsigned S = (unsigned)p->desc.n_systems;
+    const int S = p->desc.n_systems;
     p->dev.order = p->tune.order == 0 ? p->d_order_lpt : p->d_order_input;
     for (int st = 0; st < p->desc.nsteps; ++st)
         for (int half = 0; half < 2; ++half) {
             const int nc = (p->desc.ntemps * (p->desc.nwalkers / 2) + SYS_PRIOR_TASKS - 1) / SYS_PRIOR_TASKS;
             const size_t terms = sys_prior_terms(p->max_l), lds = terms * sizeof(double) + p->max_l * sizeof(PseqEntry);
-            hipLaunchKernelGGL(k_sys_prior, dim3(S * (unsigned)nc), dim3(SYS_PASS), lds, p->stream, p->dev, half, st, nc,
-                               (int)terms);
-            EMP_HIP(hipGetLastError());
+            const int most = systems_per_launch(nc, SYS_PASS);
+            for (int s0 = 0; s0 < S; s0 += most) {
+                hipLaunchKernelGGL(k_sys_prior, dim3((unsigned)std::min(most, S - s0) * (unsigned)nc), dim3(SYS_PASS), lds,
+                                   p->stream, p->dev, s0, half, st, nc, (int)terms);
+                EMP_HIP(hipGetLastError());
+            }
             if (int rc = launch_lik<false>(p, half, st)) return rc;
         }
-    hipLaunchKernelGGL(k_sys_swap, dim3(S), dim3(SYS_PASS), 0, p->stream, p->dev);
+    hipLaunchKernelGGL(k_sys_swap, dim3((unsigned)S), dim3(SYS_PASS), 0, p->stream, p->dev);
     EMP_HIP(hipGetLastError());
     return EMP_OK;
 }
