@@ -161,6 +161,74 @@ __global__ __launch_bounds__(PRIOR_THREADS) void k_prior(ModelDev md, const doub
     out[b0 + threadIdx.x] = lp;
 }
 
+// The same sum by one lane per vector, for batches that fill the chip with lanes
+// (prior_each): the wave brings its vectors' rows into LDS, or, where rows of more
+// than PRIOR_ROW parameters would leave too few waves, the arguments of PRIOR_CHUNK
+// entries at a time; then every lane adds its vector's terms in sequence order, the
+// entries being scalar loads.  Bound by bandwidth for short rows, by the terms'
+// logarithms for long ones.  16 vectors per workgroup exchange every term through
+// LDS instead, which pays while there are too few vectors for the lanes: 2^20
+// vectors of 7 / 13 / 31 / 67 parameters take 108 / 174 / 321 / 806 us there and 37 /
+// 62 / 168 / 432 here (38 / 107 / 344 / 782 by a thread per vector from a copy in
+// scratch memory), 131,072 15 / 22 / 44 / 88 and 11 / 11 / 35 / 84, 65,536 11 / 14 /
+// 23 / 48 and 11 / 11 / 25 / 69.
+constexpr int PRIOR_LANES = 64, PRIOR_CHUNK = 16, PRIOR_ROW = 24;
+template <bool ROWS>
+__global__ __launch_bounds__(PRIOR_LANES) void k_prior_each(ModelDev md, const double* __restrict__ theta, int64_t B,
+                                                            int64_t ld, double* __restrict__ out) {
+#pragma clang fp contract(off)
+    constexpr int S = (ROWS ? PRIOR_ROW : PRIOR_CHUNK) + 1;      // rows on other banks
+    __shared__ double s_x[PRIOR_LANES][S];
+    const int lane = threadIdx.x, L = md.npseq;
+    const int64_t b0 = (int64_t)blockIdx.x * PRIOR_LANES;
+    const int nv = (int)(B - b0 < PRIOR_LANES ? B - b0 : PRIOR_LANES);
+    // the argument of an entry: a parameter, or the eccentricity of two
+    auto argument = [](int kind, int fa, int fb, double va, double vb, const double* row) {
+#pragma clang fp contract(off)
+        if (kind == 0) return row[fa];
+        const double s3 = fa >= 0 ? row[fa] : va, s4 = fb >= 0 ? row[fb] : vb;
+        return s3 * s3 + s4 * s4;
+    };
+    double lp = 0.0;
+    bool out_of = lane >= nv;      // later: -inf at a block's end, where the sum stops
+    if (ROWS) {
+        const int D = md.D;
+        for (int e = lane; e < nv * D; e += PRIOR_LANES) {
+            const int r = e / D, c = e - r * D;
+            s_x[r][c] = theta[(b0 + r) * ld + c];
+        }
+        wave_sync();
+        for (int i = 0; i < L; ++i) {
+            const PseqEntry& pe = md.pseq_e[i];
+            if (pe.kind == 2) out_of = out_of || lp == -__builtin_inf();
+            else if (!out_of) lp += prior_term(pe.term, argument(pe.kind, pe.fa, pe.fb, pe.va, pe.vb, s_x[lane]));
+        }
+    } else {
+        const int il = lane % PRIOR_CHUNK, r0 = lane / PRIOR_CHUNK;
+        for (int i0 = 0; i0 < L; i0 += PRIOR_CHUNK) {
+            if (i0 + il < L && md.pseq_e[i0 + il].kind != 2) {
+                const PseqEntry& pe = md.pseq_e[i0 + il];
+                const int kind = pe.kind, fa = pe.fa, fb = pe.fb;
+                const double va = pe.va, vb = pe.vb;
+#pragma unroll
+                for (int k = 0; k < PRIOR_CHUNK; ++k) {
+                    const int r = k * (PRIOR_LANES / PRIOR_CHUNK) + r0;
+                    if (r < nv) s_x[r][il] = argument(kind, fa, fb, va, vb, theta + (b0 + r) * ld);
+                }
+            }
+            wave_sync();
+            const int n = min(PRIOR_CHUNK, L - i0);
+            for (int q = 0; q < n; ++q) {
+                const PseqEntry& pe = md.pseq_e[i0 + q];
+                if (pe.kind == 2) out_of = out_of || lp == -__builtin_inf();
+                else if (!out_of) lp += prior_term(pe.term, s_x[lane][q]);
+            }
+            wave_sync();
+        }
+    }
+    if (lane < nv) out[b0 + lane] = lp;
+}
+
 __global__ __launch_bounds__(BLOCK) void k_model_eval(ModelDev md, const double* __restrict__ theta,
                                                       double* out_model, double* out_err2) {
     __shared__ SlotLDS<1> sl;
@@ -239,16 +307,29 @@ int emp_launch_lnl(const EmpModel* m, const double* d_theta, int64_t B, int64_t 
     return EMP_EINVAL;
 }
 
+// One lane per vector from one wave per SIMD on, two for rows of more than
+// PRIOR_ROW parameters (measured at k_prior_each).
+static bool prior_each(const EmpModel* m, int64_t B) {
+    const int64_t lanes = (int64_t)m->n_cu * 4 * PRIOR_LANES;
+    return B >= (m->dev.D <= PRIOR_ROW ? 1 : 2) * lanes;
+}
+
 int emp_launch_prior(const EmpModel* m, const double* d_theta, int64_t B, int64_t ld, double* d_lnp,
                      hipStream_t s) {
     if (B <= 0) return EMP_OK;
     constexpr int64_t PIECE = (int64_t)1 << 24;      // a grid holds fewer than 2^32 threads
+    const bool each = prior_each(m, B);
     const int row = prior_row(m->dev.npseq);
     const size_t lds = (size_t)PRIOR_VECS * row * sizeof(double) + (size_t)row * sizeof(int);
     for (int64_t b = 0; b < B; b += PIECE) {
-        const int64_t n = std::min(PIECE, B - b), grid = (n + PRIOR_VECS - 1) / PRIOR_VECS;
-        hipLaunchKernelGGL(k_prior, dim3((unsigned)grid), dim3(PRIOR_THREADS), lds, s, m->dev, d_theta + b * ld, n, ld,
-                           d_lnp + b);
+        const int64_t n = std::min(PIECE, B - b), per = each ? PRIOR_LANES : PRIOR_VECS;
+        const dim3 grid((unsigned)((n + per - 1) / per));
+        if (each && m->dev.D <= PRIOR_ROW)
+            hipLaunchKernelGGL(k_prior_each<true>, grid, dim3(PRIOR_LANES), 0, s, m->dev, d_theta + b * ld, n, ld, d_lnp + b);
+        else if (each)
+            hipLaunchKernelGGL(k_prior_each<false>, grid, dim3(PRIOR_LANES), 0, s, m->dev, d_theta + b * ld, n, ld, d_lnp + b);
+        else
+            hipLaunchKernelGGL(k_prior, grid, dim3(PRIOR_THREADS), lds, s, m->dev, d_theta + b * ld, n, ld, d_lnp + b);
     }
     EMP_HIP(hipGetLastError());
     return EMP_OK;
