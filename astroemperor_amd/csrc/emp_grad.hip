@@ -1297,15 +1297,16 @@ static void launch_grad_t(const ModelDev& md, const double* th, int64_t B, int64
 // 84 / 86 / 168 / 238 (7 planets with MA(1), mixed: 135 / 139 / 223 / 361
 // against 172 / 166 / 320 / 536).
 constexpr int GRAD1_NW = 2;
-// Four with the moving average while the batch has at most three vectors per
-// compute unit: the launch is then one vector's chain of tiles long, and four
-// waves halve the tiles.  FP64 at 2 / 4 waves per vector: 7 planets x 1747 epochs
+// Four with the moving average, for series of more than one tile, while the batch
+// has at most three vectors per compute unit: the launch is then one vector's chain
+// of tiles long, and four waves halve the tiles.  FP64 at 2 / 4 waves per vector: 7 planets x 1747 epochs
 // with a global MA(1), 200 / 768 / 1024 vectors 76 / 51, 92 / 74 and 96 / 102 us;
 // 2 x 10^4 with MA(1) per instrument 197 / 113, 236 / 159 and 243 / 189 us; 6 x
-// 300, 26 / 18, 29 / 24 and 31 / 33 us.
+// 300, 26 / 18, 29 / 24 and 31 / 33 us; 7 x 256, one tile of two waves, 19 / 19 and
+// 24 / 27 us (200, 768).
 constexpr int GRAD1_NW_FEW = 4;
 static int grad1_waves(const EmpModel* m, int64_t B) {
-    return m->dev.ma_active && B <= 3 * (int64_t)m->n_cu ? GRAD1_NW_FEW : GRAD1_NW;
+    return m->dev.ma_active && m->dev.N > 128 * GRAD1_NW && B <= 3 * (int64_t)m->n_cu ? GRAD1_NW_FEW : GRAD1_NW;
 }
 // LDS for the copies of the waves' sums (InsLayout) that keeps the KM = 8
 // instances' 6 workgroups per CU (160 KB, 20 KB of each without the copies).

@@ -1,6 +1,6 @@
 """The single-pass adjoint's two shapes with a moving average: four waves per
-vector (tiles of 512 epochs) up to three vectors per compute unit, two (tiles of
-256) beyond.  On both sides of that batch size and around one and two tiles of
+vector (tiles of 512 epochs) up to three vectors per compute unit of more than 256
+epochs, else two (tiles of 256).  On both sides of that batch size and around one and two tiles of
 either, against the two-pass kernel, which computes the same sums in another order:
 lnL to 1e-12 relative and the gradient to 1e-9 of max(|g|, 1), the bounds the two
 kernels are held to on the catalogue stars."""
