@@ -276,10 +276,13 @@ int emp_pick_wpt(const EmpModel* m, int64_t B, bool halfstep) {
     // 111 / 87 / 77 / 78 us (the rule: 4), 6 x 60 at 3000 epochs, FP64, 179 / 111 /
     // 75 / 64 us (8), 8 x 200 at 400 epochs 56 / 52 / 49 / 49 us (4), 16 x 1024 at
     // 10^4 epochs 2.38 / 2.21 / 2.07 / 2.17 ms (4).
+    // Models without planets do little per epoch: about 8 waves per SIMD, one per
+    // vector beyond (FP64, no moving average, 8192 vectors of 1000 / 3000 / 10^4
+    // epochs at 1 / 2 / 4: 18 / 23 / 26, 34 / 43 / 41 and 94 / 107 / 94 us).
     const int64_t simds = (int64_t)m->n_cu * 4;
-    const int N = m->dev.N, wmin = N >= 1024 ? 2 : 1;
+    const int N = m->dev.N, wmin = N >= 1024 && m->dev.K ? 2 : 1, per_simd = m->dev.K ? 32 : 8;
     int wpt = 1;
-    while (wpt < 8 && (B * wpt < 32 * simds || wpt < wmin)) {
+    while (wpt < 8 && (B * wpt < per_simd * simds || wpt < wmin)) {
         const int lanes = 64 * wpt * 2;
         if (halfstep ? (lanes > N || (4 * lanes > N && B * wpt >= 4 * simds)) : 3 * lanes > N) break;
         wpt *= 2;
