@@ -1299,13 +1299,18 @@ static void launch_grad_t(const ModelDev& md, const double* th, int64_t B, int64
 constexpr int GRAD1_NW = 2;
 // Four with the moving average, for series of more than one tile, while the batch
 // has at most three vectors per compute unit: the launch is then one vector's chain
-// of tiles long, and four waves halve the tiles.  FP64 at 2 / 4 waves per vector: 7 planets x 1747 epochs
-// with a global MA(1), 200 / 768 / 1024 vectors 76 / 51, 92 / 74 and 96 / 102 us;
-// 2 x 10^4 with MA(1) per instrument 197 / 113, 236 / 159 and 243 / 189 us; 6 x
-// 300, 26 / 18, 29 / 24 and 31 / 33 us; 7 x 256, one tile of two waves, 19 / 19 and
-// 24 / 27 us (200, 768).
-constexpr int GRAD1_NW_FEW = 4;
+// of tiles long, and four waves halve the tiles.  FP64 at 2 / 4 waves per vector: 7
+// planets x 1747 epochs with a global MA(1), 200 / 768 / 1024 vectors 76 / 51, 92 /
+// 74 and 96 / 102 us; 2 x 10^4 with MA(1) per instrument 197 / 113, 236 / 159 and
+// 243 / 189 us; 6 x 300, 26 / 18, 29 / 24 and 31 / 33 us; 7 x 256, one tile of two
+// waves, 19 / 19 and 24 / 27 us (200, 768).
+// One for series of at most one wave's tile, which leave a second wave without
+// epochs.  FP64 at 2 waves / 1 / the two-pass kernel, 2000 and 65,536 vectors: 7 x 29
+// with MA(1) 52 / 28 / 27 and 967 / 597 / 701 us, 3 x 63 without 21 / 17 / 19 and 453 /
+// 299 / 446, 1 x 128 15 / 14 / 18 and 283 / 211 / 427.
+constexpr int GRAD1_NW_FEW = 4, GRAD1_NW_SHORT = 1;
 static int grad1_waves(const EmpModel* m, int64_t B) {
+    if (m->dev.N <= 128 * GRAD1_NW_SHORT) return GRAD1_NW_SHORT;
     return m->dev.ma_active && m->dev.N > 128 * GRAD1_NW && B <= 3 * (int64_t)m->n_cu ? GRAD1_NW_FEW : GRAD1_NW;
 }
 // LDS for the copies of the waves' sums (InsLayout) that keeps the KM = 8
@@ -1409,11 +1414,15 @@ int emp_launch_grad_ws(const EmpModel* m, const double* th, int64_t B, int64_t l
         // Eight copies of the wave's sums, fewer where many instruments would cost occupancy.
         const int rows = nw * InsLayout(md, has_post(md)).rows;
         int cl = 3;
-        while (cl && (rows << cl) * sizeof(double) > GRAD1_INS_BYTES * (nw / GRAD1_NW)) --cl;
+        while (cl && (rows << cl) * sizeof(double) > GRAD1_INS_BYTES * nw / GRAD1_NW) --cl;
         const size_t lds = (size_t)(rows << cl) * sizeof(double);
 #define EMP_CASE1(P, E, A, W, M, T) hipLaunchKernelGGL((k_lnl_grad1<P, E, A, W, M, T>), dim3((unsigned)B), dim3(64 * W), lds, s, md, th, B, ld, lnl, grad, nf, stale, cl)
-#define EMP_CASE1M(P, E, A, W, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, W, GRAD1_FEW, T); else if (md.K <= 6) EMP_CASE1(P, E, A, W, 6, T); else EMP_CASE1(P, E, A, W, KMAX, T); }
-#define EMP_CASE1A(P, E, T) { if (!md.ma_active) EMP_CASE1M(P, E, false, GRAD1_NW, T) else if (nw == GRAD1_NW) EMP_CASE1M(P, E, true, GRAD1_NW, T) else EMP_CASE1M(P, E, true, GRAD1_NW_FEW, T) }
+#define EMP_CASE1M(P, E, A, W, T) { if (md.K <= GRAD1_FEW) EMP_CASE1(P, E, A, W, GRAD1_FEW, T); else if (W == GRAD1_NW && md.K <= 6) EMP_CASE1(P, E, A, GRAD1_NW, 6, T); else EMP_CASE1(P, E, A, W, KMAX, T); }
+#define EMP_CASE1A(P, E, T) { \
+    if (!md.ma_active) { if (nw == GRAD1_NW_SHORT) EMP_CASE1M(P, E, false, GRAD1_NW_SHORT, T) else EMP_CASE1M(P, E, false, GRAD1_NW, T) } \
+    else if (nw == GRAD1_NW_SHORT) EMP_CASE1M(P, E, true, GRAD1_NW_SHORT, T) \
+    else if (nw == GRAD1_NW_FEW) EMP_CASE1M(P, E, true, GRAD1_NW_FEW, T) \
+    else EMP_CASE1M(P, E, true, GRAD1_NW, T) }
 #define EMP_CASE1T(P, E) { if (model_tp(md)) EMP_CASE1A(P, E, true) else EMP_CASE1A(P, E, false) }
         if (precision == 0) { if (has_post(md)) EMP_CASE1T(0, 1) else EMP_CASE1T(0, 0) }
         else { if (has_post(md)) EMP_CASE1T(1, 1) else EMP_CASE1T(1, 0) }

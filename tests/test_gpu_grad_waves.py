@@ -1,9 +1,9 @@
-"""The single-pass adjoint's two shapes with a moving average: four waves per
-vector (tiles of 512 epochs) up to three vectors per compute unit of more than 256
-epochs, else two (tiles of 256).  On both sides of that batch size and around one and two tiles of
-either, against the two-pass kernel, which computes the same sums in another order:
-lnL to 1e-12 relative and the gradient to 1e-9 of max(|g|, 1), the bounds the two
-kernels are held to on the catalogue stars."""
+"""The single-pass adjoint's shapes: one wave per vector up to 128 epochs; with a
+moving average four (tiles of 512 epochs) up to three vectors per compute unit of
+more than 256 epochs; else two (tiles of 256).  On both sides of these limits and
+around one and two tiles, against the two-pass kernel, which computes the same sums
+in another order: lnL to 1e-12 relative and the gradient to 1e-9 of max(|g|, 1), the
+bounds the two kernels are held to on the catalogue stars."""
 import numpy as np
 import pytest
 
@@ -13,8 +13,8 @@ from tests.test_gpu_grad_single_pass_edges import _draws, _model
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ma", ["instrument", "global", "strong"])
-@pytest.mark.parametrize("n,k,param,acc", [(7, 1, 1, 0), (255, 2, 6, 0), (256, 4, 1, 1), (257, 6, 1, 0), (511, 8, 3, 0),
+@pytest.mark.parametrize("ma", ["none", "instrument", "global", "strong"])
+@pytest.mark.parametrize("n,k,param,acc", [(7, 1, 1, 0), (127, 8, 6, 0), (128, 5, 1, 0), (129, 7, 6, 2), (255, 2, 6, 0), (256, 4, 1, 1), (257, 6, 1, 0), (511, 8, 3, 0),
                                            (512, 7, 6, 0), (513, 3, 0, 2), (1023, 5, 6, 0), (1025, 4, 4, 0)])
 def test_both_shapes_match_two_pass(n, k, param, acc, ma):
     rng = np.random.default_rng(n + k)
