@@ -183,7 +183,7 @@ __device__ __forceinline__ void post_accumulate(const ModelDev& md, const SL& sl
     for (int c = 0; c < md.n_cos; ++c) {
         const double r = reduce_2pi(cos_phase(sl, c, t));
         double sn, cs;
-        sincos_tab(tab, cos_arg(r), sn, cs);
+        sincos_tab(tab, __builtin_fabs(r), sn, cs);
         const double dph = -sl.cosw[c][0] * (r < 0.0 ? -sn : sn);
         atomicAdd(&acc[(3 * c + 0) << cl], w * cs);
         atomicAdd(&acc[(3 * c + 1) << cl], w * dph);

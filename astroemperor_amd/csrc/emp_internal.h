@@ -51,7 +51,8 @@ struct ModelDev {
     int sai_w;            // most activity columns of one instrument (0: no activity terms)
     const double* sai;    // [sai_w][N] column c of each epoch's own instrument, device order
     const int* sai_base;  // [I + 1] first coefficient (within the block) of each instrument
-    const double* t;      // [N] device order
+    const double* t;      // [N + 1] device order, then the largest |t| (as a field here it spills scalar registers
+                          //     in the adjoint's loop: 6% with a sinusoid at 1 planet x 1500 epochs)
     const double* y;      // [N]
     const double* s2;     // [N] yerr^2
     const double* dt;     // [N] t_i - t_{i-1} within an MA segment, -1 at a segment start;
@@ -69,7 +70,6 @@ struct ModelDev {
     const double2* sctab;             // [SC_N + 1] (sin, cos) of k pi / SC_N
     double lnl_const;                 // -0.5 ln(2 pi) N
     double t0;                        // X_[0] (acceleration origin)
-    double tmax;                      // largest |t|
 };
 
 // Per-slot LDS scratch of the likelihood kernels.  KTE: the entry of the

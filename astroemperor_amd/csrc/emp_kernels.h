@@ -92,11 +92,15 @@ __device__ inline double prior_vector_wave(const ModelDev& md, const double* th,
 // start, which is clamped.
 __device__ __forceinline__ PlanetC planet_slot(const ModelDev& md, const double* th, int p) {
     PlanetC pc = planet_setup(th + md.off_kep + 5 * p, md.param, md.use_c);
-    const double reach = __builtin_fabs(pc.freq) * (md.tmax + __builtin_fabs(pc.tp)) + __builtin_fabs(pc.phase);
+    const double reach = __builtin_fabs(pc.freq) * (md.t[md.N] + __builtin_fabs(pc.tp)) + __builtin_fabs(pc.phase);
     const bool table = md.N >= KT_MIN_EPOCHS && !pc.bad && pc.e <= KT_EMAX && reach <= KT_MMAX;
     pc.ktab = !table ? 0 : md.N < KT_SHORT ? 2 : 1;
     return pc;
 }
+
+// Largest phase of a cosine term: reduce_2pi leaves up to 1.2e-16 of it above pi,
+// here 4.2e-3 rad, within the half step (6.1e-3) that the sin/cos table takes.
+constexpr double COS_MMAX = 35184372088832.0;      // 2^45
 
 // The slot's other constants (instruments, acceleration, cosine terms) and the
 // planets' Kepler path flags, kf those of planet `lane`.  Called by a whole wave.
@@ -134,6 +138,10 @@ __device__ __forceinline__ void slot_rest(const ModelDev& md, SL& sl, int lane, 
             const double* th = sl.theta + md.off_mag;
             A = th[1 + c]; f = (c == 0 ? PI_D : 2.0 * PI_D) / th[0]; ph = th[3 + c];
         }
+        // A phase beyond FP64's resolution reduces to no angle of the sin/cos
+        // table: such a term is held at phase 0 (one that is not finite stays so).
+        const double reach = __builtin_fabs(f) * md.t[md.N] + __builtin_fabs(ph);
+        if (reach > COS_MMAX && reach < __builtin_inf()) f = ph = 0.0;
         sl.cosw[lane][0] = A;
         sl.cosw[lane][1] = f;
         sl.cosw[lane][2] = ph;
@@ -235,14 +243,6 @@ __device__ __forceinline__ double cos_phase(const SL& sl, int c, double t) {
     return sl.cosw[c][1] * t + sl.cosw[c][2];
 }
 
-// |r| of a reduced phase r, held in the sin/cos table's range (half a step past
-// pi): a phase beyond FP64's resolution does not reduce to [0, pi].  NaN stays.
-__device__ __forceinline__ double cos_arg(double r) {
-    constexpr double MOST = PI_D + 0.49 * SC_H;
-    const double a = __builtin_fabs(r);
-    return a > MOST ? MOST : a;
-}
-
 // Terms added after the moving average: in the reference's block order
 // StellarActivity, Sinusoid and MagneticCycle follow MOAV (emp/emp.py:
 // 2628-2650), so the MA residuals do not contain them.
@@ -273,7 +273,7 @@ __device__ __forceinline__ double epoch_post(const ModelDev& md, const SL& sl, c
 #pragma unroll 1
     for (int c = 0; c < md.n_cos; ++c) {
         double sn, cs;
-        sincos_tab(tb, cos_arg(reduce_2pi(cos_phase(sl, c, t))), sn, cs);
+        sincos_tab(tb, __builtin_fabs(reduce_2pi(cos_phase(sl, c, t))), sn, cs);
         v = __builtin_fma(sl.cosw[c][0], cs, v);
     }
     return v;

@@ -531,8 +531,6 @@ int emp_model_host(const EmpModelDesc* d, ModelHost* h) {
     md.lnl_const = -0.5 * std::log(2.0 * M_PI) * (double)N;
     md.npseq = (int)h->pseq.size();
     md.t0 = d->t[0];
-    md.tmax = 0.0;
-    for (int i = 0; i < N; ++i) md.tmax = std::fmax(md.tmax, std::fabs(d->t[i]));
     // Fixed MA timescales (the usual setup): the weight exp(-dt / tau) of
     // every epoch is the same for all parameter vectors; compute it once.
     md.ma_wfixed = 0;
@@ -550,6 +548,14 @@ int emp_model_host(const EmpModelDesc* d, ModelHost* h) {
             }
         }
     }
+    // One entry past the epochs (the columns stay of one length): the largest |t|.
+    double tmax = 0.0;
+    for (int i = 0; i < N; ++i) tmax = std::fmax(tmax, std::fabs(d->t[i]));
+    h->t.push_back(tmax);
+    h->y.push_back(0.0);
+    h->s2.push_back(1.0);
+    h->dt.push_back(0.0);
+    h->ins.push_back(0);
     return EMP_OK;
 }
 

@@ -1,5 +1,5 @@
 """Cosine terms whose phase is beyond FP64's resolution: no reduction brings it to
-[-pi, pi], so the sin/cos table's argument is held in the table's range.  The value
+[-pi, pi], the sin/cos table's range, so the term is held at phase 0.  The value
 of such a term is a cosine of some angle (at most its amplitude), and the likelihood
 and its gradient are the numbers that belong to it; a phase that is not a number
 stays none."""
