@@ -88,7 +88,7 @@ struct SlotLDSt {
 
 // The slot of a workgroup that holds `SLOTS` of them: the interval tables
 // (8 KiB per slot) where there are at most two, the node tables (4 KiB)
-// where more would cost occupancy or not fit (16 slots: 175 KiB).
+// where more would cost occupancy (four to eight slots).
 template <int SLOTS>
 using SlotLDS = SlotLDSt<std::conditional_t<(SLOTS <= 2), float4, float2>>;
 
@@ -112,7 +112,7 @@ struct EmpModel {
 };
 
 // Host-side preparation of one model: validated, epochs in device order
-// (grouped by instrument when the per-instrument moving average is active),
+// (grouped by instrument unless a global moving average is active),
 // MA time steps, free/fixed maps, prior block starts.  dev holds the scalars;
 // its pointers are left null for the caller to place the arrays.
 struct ModelHost {

@@ -2,8 +2,9 @@
 // and PT kernels.
 //
 // Launch geometry: a parameter vector belongs to WPT waves.  With WPT > 1 the
-// workgroup is those waves; with one wave per vector the waves of a workgroup
-// share the sin/cos table and nothing else.  The vector's waves walk the epochs
+// workgroup is those waves (in the two-pass adjoint several such vectors, which
+// wait together); with one wave per vector the waves of a workgroup share the
+// sin/cos table and nothing else.  The vector's waves walk the epochs
 // in chunks, each lane with two consecutive epochs (one in a last chunk of at
 // most 64 WPT), read straight from global memory: the data of every vector are
 // the same few KB to hundreds of KB, in L1 and L2.
@@ -666,7 +667,7 @@ __device__ __forceinline__ void lnl_chunk(const ModelDev& md, const SL& sl, cons
 // two waves on) and no tile staging: one barrier per chunk with the MA, none
 // without.  Measured against one epoch per lane with LDS tiles shared by the
 // vectors of a 512-thread workgroup: 8192 vectors of 7 planets x 10^4 epochs,
-// MA(1), mixed, 1.10 -> 1.01 ms; 2560 of 3 x 1530 FP64 45 -> 41 us; 1283 of 4 x
+// MA(1), mixed, 1.10 -> 0.93 ms; 2560 of 3 x 1530 FP64 45 -> 38 us; 1283 of 4 x
 // 783 with a sinusoid 43 -> 22 us (that instance also lost the MA orders above
 // 1, 84 -> 74 VGPRs); stretch sweeps at 16 x 1024 x 10^4, FP64, 3.6 -> 2.5 ms.
 template <int PREC, int WPT, bool WRITE, bool WEPS = false, int EXT = 2, class SL>

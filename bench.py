@@ -62,14 +62,14 @@ PEAK_FP64_TFLOPS = 78.6       # MI355X FP64 vector, FMA = 2 flops
 # (workload, kernel, precision); values (FETCH_SIZE, WRITE_SIZE).  Source:
 # profiles/hbm_traffic_half_step_adjoint_systems.md.
 TRAFFIC_KIB = {
-    ("c5", "k_pt_half", "mixed"): (4201.5, 1471.4),       # k_pt_half<1, 4, 0>, 8192 proposals
-    ("c5", "k_pt_half", "fp64"): (4224.9, 1471.4),        # k_pt_half<0, 4, 0>
-    ("c5", "k_lnl_grad", "mixed"): (10389.6, 94609.6),    # k_lnl_grad1<1, 0, true, 2, 8, false>, 8192 vectors
-    ("c5", "k_lnl_grad", "fp64"): (10472.4, 95612.1),     # k_lnl_grad1<0, 0, true, 2, 8, false>
-    ("c2", "k_pt_step", "mixed"): (1199.0, 471.4),        # k_pt_step<1, 4, 0>, 1280 proposals
-    ("c2", "k_pt_step", "fp64"): (1208.7, 481.4),         # k_pt_step<0, 4, 0>
-    ("c3", "k_sys sweep", "mixed"): (975874.0, 163064.8),  # 2 k_sys_prior, 2 k_sys_lik<1, 1>, k_sys_swap, 4096 systems
-    ("c3", "k_sys sweep", "fp64"): (976013.6, 163037.0),   # the same with k_sys_lik<0, 1>
+    ("c5", "k_pt_half", "mixed"): (4216.2, 1471.4),       # k_pt_half<1, 4, 0>, 8192 proposals
+    ("c5", "k_pt_half", "fp64"): (4236.9, 1471.4),        # k_pt_half<0, 4, 0>
+    ("c5", "k_lnl_grad", "mixed"): (10394.0, 94842.1),    # k_lnl_grad1<1, 0, true, 2, 8, false>, 8192 vectors
+    ("c5", "k_lnl_grad", "fp64"): (10476.3, 94844.5),     # k_lnl_grad1<0, 0, true, 2, 8, false>
+    ("c2", "k_pt_step", "mixed"): (1190.5, 471.4),        # k_pt_step<1, 4, 0>, 1280 proposals
+    ("c2", "k_pt_step", "fp64"): (1220.7, 471.4),         # k_pt_step<0, 4, 0>
+    ("c3", "k_sys sweep", "mixed"): (979968.4, 163066.1),  # 2 k_sys_prior, 2 k_sys_lik<1, 1>, k_sys_swap, 4096 systems
+    ("c3", "k_sys sweep", "fp64"): (980038.6, 163044.3),   # the same with k_sys_lik<0, 1>
 }
 FETCH_SCALE, WRITE_SCALE = 2.00, 1.00
 
@@ -612,7 +612,7 @@ def main():
     dom = "k_lnl_grad" if share["k_lnl_grad"] >= share["k_pt_half"] else "k_pt_half"
     roof = dict(mixed[f"roofline_{dom}"])
     roof["time_share"] = share[dom]
-    roof["convention"] = ("FP64-equivalent flops = 2 x ops; lnL per vector: planet-epochs x ops_kep (127 FP64 / 51 "
+    roof["convention"] = ("FP64-equivalent flops = 2 x ops; lnL per vector: planet-epochs x ops_kep (63 FP64 / 51 "
                           "mixed) + epochs x 46 + MA epochs x 23; adjoint: the same + planet-epochs x 24 + epochs x 4 "
                           "+ MA epochs x 4")
     roof["fp64_path"] = {k: fp64[f"roofline_{dom}"][k] for k in ("achieved", "frac", "launch_ms")}
